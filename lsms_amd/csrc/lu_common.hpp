@@ -108,19 +108,6 @@ __device__ __forceinline__ GCx<T> *tile_ptr(const SolveDesc &d, int ti, int tj) 
 }
 __device__ __forceinline__ long tile_ld(const SolveDesc &d) { return d.tiled ? kTile : d.ld; }
 
-// Wave-wide argmax of v (ties -> smallest index); all lanes get the result.
-template <class T>
-__device__ inline void wave_argmax(T &v, int &idx) {
-  for (int off = 32; off >= 1; off >>= 1) {
-    T ov = __shfl_xor(v, off, 64);
-    int oi = __shfl_xor(idx, off, 64);
-    if (ov > v || (ov == v && oi < idx)) {
-      v = ov;
-      idx = oi;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Complex 32x32x64 wave product on MFMA 16x16x4, 3M form:
 //   P1 = Ar Br, P2 = Ai Bi, P3 = (Ar+Ai)(Br+Bi);  re = P1 - P2, im = P3 - P1 - P2

@@ -10,7 +10,7 @@
 // pivoting scheme of the reference's block-inverse solvers.
 //
 // Per step s (tile column c0 = 64 s), batched over all solves:
-//   k_lu_diag    factor A_ss = P^T L U in LDS; store L^-1, U^-1 and P
+//   k_lu_diag    factor A_ss = P^T L U in LDS (tile_lu.hpp); store L^-1, U^-1 and P
 //   k_lu_panel   L_is = A_is U^-1 (tiles below), U_sj = L^-1 P A_sj (right)
 //   k_lu_update  A_ij -= L_is U_sj                     <- MFMA, dominant
 // with the steps taken in groups (k_lu_cross, k_lu_trail: the trailing
@@ -25,161 +25,9 @@
 // All kernels are templated on the real type: double (complex FP64, MFMA
 // v_mfma_f64_16x16x4f64) or float (complex FP32, v_mfma_f32_16x16x4f32).
 #include "lu_common.hpp"
+#include "tile_lu.hpp"
 
 namespace lsmsx {
-
-// In-LDS LU with partial pivoting of a 64x64 tile A[col][row].  Pivot rows
-// for column j come from [j, nd) while j < nd and from [j, 64) afterwards,
-// so rows >= nd (the central site of the last tile) never pivot into the
-// non-central part.  Full-row swaps (LAPACK getrf convention inside the
-// tile), piv[] the swap sequence, perm[] the resulting permutation.  256 threads.
-template <class T>
-__device__ void tile_lu_lds(CxT<T> (*A)[kTile + 1], int nd, int *piv, int *perm, int *sinfo,
-                            double *sminpiv, int col_base) {
-  typedef CxT<T> V;
-  const int tid = threadIdx.x;
-  for (int j = 0; j < kTile; j++) {
-    const int hi = (j < nd) ? nd : kTile;
-    if (tid < 64) {
-      // wave 0: pivot search, row swap (lane = column) and column scaling;
-      // wave-scope ordering of its LDS traffic is enough between them
-      T v = (tid >= j && tid < hi) ? cabs1(A[j][tid]) : T(-1);
-      int idx = tid;
-      wave_argmax(v, idx);
-      if (tid == 0) {
-        piv[j] = idx;
-        int t = perm[j];
-        perm[j] = perm[idx];
-        perm[idx] = t;
-        double ax = A[j][idx].x, ay = A[j][idx].y;
-        double a = sqrt(ax * ax + ay * ay);
-        if (a < *sminpiv) *sminpiv = a;
-        if (v == T(0) && *sinfo == 0) *sinfo = col_base + j + 1;
-      }
-      const int p = idx;
-      if (p != j) {
-        V t = A[tid][j];
-        A[tid][j] = A[tid][p];
-        A[tid][p] = t;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const V a = A[j][j];
-      if ((a.x != T(0) || a.y != T(0)) && tid > j) A[j][tid] = cmul2(A[j][tid], crecip(a));
-    }
-    __syncthreads();
-    const V a = A[j][j];
-    const bool nz = (a.x != T(0) || a.y != T(0));
-    // rank-1 update of the trailing block: thread (row r = tid % 64, column
-    // class tid / 64) takes columns c > j of its class, with l = A(r, j) read
-    // once
-    if (nz && (tid & 63) > j) {
-      const int r = tid & 63;
-      const V l = A[j][r];
-      int c = tid >> 6;
-      if (c <= j) c += ((j - c) / 4 + 1) * 4;
-      // four columns at a time, all loads before the stores, so the LDS
-      // round trips overlap
-      for (; c < 64; c += 16) {
-        V u[4], x[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (c + 4 * q < 64) {
-            u[q] = A[c + 4 * q][j];
-            x[q] = A[c + 4 * q][r];
-          }
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (c + 4 * q < 64) {
-            x[q].x -= l.x * u[q].x - l.y * u[q].y;
-            x[q].y -= l.x * u[q].y + l.y * u[q].x;
-            A[c + 4 * q][r] = x[q];
-          }
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// In-place inversion of the factored tile: unit-lower L (waves 0 and 2 own
-// rows) and upper U (waves 1 and 3 own rows).  L^-1: for j = 63..0,
-// X[r][j] = -(L[r][j] + sum_{j<k<r} X[r][k] L[k][j]) for r > j.  U^-1: for
-// j = 0..63, X[j][j] = 1/U[j][j], X[r][j] = -X[j][j] sum_{r<=k<j} X[r][k] U[k][j].
-// Each sum is split between the two waves of its part by the parity of k
-// (two accumulators per thread), so the dependent LDS loads of a row are a
-// quarter as long; the second wave's half goes through LDS.
-template <class T>
-__device__ void tile_invert_lds(CxT<T> (*A)[kTile + 1]) {
-  typedef CxT<T> V;
-  __shared__ V part[2][kTile];
-  const int tid = threadIdx.x, r = tid & 63, w = tid >> 6;
-  const bool lpart = (w & 1) == 0;  // waves 0, 2: L^-1; waves 1, 3: U^-1
-  const int half = w >> 1;          // the parity of k this wave sums
-  auto madd = [](V &acc, V x, V y) {
-    acc.x += x.x * y.x - x.y * y.y;
-    acc.y += x.x * y.y + x.y * y.x;
-  };
-  for (int jj = 0; jj < kTile; jj++) {
-    const int jl = kTile - 1 - jj;
-    const int ju = jj;
-    V s0 = czero<V>(), s1 = czero<V>();
-    if (lpart) {
-      if (r > jl) {
-        int k = jl + 1 + half;
-        for (; k + 2 < r; k += 4) {
-          madd(s0, A[k][r], A[jl][k]);
-          madd(s1, A[k + 2][r], A[jl][k + 2]);
-        }
-        if (k < r) madd(s0, A[k][r], A[jl][k]);
-      }
-    } else if (r < ju) {
-      int k = r + half;
-      for (; k + 2 < ju; k += 4) {
-        madd(s0, A[k][r], A[ju][k]);
-        madd(s1, A[k + 2][r], A[ju][k + 2]);
-      }
-      if (k < ju) madd(s0, A[k][r], A[ju][k]);
-    }
-    s0.x += s1.x;
-    s0.y += s1.y;
-    if (half == 1) part[lpart ? 0 : 1][r] = s0;
-    __syncthreads();
-    V nv = czero<V>();
-    if (half == 0) {
-      const V o = part[lpart ? 0 : 1][r];
-      s0.x += o.x;
-      s0.y += o.y;
-      if (lpart) {
-        if (r > jl) {
-          const V a = A[jl][r];
-          nv.x = -(a.x + s0.x);
-          nv.y = -(a.y + s0.y);
-        }
-      } else {
-        const V ujj = A[ju][ju];
-        const bool nz = (ujj.x != T(0) || ujj.y != T(0));
-        const V xjj = nz ? crecip(ujj) : czero<V>();
-        if (r < ju) {
-          const V v = cmul2(s0, xjj);
-          nv.x = -v.x;
-          nv.y = -v.y;
-        } else if (r == ju) {
-          nv = xjj;
-        }
-      }
-    }
-    __syncthreads();  // every read of this step is done
-    if (half == 0) {
-      if (lpart) {
-        if (r > jl) A[jl][r] = nv;
-      } else if (r <= ju) {
-        A[ju][r] = nv;
-      }
-    }
-    __syncthreads();
-  }
-}
 
 // Stage a 64 x 64 tile (column stride ld) in LDS, S[col][row] =
 // src[rowmap(row) + ld col]: the 16 loads of a thread are all issued before
@@ -274,69 +122,60 @@ __device__ __forceinline__ void write_split_planes(float2 (*Ts)[kTile + 1], bool
 }
 
 // ---------------------------------------------------------------------------
-// Diagonal tile of step s: factor, write back L\U, store L^-1 (strict lower)
-// and U^-1 (upper incl. diagonal) packed in one tile, and the permutation.
+// The factors of a tile, as tile_lu and tile_invert_upper left them in t, to
+// the solve: L^-1 (strict lower) and U^-1 (upper incl. diagonal) packed in one
+// tile, the permutation and the pivot status; on the split path also the
+// planes of both for the fused panel's FP16 products.  256 threads.
+template <class T>
+__device__ __forceinline__ void store_tile(TileLds<T> &t, const SolveDesc &d, int step) {
+  typedef CxT<T> V;
+  const int tid = threadIdx.x;
+  if (tid < kTile) d.perm[step * kTile + tid] = t.prow[tid];
+  if (tid == 0) {
+    if (t.info != 0 && *d.info == 0) *d.info = t.info;
+    if (t.minpiv < *d.minpiv) *d.minpiv = t.minpiv;
+  }
+  GCx<T> *inv = (GCx<T> *)d.inv + step * d.inv_stride;
+#pragma unroll
+  for (int q = 0; q < kTile / 4; q++) {
+    const int r = tid & 63, c = (tid >> 6) + 4 * q;
+    inv[r + kTile * c] = t.get(c, r);
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (d.ihp) {
+      // L^-1 (unit lower, L layout) and U^-1 (U layout)
+      _Float16 *ip = (_Float16 *)d.ihp;
+      write_planes(
+          [&](int i, int k) {
+            V v = t.get(k, i);
+            v.x = i > k ? v.x : (i == k ? 1.f : 0.f);
+            v.y = i > k ? v.y : 0.f;
+            return v;
+          },
+          true, ip, d.ihe);
+      write_planes([&](int j, int k) { return upper_at<T>(t, k, j); }, false, ip + kPlaneHalves,
+                   d.ihe + 1);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Diagonal tile of step s: L^-1, U^-1 and the permutation (the factors
+// themselves are not needed again).  One tile takes 36 us in FP64 and
+// 33 us in FP32 alone on the chip; the LU in LDS with a rank-1 update and
+// workgroup barriers per column, and the inverses column by column, that it
+// replaces took 200 and 189 us, which was most of a single solve (N = 2160: 33
+// of them one after another).
 template <class T>
 __global__ __launch_bounds__(256) void k_lu_diag(const SolveDesc *__restrict__ descs, int step) {
-  typedef CxT<T> V;
   const SolveDesc &d = descs[blockIdx.x];
   step -= d.step0;
   if (step < 0 || step > d.nt - 1 || (step == d.nt - 1 && !d.full_lu)) return;
   if (d.conv && *d.conv) return;
-  __shared__ V A[kTile][kTile + 1];
-  __shared__ int piv[kTile], perm[kTile];
-  __shared__ int sinfo;
-  __shared__ double sminpiv;
-  const int tid = threadIdx.x;
-  const int c0 = step * kTile;
-  GCx<T> *Mt = tile_ptr<T>(d, step, step);
-  const long ld = tile_ld(d);
-  stage_tile<T>(A, Mt, ld, [](int r) { return r; });
-  if (tid < kTile) perm[tid] = tid;
-  if (tid == 0) {
-    sinfo = 0;
-    sminpiv = 1e300;
-  }
-  __syncthreads();
-  tile_lu_lds<T>(A, kTile, piv, perm, &sinfo, &sminpiv, c0);
-  for (int e = tid; e < kTile * kTile; e += 256) {
-    int r = e & 63, c = e >> 6;
-    Mt[r + ld * c] = A[c][r];
-  }
-  if (tid < kTile) d.perm[step * kTile + tid] = perm[tid];
-  if (tid == 0) {
-    if (sinfo != 0 && *d.info == 0) *d.info = sinfo;
-    if (sminpiv < *d.minpiv) *d.minpiv = sminpiv;
-  }
-  __syncthreads();
-  tile_invert_lds<T>(A);
-  GCx<T> *inv = (GCx<T> *)d.inv + step * d.inv_stride;
-  for (int e = tid; e < kTile * kTile; e += 256) {
-    int r = e & 63, c = e >> 6;
-    inv[r + kTile * c] = A[c][r];
-  }
-  if constexpr (sizeof(T) == 4) {
-    if (d.ihp) {
-      // split planes of L^-1 (unit lower, L layout) and U^-1 (U layout) for
-      // the fused panel's FP16 products
-      _Float16 *ip = (_Float16 *)d.ihp;
-      write_planes(
-          [&](int i, int k) {
-            V v = czero<V>();
-            if (i > k) v = A[k][i];
-            if (i == k) v.x = 1.f;
-            return v;
-          },
-          true, ip, d.ihe);
-      write_planes(
-          [&](int j, int k) {
-            V v = czero<V>();
-            if (k <= j) v = A[j][k];
-            return v;
-          },
-          false, ip + kPlaneHalves, d.ihe + 1);
-    }
-  }
+  __shared__ TileLds<T> t;
+  tile_lu<T>(t, tile_ptr<T>(d, step, step), tile_ld(d), kTile, step * kTile);
+  tile_invert_upper<T>(t);
+  store_tile<T>(t, d, step);
 }
 
 // Cross update of tile (ti, tj) inside the split-FP16 panel, C = A - sum over
@@ -805,92 +644,70 @@ __global__ __launch_bounds__(256) void k_lu_trail(const SolveDesc *__restrict__ 
 // The trailing kc x kc block becomes LU(S), S the Schur complement.
 //   plain FP64 path: solve S tau00 = t0 from the S factors;
 //   refined paths (d.X set; FP32 mixed or FP64 refined): store the tile's
-//   factors, inverses and permutation like k_lu_diag, for the refinement.
+//   inverses and permutation like k_lu_diag, for the refinement.
 template <class T>
 __global__ __launch_bounds__(256) void k_lu_last(const SolveDesc *__restrict__ descs) {
   typedef CxT<T> V;
   const SolveDesc &d = descs[blockIdx.x];
   if (d.conv && *d.conv) return;
-  __shared__ V A[kTile][kTile + 1];
-  __shared__ V X[kTile][kTile + 1];
-  __shared__ int piv[kTile], perm[kTile];
-  __shared__ int sinfo;
-  __shared__ double sminpiv;
-  const int tid = threadIdx.x;
-  const int step = d.nt - 1;
-  const int c0 = step * kTile;
-  const int kc = d.kc, nd = kTile - kc;
-  GCx<T> *Mt = tile_ptr<T>(d, step, step);
-  const long ld = tile_ld(d);
-  stage_tile<T>(A, Mt, ld, [](int r) { return r; });
-  if (tid < kTile) perm[tid] = tid;
-  if (tid == 0) {
-    sinfo = 0;
-    sminpiv = 1e300;
-  }
-  __syncthreads();
-  tile_lu_lds<T>(A, nd, piv, perm, &sinfo, &sminpiv, c0);
-  if (tid == 0) {
-    if (sinfo != 0 && *d.info == 0) *d.info = sinfo;
-    if (sminpiv < *d.minpiv) *d.minpiv = sminpiv;
-  }
-  if (d.X != nullptr) {  // refinement follows: keep the tile's factors
-    for (int e = tid; e < kTile * kTile; e += 256) {
-      int r = e & 63, c = e >> 6;
-      Mt[r + ld * c] = A[c][r];
-    }
-    if (tid < kTile) d.perm[step * kTile + tid] = perm[tid];
-    __syncthreads();
-    tile_invert_lds<T>(A);
-    GCx<T> *inv = (GCx<T> *)d.inv + step * d.inv_stride;
-    for (int e = tid; e < kTile * kTile; e += 256) {
-      int r = e & 63, c = e >> 6;
-      inv[r + kTile * c] = A[c][r];
-    }
+  __shared__ TileLds<T> t;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int step = d.nt - 1, kc = d.kc, nd = kTile - kc;
+  tile_lu<T>(t, tile_ptr<T>(d, step, step), tile_ld(d), nd, step * kTile);
+  if (d.X != nullptr) {  // refinement follows
+    tile_invert_upper<T>(t);
+    store_tile<T>(t, d, step);
     return;
   }
-  // X = P_S t0, then unit-lower and upper solves with the S factors; one
-  // thread per right-hand side.
-  for (int e = tid; e < kc * kc; e += 256) {
-    int r = e % kc, c = e / kc;
-    double2 t = d.t0[r + (long)d.ldt * c];
-    X[c][r].x = t.x;
-    X[c][r].y = t.y;
+  if (tid == 0) {
+    if (t.info != 0 && *d.info == 0) *d.info = t.info;
+    if (t.minpiv < *d.minpiv) *d.minpiv = t.minpiv;
   }
-  __syncthreads();
-  if (tid < kc) {
-    const int c = tid;
-    for (int j = nd; j < kTile; j++) {
-      int p = piv[j];
-      if (p != j) {
-        V t = X[c][j - nd];
-        X[c][j - nd] = X[c][p - nd];
-        X[c][p - nd] = t;
+  // one lane per row of the tile and four right-hand sides per wave at a time
+  // in registers: y = L_S^-1 P_S t0, then U_S x = y column by column, the row
+  // just finished broadcast by readlane (a zero diagonal of U counts as 1)
+  constexpr int kRhs = 4;
+  const int row = t.prow[lane] - nd;  // row of t0 in this position (central rows only)
+  V ur = t.dinv[lane];
+  if (ur.x == T(0) && ur.y == T(0)) ur.x = T(1);
+  for (int c0 = 0; c0 < kc; c0 += 4 * kRhs) {
+    V b[kRhs], y[kRhs];
+#pragma unroll
+    for (int q = 0; q < kRhs; q++) {
+      const int c = c0 + w + 4 * q;
+      b[q] = czero<V>();
+      if (lane >= nd && c < kc) {
+        const double2 v = d.t0[row + (long)d.ldt * c];
+        b[q].x = v.x;
+        b[q].y = v.y;
+      }
+      y[q] = b[q];
+    }
+    for (int j = nd; j < kTile - 1; j++) {
+      V l = t.get(j, lane);
+      l.x = lane > j ? l.x : T(0);
+      l.y = lane > j ? l.y : T(0);
+#pragma unroll
+      for (int q = 0; q < kRhs; q++) y[q] = cadd_mul(y[q], l, lane_value2(b[q], j));
+    }
+    for (int j = kTile - 1; j >= nd; j--) {
+      V u = t.get(j, lane);
+      u.x = lane < j ? u.x : T(0);
+      u.y = lane < j ? u.y : T(0);
+      const V r = lane_value2(ur, j);
+#pragma unroll
+      for (int q = 0; q < kRhs; q++) {
+        const V xj = cmul2(lane_value2(y[q], j), r);
+        y[q] = csub_mul(y[q], u, xj);
+        if (lane == j) y[q] = xj;
       }
     }
-    for (int j = 0; j < kc; j++) {
-      V xj = X[c][j];
-      for (int r = j + 1; r < kc; r++) {
-        V l = A[nd + j][nd + r];
-        X[c][r].x -= l.x * xj.x - l.y * xj.y;
-        X[c][r].y -= l.x * xj.y + l.y * xj.x;
-      }
+#pragma unroll
+    for (int q = 0; q < kRhs; q++) {
+      const int c = c0 + w + 4 * q;
+      if (lane >= nd && c < kc) d.tau00[(lane - nd) + kc * c] = make_double2(y[q].x, y[q].y);
     }
-    for (int j = kc - 1; j >= 0; j--) {
-      V u = A[nd + j][nd + j];
-      V xj = (u.x != T(0) || u.y != T(0)) ? cmul2(X[c][j], crecip(u)) : X[c][j];
-      X[c][j] = xj;
-      for (int r = 0; r < j; r++) {
-        V uu = A[nd + j][nd + r];
-        X[c][r].x -= uu.x * xj.x - uu.y * xj.y;
-        X[c][r].y -= uu.x * xj.y + uu.y * xj.x;
-      }
-    }
-  }
-  __syncthreads();
-  for (int e = tid; e < kc * kc; e += 256) {
-    int r = e % kc, c = e / kc;
-    d.tau00[r + kc * c] = make_double2(X[c][r].x, X[c][r].y);
   }
 }
 
