@@ -41,14 +41,12 @@ __device__ __forceinline__ void store_acc(GZ *C, long ld, const Acc3<double> &q)
       }
 }
 
-// C -= A B for one 64x64 tile, C entering the 3M sums (as k_lu_update).
+// C -= A B for one 64x64 tile, -C entering the 3M sums (as update_tile of the LU).
 __device__ __forceinline__ void tile_update(const GZ *__restrict__ A, const GZ *__restrict__ B,
                                             GZ *__restrict__ C, long ld) {
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
-  A += wr;
-  B += ld * wc;
   C += wr + ld * wc;
   Acc3<double> q;
 #pragma unroll
@@ -58,13 +56,20 @@ __device__ __forceinline__ void tile_update(const GZ *__restrict__ A, const GZ *
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         Z c = C[(16 * bi + li) + ld * (16 * bj + acc_row<double>(kq, r))];
-        q.p[0][bj][bi][r] = c.x;
+        q.p[0][bj][bi][r] = -c.x;
         q.p[1][bj][bi][r] = 0.0;
-        q.p[2][bj][bi][r] = c.x + c.y;
+        q.p[2][bj][bi][r] = -c.x - c.y;
       }
-  wave_gemm3m<double, true>([&](int i, int k) { return A[i + ld * k]; },
-                            [&](int k, int j) { return B[k + ld * j]; }, q);
-  store_acc(C, ld, q);
+  wave_gemm3m_k(A + wr, B + ld * wc, ld, kTile / 4, q);
+#pragma unroll
+  for (int bj = 0; bj < 2; bj++)
+#pragma unroll
+    for (int bi = 0; bi < 2; bi++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        C[(16 * bi + li) + ld * (16 * bj + acc_row<double>(kq, r))] =
+            Z{q.p[1][bj][bi][r] - q.p[0][bj][bi][r],
+              q.p[0][bj][bi][r] + q.p[1][bj][bi][r] - q.p[2][bj][bi][r]};
 }
 
 // Fill Y with zeros: one 64-column strip per workgroup.
@@ -102,7 +107,7 @@ __global__ __launch_bounds__(256) void k_inv_fwd_panel(const SolveDesc *__restri
   Acc3<double> q;
   zero_acc(q);
   // A(i,k) = L^-1(wr+i, k), unit lower; B(k,j) = (P Y_sc)(k, wc+j)
-  wave_gemm3m<double, false>([&](int i, int k) {
+  wave_gemm3m<double>([&](int i, int k) {
                                int ii = wr + i;
                                Z v = Z{ii == k ? 1.0 : 0.0, 0.0};
                                if (ii > k) v = inv[ii + kTile * k];
@@ -147,7 +152,7 @@ __global__ __launch_bounds__(256) void k_inv_bwd_panel(const SolveDesc *__restri
   Acc3<double> q;
   zero_acc(q);
   // A(i,k) = U^-1(wr+i, k), upper incl. diagonal; B(k,j) = Y_sc(k, wc+j)
-  wave_gemm3m<double, false>([&](int i, int k) {
+  wave_gemm3m<double>([&](int i, int k) {
                                int ii = wr + i;
                                Z v = Z{0.0, 0.0};
                                if (k >= ii) v = inv[ii + kTile * k];

@@ -124,15 +124,11 @@ struct Acc3 {
 };
 
 // One k-step (12 MFMAs) of the 3M product from operands already in registers.
-template <class T, bool NEGA>
+template <class T>
 __device__ __forceinline__ void gemm3m_step(CxT<T> (&av)[2], CxT<T> (&bv)[2], Acc3<T> &q) {
   T as[2], bs[2];
 #pragma unroll
   for (int t = 0; t < 2; t++) {
-    if (NEGA) {
-      av[t].x = -av[t].x;
-      av[t].y = -av[t].y;
-    }
     as[t] = av[t].x + av[t].y;
     bs[t] = bv[t].x + bv[t].y;
   }
@@ -154,7 +150,7 @@ __device__ __forceinline__ void gemm3m_step(CxT<T> (&av)[2], CxT<T> (&bv)[2], Ac
 // cycles) covers an L2 round trip in FP64; FP32 steps (384 cycles) with both
 // operands in L2 load three steps ahead (callers whose occupancy matters more
 // pass PF = 1).
-template <class T, bool NEGA, int PF = (sizeof(T) == 4 ? 3 : 1), class FA, class FB>
+template <class T, int PF = (sizeof(T) == 4 ? 3 : 1), class FA, class FB>
 __device__ __forceinline__ void wave_gemm3m(FA fa, FB fb, Acc3<T> &q) {
   typedef CxT<T> V;
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
@@ -174,7 +170,7 @@ __device__ __forceinline__ void wave_gemm3m(FA fa, FB fb, Acc3<T> &q) {
           bn[t] = fb(k0 + 4 + kq, 16 * t + li);
         }
       }
-      gemm3m_step<T, NEGA>(a, b, q);
+      gemm3m_step<T>(a, b, q);
 #pragma unroll
       for (int t = 0; t < 2; t++) {
         a[t] = an[t];
@@ -204,8 +200,61 @@ __device__ __forceinline__ void wave_gemm3m(FA fa, FB fb, Acc3<T> &q) {
     }
     const int c = ks % (PF + 1);
     V av[2] = {a[c][0], a[c][1]}, bv[2] = {b[c][0], b[c][1]};
-    gemm3m_step<T, NEGA>(av, bv, q);
+    gemm3m_step<T>(av, bv, q);
   }
+}
+
+// q += A B over 4 nk values of k in FP64 (nk a multiple of 4), A(i, k) at A[i +
+// ld k], B(k, j) at B[k + ld j], both wave-uniform.  An FP64 MFMA holds its
+// SIMD's VALU for all of its 64 cycles, whichever wave the VALU work is of, so
+// every other instruction of the loop adds to its time: the operands come by
+// buffer loads whose k offset is scalar, three k-steps ahead, and the only VALU
+// work left of a step are the four sums of the 3M form (through pointers, with
+// A negated, it was 17 instructions; 64 solves of N = 2160: trailing updates
+// 23.8 -> 22.4 ms, 75% of the MFMA cycles at the clock the card holds there,
+// the rest being the loads and stores of C at K = 128).
+__device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<double> *B, long ld,
+                                              int nk, Acc3<double> &q) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef unsigned b128 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
+  constexpr int kRange = 0x7fffffff, kFlags = 0x00027000;  // raw buffer, byte offsets
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, kRange, kFlags);
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, kRange, kFlags);
+  const int ld16 = (int)ld * 16;
+  const int va = 16 * li + ld16 * kq;           // A(li, kq), and 16 rows below
+  const int vb = 16 * kq + ld16 * li, vb2 = vb + 16 * ld16;  // B(kq, li), B(kq, 16 + li)
+  constexpr int PF = 3;
+  double2 a[PF + 1][2], b[PF + 1][2];
+  auto get = [](b128 x) __attribute__((always_inline)) {
+    return double2{__hiloint2double(x[1], x[0]), __hiloint2double(x[3], x[2])};
+  };
+  auto load = [&](int slot, int ks) __attribute__((always_inline)) {
+    const int sa = 4 * ks * ld16, sb = 64 * ks;
+    a[slot][0] = get(__builtin_amdgcn_raw_buffer_load_b128(ra, va, sa, 0));
+    a[slot][1] = get(__builtin_amdgcn_raw_buffer_load_b128(ra, va + 256, sa, 0));
+    b[slot][0] = get(__builtin_amdgcn_raw_buffer_load_b128(rb, vb, sb, 0));
+    b[slot][1] = get(__builtin_amdgcn_raw_buffer_load_b128(rb, vb2, sb, 0));
+  };
+  auto step = [&](int slot) __attribute__((always_inline)) {
+    double2 av[2] = {a[slot][0], a[slot][1]}, bv[2] = {b[slot][0], b[slot][1]};
+    gemm3m_step<double>(av, bv, q);
+  };
+#pragma unroll
+  for (int i = 0; i < PF; i++) load(i, i);
+  int ks = 0;
+#pragma unroll 1
+  for (; ks < nk - 4; ks += 4) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      load((i + PF) & 3, ks + i + PF);
+      step(i);
+    }
+  }
+  load(PF, ks + PF);
+#pragma unroll
+  for (int i = 0; i < 4; i++) step(i);
+#endif
 }
 
 template <class T>

@@ -448,7 +448,7 @@ __device__ __forceinline__ void panel_tile(const SolveDesc &d, int step, int ncr
     constexpr int kPanelPF = sizeof(T) == 8 ? 3 : 1;
     if (lower) {
       // A(i,k) = Ts(wr+i, k); B(k,j) = U^-1(k, wc+j), upper incl. diagonal
-      wave_gemm3m<T, false, kPanelPF>([&](int i, int k) { return Ts[k][wr + i]; },
+      wave_gemm3m<T, kPanelPF>([&](int i, int k) { return Ts[k][wr + i]; },
                                       [&](int k, int j) {
                                         int jj = wc + j;
                                         V v = czero<V>();
@@ -458,7 +458,7 @@ __device__ __forceinline__ void panel_tile(const SolveDesc &d, int step, int ncr
                                       q);
     } else {
       // A(i,k) = L^-1(wr+i, k), unit lower; B(k,j) = (P A_sj)(k, wc+j)
-      wave_gemm3m<T, false, kPanelPF>([&](int i, int k) {
+      wave_gemm3m<T, kPanelPF>([&](int i, int k) {
                                         int ii = wr + i;
                                         V v = czero<V>();
                                         if (ii == k) v.x = T(1);
@@ -530,18 +530,18 @@ __global__ __launch_bounds__(256) void k_lu_panel_h(const SolveDesc *__restrict_
 }
 
 // C(ti, tj) -= sum_{u < ns} L(ti, s0+u) U(s0+u, tj): one 64x64 tile per
-// workgroup, a 32x32 quarter per wave.  C enters the 3M sums at the start
-// (q1 = Cre, q2 = 0, q3 = Cre + Cim, products accumulated with -A), so
-// C' = (q1 - q2, q3 - q1 - q2): the tile is read and written once however
-// many rank-64 panels are applied.
+// workgroup, a 32x32 quarter per wave.  -C enters the 3M sums at the start
+// (q1 = -Cre, q2 = 0, q3 = -(Cre + Cim)), so C' = (q2 - q1, q1 + q2 - q3): the
+// tile is read and written once however many rank-64 panels are applied, and
+// no operand is negated.
 template <class T>
 __device__ __forceinline__ void update_tile(const SolveDesc &d, int ti, int tj, int s0, int ns) {
-  typedef CxT<T> V;
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
   const long ld = tile_ld(d);
   GCx<T> *__restrict__ C = tile_ptr<T>(d, ti, tj) + wr + ld * wc;
+  typedef T cv2 __attribute__((ext_vector_type(2)));
   Acc3<T> q;
 #pragma unroll
   for (int bj = 0; bj < 2; bj++)
@@ -551,32 +551,33 @@ __device__ __forceinline__ void update_tile(const SolveDesc &d, int ti, int tj, 
       for (int r = 0; r < 4; r++) {
         // C is read and written once per group: non-temporal, so that the
         // panels the other tiles read stay in L2
-        typedef T cv2 __attribute__((ext_vector_type(2)));
         const cv2 c = __builtin_nontemporal_load(
             (const cv2 *)&C[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))]);
-        q.p[0][bj][bi][r] = c.x;
+        q.p[0][bj][bi][r] = -c.x;
         q.p[1][bj][bi][r] = T(0);
-        q.p[2][bj][bi][r] = c.x + c.y;
+        q.p[2][bj][bi][r] = -c.x - c.y;
       }
-  for (int u = 0; u < ns; u++) {
-    const GCx<T> *__restrict__ A = tile_ptr<T>(d, ti, s0 + u) + wr;
-    const GCx<T> *__restrict__ B = tile_ptr<T>(d, s0 + u, tj) + ld * wc;
-    wave_gemm3m<T, true>([&](int i, int k) { return A[i + ld * k]; },
-                         [&](int k, int j) { return B[k + ld * j]; }, q);
+  if constexpr (sizeof(T) == 8) {
+    // column-major: the panels of consecutive steps are consecutive in k
+    wave_gemm3m_k(tile_ptr<T>(d, ti, s0) + wr, tile_ptr<T>(d, s0, tj) + ld * wc, ld, 16 * ns, q);
+  } else {
+    for (int u = 0; u < ns; u++) {
+      const GCx<T> *__restrict__ A = tile_ptr<T>(d, ti, s0 + u) + wr;
+      const GCx<T> *__restrict__ B = tile_ptr<T>(d, s0 + u, tj) + ld * wc;
+      wave_gemm3m<T>([&](int i, int k) { return A[i + ld * k]; },
+                            [&](int k, int j) { return B[k + ld * j]; }, q);
+    }
   }
 #pragma unroll
   for (int bj = 0; bj < 2; bj++)
 #pragma unroll
     for (int bi = 0; bi < 2; bi++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        V o;
-        o.x = q.p[0][bj][bi][r] - q.p[1][bj][bi][r];
-        o.y = q.p[2][bj][bi][r] - q.p[0][bj][bi][r] - q.p[1][bj][bi][r];
-        typedef T cv2 __attribute__((ext_vector_type(2)));
-        __builtin_nontemporal_store(cv2{o.x, o.y},
-                                    (cv2 *)&C[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))]);
-      }
+      for (int r = 0; r < 4; r++)
+        __builtin_nontemporal_store(
+            cv2{q.p[1][bj][bi][r] - q.p[0][bj][bi][r],
+                q.p[0][bj][bi][r] + q.p[1][bj][bi][r] - q.p[2][bj][bi][r]},
+            (cv2 *)&C[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))]);
 }
 
 // Trailing update of step s: A_ij -= L_is U_sj for all i, j > s.
