@@ -449,6 +449,18 @@ std::vector<int> site_offsets(const AtomDev &a, int nsc, bool solver) {
   return off;
 }
 
+// Copy of an n x n complex matrix between host and device.  Without gaps
+// between the columns it goes as one run of bytes: the row-wise copy of
+// pageable memory reaches 1.7 GB/s (9.5 of the 10.5 ms of a solve with
+// n = 999), the plain copy about 30 GB/s.
+int copy_square(void *dst, long ldd, const void *src, long lds, long n, hipMemcpyKind kind,
+                hipStream_t st) {
+  const size_t z = sizeof(double2);
+  if (ldd == n && lds == n) HIPCHK(hipMemcpyAsync(dst, src, z * n * n, kind, st));
+  else HIPCHK(hipMemcpy2DAsync(dst, z * ldd, src, z * lds, z * n, n, kind, st));
+  return 0;
+}
+
 // Steps per trailing update: with the split-FP16 update the context's
 // split_group (4, 8 or 16, default 8: the trailing matrix is read and
 // written once per group, the fused panels of a group's later steps apply
@@ -1905,8 +1917,7 @@ int lsmsx_build_kkr(lsmsx_ctx *c, int atom_id, int ispin, int iie, const double 
   if (int r = c->desc.ensure(1)) return r;
   if (int r = assemble_reference_layout(c, a, ispin, iie, prel, nsc, nspola, c->M.p, c->desc.p))
     return r;
-  HIPCHK(hipMemcpy2DAsync(m, sizeof(double2) * ldm, c->M.p, sizeof(double2) * N,
-                          sizeof(double2) * N, N, hipMemcpyDeviceToHost, c->stream));
+  if (int r = copy_square(m, ldm, c->M.p, N, N, hipMemcpyDeviceToHost, c->stream)) return r;
   HIPCHK(hipStreamSynchronize(c->stream));
   drain_profile(c);
   return 0;
@@ -1941,8 +1952,7 @@ int lsmsx_solve_tau00_matrix(lsmsx_ctx *c, int n, int k, const double *m, int ld
   if (int r = c->tau.ensure((size_t)k * k)) return r;
   if (int r = c->t0buf.ensure((size_t)k * k)) return r;
   if (int r = c->desc.ensure(1)) return r;
-  HIPCHK(hipMemcpy2DAsync(c->tmpM.p, sizeof(double2) * n, m, sizeof(double2) * ldm,
-                          sizeof(double2) * n, n, hipMemcpyHostToDevice, c->stream));
+  if (int r = copy_square(c->tmpM.p, n, m, ldm, n, hipMemcpyHostToDevice, c->stream)) return r;
   HIPCHK(hipMemcpyAsync(c->t0buf.p, t0, sizeof(double2) * k * k, hipMemcpyHostToDevice,
                         c->stream));
   SolveDesc d{};
@@ -2213,8 +2223,7 @@ int lsmsx_tau_full(lsmsx_ctx *c, int atom_id, int ispin, int iie, const double *
                      c->ldT, c->colmap.p, c->colmap.p + Ns, c->tfull.p, (long)N);
   if (int r = check_launch("k_tau_full_out")) return r;
   int hinfo = 0;
-  HIPCHK(hipMemcpy2DAsync(tau, sizeof(double2) * ldtau, c->tfull.p, sizeof(double2) * N,
-                          sizeof(double2) * N, N, hipMemcpyDeviceToHost, c->stream));
+  if (int r = copy_square(tau, ldtau, c->tfull.p, N, N, hipMemcpyDeviceToHost, c->stream)) return r;
   HIPCHK(hipMemcpyAsync(&hinfo, c->info.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   drain_profile(c);
