@@ -21,6 +21,8 @@
 //   x_s = U_ss^-1 (y_s - sum_{t>s} U_st x_t)
 // with the diagonal-tile inverses and permutations kept by the factorization;
 // the sums are taken right-looking, one tile column per launch (k_ir_step).
+#include <type_traits>
+
 #include "lu_common.hpp"
 
 namespace lsmsx {
@@ -366,61 +368,14 @@ __global__ __launch_bounds__(512) void k_ir_residual_g_finish(const SolveDesc *_
   }
 }
 
-// Wave-level 3M product for the refinement sweeps: acc(16 x 16nb) of rows
-// i0.. += sum_k Bop(k, j) * Aop(i0 + i, k), transposed MFMA form as in the LU
-// update (a-operand Bop(k0+kq, j0+li), b-operand Aop(i0+li, k0+kq)).
-// Register r of lane (li, kq) holds output (row i0+li, column 16jb +
-// acc_row<T>(kq, r)).
+// 3M sums of a wave's 16 x 16nb block in the refinement sweeps: transposed
+// MFMA form as in the LU update (a-operand B(k0+kq, j0+li), b-operand
+// A(i0+li, k0+kq)).  Register r of lane (li, kq) holds output (row i0+li,
+// column 16jb + acc_row<T>(kq, r)).
 template <class T>
 struct AccIR {
   Acc4<T> p[3][2];
 };
-
-// The k range is consumed in batches of 8 k-steps whose operand loads are
-// all issued before their MFMAs: one workgroup per solve leaves few waves per
-// SIMD, so latency is hidden by loads in flight, not by occupancy.
-template <class T, int U = 8, class FA, class FB>
-__device__ __forceinline__ void sweep_gemm(FA fa, FB fb, int k_begin, int k_end, int nb,
-                                           AccIR<T> &q) {
-  typedef CxT<T> V;
-  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
-  int kb = k_begin;
-  for (; kb + 4 * U <= k_end; kb += 4 * U) {
-    V a[U], b[U][2];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      a[u] = fa(li, kb + 4 * u + kq);
-      b[u][0] = fb(kb + 4 * u + kq, li);
-      if (nb > 1) b[u][1] = fb(kb + 4 * u + kq, 16 + li);
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const T as = a[u].x + a[u].y;
-#pragma unroll
-      for (int jb = 0; jb < 2; jb++) {
-        if (jb < nb) {
-          const V bb = b[u][jb];
-          q.p[0][jb] = mfma4(bb.x, a[u].x, q.p[0][jb]);
-          q.p[1][jb] = mfma4(bb.y, a[u].y, q.p[1][jb]);
-          q.p[2][jb] = mfma4(bb.x + bb.y, as, q.p[2][jb]);
-        }
-      }
-    }
-  }
-  for (int k0 = kb; k0 < k_end; k0 += 4) {
-    V a = fa(li, k0 + kq);
-    T as = a.x + a.y;
-#pragma unroll
-    for (int jb = 0; jb < 2; jb++) {
-      if (jb < nb) {
-        V b = fb(k0 + kq, 16 * jb + li);
-        q.p[0][jb] = mfma4(b.x, a.x, q.p[0][jb]);
-        q.p[1][jb] = mfma4(b.y, a.y, q.p[1][jb]);
-        q.p[2][jb] = mfma4(b.x + b.y, as, q.p[2][jb]);
-      }
-    }
-  }
-}
 
 // 3M sums started from C: q1 = Cre, q2 = 0, q3 = Cre + Cim; with the
 // products accumulated against -A this gives C - A B = (q1 - q2, q3 - q1 - q2).
@@ -484,9 +439,23 @@ __global__ __launch_bounds__(256) void k_ir_step(const SolveDesc *__restrict__ d
   const int i0 = t * kTile + 16 * w, rs = s * kTile;
   // factor tile (t, s), rows of this wave
   const GCx<T> *__restrict__ Wt = tile_ptr<T>(d, t, s < 0 ? 0 : s) + 16 * w;
+  const bool diag = FWD ? t == s + 1 : t == s - 1;
+  const GCx<T> *__restrict__ inv = (const GCx<T> *)d.inv + t * d.inv_stride + 16 * w + li;
   // every global load of the step is issued before the first wait: the
-  // factor tile (t, s) in MFMA layout, r_t, and the 64 x kc block of tile s
-  V a[kTile / 4], st[8];
+  // factor tile (t, s) in MFMA layout, r_t, the 64 x kc block of tile s, and
+  // in the workgroup of the next diagonal tile that tile's inverse and pivots.
+  // The launch is one link of a serial chain and as long as the latencies in
+  // it: with the inverse loaded behind the product, four k-steps at a time,
+  // 32 canted solves of N = 864 took 3.34 ms, so 2.93 ms.
+  V a[kTile / 4], st[8], ia[kTile / 4];
+  int pk[kTile / 4];
+  if (diag) {
+#pragma unroll
+    for (int u = 0; u < kTile / 4; u++) {
+      ia[u] = ldg<T>(inv + kTile * (4 * u + kq));
+      pk[u] = FWD ? ((const LSMSX_GLOBAL int *)d.perm)[t * kTile + 4 * u + kq] : 4 * u + kq;
+    }
+  }
   if (s >= 0 && !first) {
 #pragma unroll
     for (int u = 0; u < kTile / 4; u++) a[u] = ldg<T>(Wt + li + ld * (4 * u + kq));
@@ -526,9 +495,7 @@ __global__ __launch_bounds__(256) void k_ir_step(const SolveDesc *__restrict__ d
       }
     }
   }
-  const bool diag = FWD ? t == s + 1 : t == s - 1;
   if (diag) {
-    const GCx<T> *inv = (const GCx<T> *)d.inv + t * d.inv_stride;
     auto to_buf = [&]() {
       __syncthreads();
 #pragma unroll
@@ -539,37 +506,39 @@ __global__ __launch_bounds__(256) void k_ir_step(const SolveDesc *__restrict__ d
       __syncthreads();
       acc_zero<T>(q);
     };
-    // upper U^-1 of the diagonal tile, diagonal included
-    auto apply_uinv = [&]() {
-      sweep_gemm<T, 4>([&](int i, int k) {
-                      const int ii = 16 * w + i;
-                      V u;
-                      u.x = T(0);
-                      u.y = T(0);
-                      if (k >= ii) u = inv[ii + kTile * k];
-                      return u;
-                    },
-                    [&](int k, int j) { return buf[k][j]; }, 0, kTile, nb, q);
+    // the block times the unit lower L^-1 (rows of buf in pivot order) or the
+    // upper U^-1, diagonal included, both from the tile in ia
+    const int ii = 16 * w + li;
+    auto apply = [&](auto lower) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < kTile / 4; u++) {
+        const int k = 4 * u + kq;
+        V l = ia[u];
+        if (lower ? ii <= k : ii > k) {
+          l.x = lower && ii == k ? T(1) : T(0);
+          l.y = T(0);
+        }
+        const T ls = l.x + l.y;
+#pragma unroll
+        for (int jb = 0; jb < 2; jb++) {
+          if (jb < nb) {
+            const V bb = buf[lower ? pk[u] : k][16 * jb + li];
+            q.p[0][jb] = mfma4(bb.x, l.x, q.p[0][jb]);
+            q.p[1][jb] = mfma4(bb.y, l.y, q.p[1][jb]);
+            q.p[2][jb] = mfma4(bb.x + bb.y, ls, q.p[2][jb]);
+          }
+        }
+      }
     };
     to_buf();
     if (FWD) {
-      // unit lower L^-1 applied to the permuted rows
-      const int *perm = d.perm + t * kTile;
-      sweep_gemm<T, 4>([&](int i, int k) {
-                      const int ii = 16 * w + i;
-                      V l;
-                      l.x = ii == k ? T(1) : T(0);
-                      l.y = T(0);
-                      if (ii > k) l = inv[ii + kTile * k];
-                      return l;
-                    },
-                    [&](int k, int j) { return buf[perm[k]][j]; }, 0, kTile, nb, q);
+      apply(std::true_type{});
       if (t == nt - 1) {
         to_buf();
-        apply_uinv();
+        apply(std::false_type{});
       }
     } else {
-      apply_uinv();
+      apply(std::false_type{});
     }
   }
 #pragma unroll
