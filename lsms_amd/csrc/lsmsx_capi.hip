@@ -2519,8 +2519,8 @@ int lsmsx_green_mt(lsmsx_ctx *c, int nsolve, int lmax, int iprpts, int n_spin_po
                         hipMemcpyHostToDevice, st));
   if (green)
     HIPCHK(hipMemsetAsync(c->gf_green.p, 0, (size_t)nsolve * iprpts * sizeof(double2), st));
-  hipLaunchKernelGGL(k_green_mt, dim3((unsigned)((nsolve + kGreenSolves - 1) / kGreenSolves)),
-                     dim3(64), 0, st, c->gf_tau.p, c->ss_zlr.p, c->ss_jlr.p, c->ss_r.p,
+  hipLaunchKernelGGL(k_green_mt, dim3((unsigned)nsolve), dim3(kGreenThreads), 0, st, c->gf_tau.p,
+                     c->ss_zlr.p, c->ss_jlr.p, c->ss_r.p,
                      c->gf_pot.p, c->gf_potof.p, nullptr, nsolve, lmax, iprpts,
                      n_spin_pola == 1 ? 2.0 : 1.0, c->gf_dos.p, green ? c->gf_green.p : nullptr);
   HIPCHK(hipGetLastError());
@@ -2649,8 +2649,8 @@ int lsmsx_green_mt_resident(lsmsx_ctx *c, int nsolve, int lmax, int iprpts, int 
                         hipMemcpyHostToDevice, st));
   if (green)
     HIPCHK(hipMemsetAsync(c->gf_green.p, 0, (size_t)nsolve * iprpts * sizeof(double2), st));
-  hipLaunchKernelGGL(k_green_mt, dim3((unsigned)((nsolve + kGreenSolves - 1) / kGreenSolves)),
-                     dim3(64), 0, st, c->gf_tau.p, c->ss_zlr.p, c->ss_jlr.p, c->ss_r.p,
+  hipLaunchKernelGGL(k_green_mt, dim3((unsigned)nsolve), dim3(kGreenThreads), 0, st, c->gf_tau.p,
+                     c->ss_zlr.p, c->ss_jlr.p, c->ss_r.p,
                      c->gf_pot.p, c->gf_potof.p, c->gf_src.p, nsolve, lmax, iprpts,
                      n_spin_pola == 1 ? 2.0 : 1.0, c->gf_dos.p, green ? c->gf_green.p : nullptr);
   HIPCHK(hipGetLastError());
@@ -2746,7 +2746,7 @@ int lsmsx_green_mt_canted(lsmsx_ctx *c, int nsolve, int lmax, int iprpts, int np
                         hipMemcpyHostToDevice, st));
   if (green)
     HIPCHK(hipMemsetAsync(c->gf_green.p, 0, (size_t)nsolve * 4 * iprpts * sizeof(double2), st));
-  hipLaunchKernelGGL(k_green_mt_canted, dim3((unsigned)((nsolve + 1) / 2)), dim3(64), 0, st,
+  hipLaunchKernelGGL(k_green_mt_canted, dim3((unsigned)nsolve), dim3(4 * kGreenThreads), 0, st,
                      c->gf_tau.p, c->ss_zlr.p, c->ss_jlr.p, c->gf_w.p, c->ss_r.p, c->gf_pot.p,
                      c->gf_potof.p, nsolve, lmax, iprpts, c->gf_dos.p,
                      green ? c->gf_green.p : nullptr);

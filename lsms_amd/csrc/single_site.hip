@@ -649,20 +649,23 @@ __global__ void k_jlr_scale(const double *__restrict__ rmesh,
 // cinterp.f at sqrt(r_sph)), mdosms_c.f and mgreen_c.f, times 2 when
 // n_spin_pola = 1 (green_function.f:184-191).
 //
-// One 64-thread workgroup per eight solves (kGreenSolves): lane 8s+2l and
-// 8s+2l+1 run the running integrals of 2 z_l z_l and 2 z_l j_l of solve s
-// over the jmt+1 points of the x mesh (a ring of four fitted points, as
-// cnewint keeps them), so every lane of the wave carries one sequential
-// integral; lane s then contracts solve s's integrals with the diagonal of
-// tau00, and all lanes form green(r) solve by solve, reading zlr/jlr with
-// consecutive lanes on consecutive radial points.
+// One workgroup per solve, kIntLanes lanes to each running integral (2 z_l z_l
+// and 2 z_l j_l).  An increment of the running integral depends on its four
+// fitted points alone, so the lanes take the intervals of the x mesh in turn
+// and one lane adds the increments up in their order.  A lane's work is a
+// serial chain of FP64 operations and bounds the kernel: with one lane per
+// integral and eight solves per wave, 512 solves were 64 waves on the whole
+// chip and took 800 us, so 177.  One lane then contracts the integrals with the
+// diagonal of tau00, and all lanes form green(r), consecutive lanes on
+// consecutive radial points.
 
 namespace {
 
-// running integral step of cnewint.f for one interval: slots of the ring in
-// rs/fr/fi, interval from slot i0 to the next; returns the increment
-__device__ zd cnewint_step(const double *rs, const double *fr, const double *fi, int i0, int ip) {
-  const int i1 = (i0 + 3) & 3, ip1 = (i0 + 1) & 3, i2 = (i0 + 2) & 3;
+// running integral step of cnewint.f for one interval: points in the slots of
+// rs/fr/fi, interval from slot 0 to slot 1, slots 3 and 2 the further points
+// of the fit (before and after); returns the increment
+__device__ zd cnewint_step(const double *rs, const double *fr, const double *fi, int ip) {
+  const int i0 = 0, i1 = 3, ip1 = 1, i2 = 2;
   double xl[4], cr[4], ci[4];
   xl[0] = rs[i1];
   xl[1] = rs[i0];
@@ -707,11 +710,19 @@ __device__ zd cnewint_step(const double *rs, const double *fr, const double *fi,
 
 namespace {
 
-// int_zz_zj.f:116-165 for one lane: the running integral (cnewint.f, ip0 = 5,
-// on x_0 = 0, x_k = sqrt(r_k)) of 2 a_l b_l with f_0 = f_1, interpolated at
-// sqrt(r_sph) (cinterp.f); a, b are radial columns, rm the mesh
-__device__ zd sphere_integral(const double2 *__restrict__ a, const double2 *__restrict__ bcol,
-                              const double *__restrict__ rm, const GreenPot &P) {
+// lanes per running integral, and intervals per round (kept in LDS); the
+// lanes of an integral are consecutive threads
+constexpr int kIntLanes = 16;
+constexpr int kIntRound = 64;
+
+// int_zz_zj.f:116-165 by kIntLanes lanes: the running integral (cnewint.f,
+// ip0 = 5, on x_0 = 0, x_k = sqrt(r_k)) of 2 a_l b_l with f_0 = f_1,
+// interpolated at sqrt(r_sph) (cinterp.f); a, b are radial columns, rm the
+// mesh.  Valid in lane sub = 0.  Every thread of the workgroup calls it with
+// the same P (it has barriers); those without an integral pass active = false.
+__device__ zd sphere_integral(bool active, const double2 *__restrict__ a,
+                              const double2 *__restrict__ bcol, const double *__restrict__ rm,
+                              const GreenPot &P, int sub, zd *inc) {
   auto fval = [&](int k) -> zd {
     const int q = k == 0 ? 0 : k - 1;
     const zd u = mk(a[q].x, a[q].y), c = mk(bcol[q].x, bcol[q].y);
@@ -720,16 +731,7 @@ __device__ zd sphere_integral(const double2 *__restrict__ a, const double2 *__re
   auto xval = [&](int k) -> double { return k == 0 ? 0.0 : sqrt(rm[k - 1]); };
   const int nr = P.jmt + 1;
   const int ip = 2 * 5 + 1;
-  double rs[4], fr[4], fi[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    rs[k] = sqrt(xval(k));
-    const zd f = fval(k);
-    fr[k] = f.x;
-    fi[k] = f.y;
-  }
   zd g = mk(0.0), w[4];
-  int i4 = 3, i0 = 0, ip2 = 4;
   auto capture = [&](int k) {
     if (k == P.i1) w[0] = g;
     if (k == P.ip1 - 1) w[1] = g;
@@ -737,26 +739,34 @@ __device__ zd sphere_integral(const double2 *__restrict__ a, const double2 *__re
     if (k == P.i2) w[3] = g;
   };
   capture(0);
-  for (int i = 1; i <= nr - 1; i++) {
-    if (i > 2 && ip2 <= nr) {
-      const zd f = fval(ip2 - 1);
-      const double xv = sqrt(xval(ip2 - 1));
+  for (int ib = 1; ib < nr; ib += kIntRound) {
+    const int ie = min(ib + kIntRound, nr);
+    if (active) {
+      for (int i = ib + sub; i < ie; i += kIntLanes) {
+        // interval i-1 .. i; the further points are i-2 and i+1, at the ends
+        // of the mesh those that cnewint's ring of four still holds
+        const int kp[4] = {i - 1, i, i == 1 ? 2 : (i == nr - 1 && i > 2 ? i - 3 : i + 1),
+                           i == 1 ? 3 : i - 2};
+        double rs[4], fr[4], fi[4];
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (q == i4) {
-          rs[q] = xv;
+        for (int q = 0; q < 4; q++) {
+          rs[q] = sqrt(xval(kp[q]));
+          const zd f = fval(kp[q]);
           fr[q] = f.x;
           fi[q] = f.y;
         }
+        inc[i - ib] = cnewint_step(rs, fr, fi, ip);
+      }
     }
-    g = g + cnewint_step(rs, fr, fi, i0, ip);
-    capture(i);
-    if (i > 1 && ip2 < nr) {
-      ip2 += 1;
-      i4 = (i4 + 1) & 3;  // the ring rotation i1..i4 advances i4 by one slot
-    }
-    i0 = (i0 + 1) & 3;
+    __syncthreads();
+    if (active && sub == 0)
+      for (int i = ib; i < ie; i++) {
+        g = g + inc[i - ib];
+        capture(i);
+      }
+    __syncthreads();
   }
+  if (!active || sub != 0) return mk(0.0);
   double xw[4];
   xw[0] = xval(P.i1);
   xw[1] = xval(P.ip1 - 1);
@@ -768,7 +778,7 @@ __device__ zd sphere_integral(const double2 *__restrict__ a, const double2 *__re
 
 }  // namespace
 
-__global__ void __launch_bounds__(64) k_green_mt(
+__global__ void __launch_bounds__(kGreenThreads) k_green_mt(
     const double2 *__restrict__ tau00, const double2 *__restrict__ zlr,
     const double2 *__restrict__ jlr, const double *__restrict__ rmesh,
     const GreenPot *__restrict__ pots, const int *__restrict__ pot_of,
@@ -776,74 +786,68 @@ __global__ void __launch_bounds__(64) k_green_mt(
     double2 *__restrict__ dos, double2 *__restrict__ green) {
   // zlr/jlr row of solve b: src_of[b] (radial functions of a single-site
   // batch left on the device) or b
-  __shared__ zd s_int[kGreenSolves][2][4];
+  __shared__ zd s_int[2][4], s_inc[kGreenThreads / kIntLanes][kIntRound];
   const int tid = threadIdx.x;
   const int nl = lmax + 1, kk = nl * nl;
-  const int b0 = blockIdx.x * kGreenSolves;
-  // phase 1: lane 8s + 2l + which runs integral `which` of channel l of solve b0 + s
+  const int b = blockIdx.x;
+  if (b >= nsolve) return;
+  // phase 1: lanes kIntLanes (2l + which) + sub run integral `which` of channel l
   {
-    const int sl = tid >> 3, l = (tid & 7) >> 1, which = tid & 1;
-    const int b = b0 + sl;
-    if (b < nsolve && l < nl) {
-      const GreenPot P = pots[pot_of[b]];
-      const double *rm = rmesh + (long)pot_of[b] * iprpts;
-      const long src = src_of ? src_of[b] : b;
-      const double2 *zl = zlr + (src * nl + l) * iprpts;
-      const double2 *ol = (which ? jlr : zlr) + (src * nl + l) * iprpts;
-      s_int[sl][which][l] = sphere_integral(zl, ol, rm, P);
-    }
+    const int it = tid / kIntLanes, sub = tid % kIntLanes, l = it >> 1, which = it & 1;
+    const GreenPot P = pots[pot_of[b]];
+    const double *rm = rmesh + (long)pot_of[b] * iprpts;
+    const long src = src_of ? src_of[b] : b;
+    const bool active = l < nl;
+    const double2 *zl = zlr + (src * nl + (active ? l : 0)) * iprpts;
+    const double2 *ol = (which ? jlr : zlr) + (src * nl + (active ? l : 0)) * iprpts;
+    const zd v = sphere_integral(active, zl, ol, rm, P, sub, s_inc[it]);
+    if (active && sub == 0) s_int[which][l] = v;
   }
   __syncthreads();
-  // phase 2: mdosms, -(sum pzzck tau - pzjck)/pi, one lane per solve
-  if (tid < kGreenSolves && b0 + tid < nsolve) {
-    const int b = b0 + tid;
-    const double2 *tb = tau00 + (long)b * kk * kk;
+  // phase 2: mdosms, -(sum pzzck tau - pzjck)/pi, one lane
+  const double2 *tb = tau00 + (long)b * kk * kk;
+  if (tid == 0) {
     zd zz = mk(0.0), zj = mk(0.0);
     for (int l = 0; l < nl; l++)
-      for (int m = -l; m <= l; m++) zj = zj + s_int[tid][1][l];
+      for (int m = -l; m <= l; m++) zj = zj + s_int[1][l];
     int lm = 0;
     for (int l = 0; l < nl; l++)
       for (int m = -l; m <= l; m++, lm++) {
         const double2 t = tb[lm + (long)lm * kk];
-        zz = zz + s_int[tid][0][l] * mk(t.x, t.y);
+        zz = zz + s_int[0][l] * mk(t.x, t.y);
       }
     const zd d = -(zz - zj) / 3.14159265358979323846;
     dos[b] = make_double2(spin * d.x, spin * d.y);
   }
-  // phase 3: mgreen, sum over l from lmax down of z (z wt_l - j (2l+1)),
-  // each solve's radial points spread over the 64 lanes
+  // phase 3: mgreen, sum over l from lmax down of z (z wt_l - j (2l+1)), the
+  // radial points spread over the lanes
   if (green) {
-    for (int sl = 0; sl < kGreenSolves; sl++) {
-      const int b = b0 + sl;
-      if (b >= nsolve) break;
-      const double2 *tb = tau00 + (long)b * kk * kk;
-      zd wt[4];
-      int i = kk - 1;
-      for (int l = lmax; l >= 0; l--) {
-        zd sum = mk(0.0);
-        for (int m = -l; m <= l; m++, i--) {
-          const double2 t = tb[i + (long)i * kk];
-          sum = sum + mk(t.x, t.y);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (q == l) wt[q] = sum;
+    zd wt[4];
+    int i = kk - 1;
+    for (int l = lmax; l >= 0; l--) {
+      zd sum = mk(0.0);
+      for (int m = -l; m <= l; m++, i--) {
+        const double2 t = tb[i + (long)i * kk];
+        sum = sum + mk(t.x, t.y);
       }
-      const int jws = pots[pot_of[b]].jws;
-      const long src = src_of ? src_of[b] : b;
-      const double2 *z0 = zlr + src * nl * iprpts, *j0 = jlr + src * nl * iprpts;
-      double2 *gb = green + (long)b * iprpts;
-      for (int ir = tid; ir < jws; ir += blockDim.x) {
-        zd acc = mk(0.0);
 #pragma unroll
-        for (int l = 3; l >= 0; l--) {
-          if (l > lmax) continue;
-          const double2 zv = z0[(long)l * iprpts + ir], jv = j0[(long)l * iprpts + ir];
-          const zd zz = mk(zv.x, zv.y), jj = mk(jv.x, jv.y);
-          acc = acc + zz * (zz * wt[l] - jj * (double)(2 * l + 1));
-        }
-        gb[ir] = make_double2(spin * acc.x, spin * acc.y);
+      for (int q = 0; q < 4; q++)
+        if (q == l) wt[q] = sum;
+    }
+    const int jws = pots[pot_of[b]].jws;
+    const long src = src_of ? src_of[b] : b;
+    const double2 *z0 = zlr + src * nl * iprpts, *j0 = jlr + src * nl * iprpts;
+    double2 *gb = green + (long)b * iprpts;
+    for (int ir = tid; ir < jws; ir += blockDim.x) {
+      zd acc = mk(0.0);
+#pragma unroll
+      for (int l = 3; l >= 0; l--) {
+        if (l > lmax) continue;
+        const double2 zv = z0[(long)l * iprpts + ir], jv = j0[(long)l * iprpts + ir];
+        const zd zz = mk(zv.x, zv.y), jj = mk(jv.x, jv.y);
+        acc = acc + zz * (zz * wt[l] - jj * (double)(2 * l + 1));
       }
+      gb[ir] = make_double2(spin * acc.x, spin * acc.y);
     }
   }
 }
@@ -853,55 +857,53 @@ __global__ void __launch_bounds__(64) k_green_mt(
 // irregular term only on the diagonal ones, then Tr and the x, y, z parts
 // with wx, wy, wz (u_sigma_u.f).  Per solve: tau00_l as four kkrsz x kkrsz
 // blocks (trgtol.f), zlr/jlr as 2 spins x (lmax+1) x iprpts, w = wx, wy, wz.
-// One 64-thread workgroup per two solves: lane 32s + 8isp + 2l + which.
-__global__ void __launch_bounds__(64) k_green_mt_canted(
+// One workgroup per solve, kIntLanes lanes to the integral 8isp + 2l + which.
+__global__ void __launch_bounds__(4 * kGreenThreads) k_green_mt_canted(
     const double2 *__restrict__ tau00, const double2 *__restrict__ zlr,
     const double2 *__restrict__ jlr, const double2 *__restrict__ wxyz,
     const double *__restrict__ rmesh, const GreenPot *__restrict__ pots,
     const int *__restrict__ pot_of, int nsolve, int lmax, int iprpts,
     double2 *__restrict__ dos, double2 *__restrict__ green) {
-  __shared__ zd s_int[2][4][2][4];
-  __shared__ zd s_d[2][4];
+  __shared__ zd s_int[4][2][4], s_inc[4 * kGreenThreads / kIntLanes][kIntRound];
+  __shared__ zd s_d[4];
   const int tid = threadIdx.x;
   const int nl = lmax + 1, kk = nl * nl;
-  const int b0 = blockIdx.x * 2;
+  const int b = blockIdx.x;
+  if (b >= nsolve) return;
   {
-    const int sl = tid >> 5, isp = (tid >> 3) & 3, l = (tid & 7) >> 1, which = tid & 1;
-    const int b = b0 + sl;
+    const int it = tid / kIntLanes, sub = tid % kIntLanes;
+    const int isp = it >> 3, l = (it & 7) >> 1, which = it & 1;
     const bool diag = (isp == 0 || isp == 3);
-    if (b < nsolve && l < nl && (which == 0 || diag)) {
-      const int zsl = (isp & 1), zsr = (isp >> 1);
-      const GreenPot P = pots[pot_of[b]];
-      const double *rm = rmesh + (long)pot_of[b] * iprpts;
-      const double2 *zl = zlr + (((long)b * 2 + zsl) * nl + l) * iprpts;
-      const double2 *ol = (which ? jlr : zlr) + (((long)b * 2 + zsr) * nl + l) * iprpts;
-      s_int[sl][isp][which][l] = sphere_integral(zl, ol, rm, P);
-    }
+    const bool active = l < nl && (which == 0 || diag);
+    const int zsl = (isp & 1), zsr = (isp >> 1), lc = active ? l : 0;
+    const GreenPot P = pots[pot_of[b]];
+    const double *rm = rmesh + (long)pot_of[b] * iprpts;
+    const double2 *zl = zlr + (((long)b * 2 + zsl) * nl + lc) * iprpts;
+    const double2 *ol = (which ? jlr : zlr) + (((long)b * 2 + zsr) * nl + lc) * iprpts;
+    const zd v = sphere_integral(active, zl, ol, rm, P, sub, s_inc[it]);
+    if (active && sub == 0) s_int[isp][which][l] = v;
   }
   __syncthreads();
-  if (tid < 8) {  // mdosms per channel
-    const int sl = tid >> 2, isp = tid & 3, b = b0 + sl;
-    if (b < nsolve) {
-      const bool diag = (isp == 0 || isp == 3);
-      const double2 *tb = tau00 + ((long)b * 4 + isp) * kk * kk;
-      zd zz = mk(0.0), zj = mk(0.0);
-      for (int l = 0; l < nl; l++)
-        for (int m = -l; m <= l; m++) zj = zj + (diag ? s_int[sl][isp][1][l] : mk(0.0));
-      int lm = 0;
-      for (int l = 0; l < nl; l++)
-        for (int m = -l; m <= l; m++, lm++) {
-          const double2 t = tb[lm + (long)lm * kk];
-          zz = zz + s_int[sl][isp][0][l] * mk(t.x, t.y);
-        }
-      zd d = zz;
-      if (diag) d = d - zj;
-      s_d[sl][isp] = -d / 3.14159265358979323846;
-    }
+  if (tid < 4) {  // mdosms per channel
+    const int isp = tid;
+    const bool diag = (isp == 0 || isp == 3);
+    const double2 *tb = tau00 + ((long)b * 4 + isp) * kk * kk;
+    zd zz = mk(0.0), zj = mk(0.0);
+    for (int l = 0; l < nl; l++)
+      for (int m = -l; m <= l; m++) zj = zj + (diag ? s_int[isp][1][l] : mk(0.0));
+    int lm = 0;
+    for (int l = 0; l < nl; l++)
+      for (int m = -l; m <= l; m++, lm++) {
+        const double2 t = tb[lm + (long)lm * kk];
+        zz = zz + s_int[isp][0][l] * mk(t.x, t.y);
+      }
+    zd d = zz;
+    if (diag) d = d - zj;
+    s_d[isp] = -d / 3.14159265358979323846;
   }
   __syncthreads();
-  if (tid < 2 && b0 + tid < nsolve) {  // recombination (green_function.f:150-162)
-    const int b = b0 + tid;
-    const zd d1 = s_d[tid][0], d2 = s_d[tid][1], d3 = s_d[tid][2], d4 = s_d[tid][3];
+  if (tid == 0) {  // recombination (green_function.f:150-162)
+    const zd d1 = s_d[0], d2 = s_d[1], d3 = s_d[2], d4 = s_d[3];
     zd out[4];
     out[0] = d1 + d4;
 #pragma unroll
@@ -914,62 +916,58 @@ __global__ void __launch_bounds__(64) k_green_mt_canted(
     for (int a = 0; a < 4; a++) dos[(long)b * 4 + a] = make_double2(out[a].x, out[a].y);
   }
   if (green) {  // mgreen per channel, then the same recombination per r
-    for (int sl = 0; sl < 2; sl++) {
-      const int b = b0 + sl;
-      if (b >= nsolve) break;
-      zd wt[4][4];
+    zd wt[4][4];
+#pragma unroll
+    for (int isp = 0; isp < 4; isp++) {
+      const double2 *tb = tau00 + ((long)b * 4 + isp) * kk * kk;
+      int i = kk - 1;
+      for (int l = lmax; l >= 0; l--) {
+        zd sum = mk(0.0);
+        for (int m = -l; m <= l; m++, i--) {
+          const double2 t = tb[i + (long)i * kk];
+          sum = sum + mk(t.x, t.y);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (q == l) wt[isp][q] = sum;
+      }
+    }
+    zd w[3][4];
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const double2 v = wxyz[(long)b * 12 + 4 * a + q];
+        w[a][q] = mk(v.x, v.y);
+      }
+    const int jws = pots[pot_of[b]].jws;
+    const double2 *zb = zlr + (long)b * 2 * nl * iprpts, *jb = jlr + (long)b * 2 * nl * iprpts;
+    for (int ir = tid; ir < jws; ir += blockDim.x) {
+      zd g[4];
 #pragma unroll
       for (int isp = 0; isp < 4; isp++) {
-        const double2 *tb = tau00 + ((long)b * 4 + isp) * kk * kk;
-        int i = kk - 1;
-        for (int l = lmax; l >= 0; l--) {
-          zd sum = mk(0.0);
-          for (int m = -l; m <= l; m++, i--) {
-            const double2 t = tb[i + (long)i * kk];
-            sum = sum + mk(t.x, t.y);
-          }
+        const int zsl = (isp & 1), zsr = (isp >> 1);
+        const bool diag = (isp == 0 || isp == 3);
+        zd acc = mk(0.0);
 #pragma unroll
-          for (int q = 0; q < 4; q++)
-            if (q == l) wt[isp][q] = sum;
+        for (int l = 3; l >= 0; l--) {
+          if (l > lmax) continue;
+          const double2 zL = zb[((long)zsl * nl + l) * iprpts + ir];
+          const double2 zR = zb[((long)zsr * nl + l) * iprpts + ir];
+          const double2 jR = jb[((long)zsr * nl + l) * iprpts + ir];
+          zd t = mk(zR.x, zR.y) * wt[isp][l];
+          if (diag) t = mk(zR.x, zR.y) * wt[isp][l] - mk(jR.x, jR.y) * (double)(2 * l + 1);
+          acc = acc + mk(zL.x, zL.y) * t;
         }
+        g[isp] = acc;
       }
-      zd w[3][4];
+      double2 *gb = green + (long)b * 4 * iprpts;
+      const zd g0 = g[0] + g[3];
+      gb[ir] = make_double2(g0.x, g0.y);
 #pragma unroll
-      for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const double2 v = wxyz[(long)b * 12 + 4 * a + q];
-          w[a][q] = mk(v.x, v.y);
-        }
-      const int jws = pots[pot_of[b]].jws;
-      const double2 *zb = zlr + (long)b * 2 * nl * iprpts, *jb = jlr + (long)b * 2 * nl * iprpts;
-      for (int ir = tid; ir < jws; ir += blockDim.x) {
-        zd g[4];
-#pragma unroll
-        for (int isp = 0; isp < 4; isp++) {
-          const int zsl = (isp & 1), zsr = (isp >> 1);
-          const bool diag = (isp == 0 || isp == 3);
-          zd acc = mk(0.0);
-#pragma unroll
-          for (int l = 3; l >= 0; l--) {
-            if (l > lmax) continue;
-            const double2 zL = zb[((long)zsl * nl + l) * iprpts + ir];
-            const double2 zR = zb[((long)zsr * nl + l) * iprpts + ir];
-            const double2 jR = jb[((long)zsr * nl + l) * iprpts + ir];
-            zd t = mk(zR.x, zR.y) * wt[isp][l];
-            if (diag) t = mk(zR.x, zR.y) * wt[isp][l] - mk(jR.x, jR.y) * (double)(2 * l + 1);
-            acc = acc + mk(zL.x, zL.y) * t;
-          }
-          g[isp] = acc;
-        }
-        double2 *gb = green + (long)b * 4 * iprpts;
-        const zd g0 = g[0] + g[3];
-        gb[ir] = make_double2(g0.x, g0.y);
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-          const zd v = g[0] * w[a][0] + g[1] * w[a][2] + g[2] * w[a][1] + g[3] * w[a][3];
-          gb[(long)(1 + a) * iprpts + ir] = make_double2(v.x, v.y);
-        }
+      for (int a = 0; a < 3; a++) {
+        const zd v = g[0] * w[a][0] + g[1] * w[a][2] + g[2] * w[a][1] + g[3] * w[a][3];
+        gb[(long)(1 + a) * iprpts + ir] = make_double2(v.x, v.y);
       }
     }
   }
