@@ -9,8 +9,8 @@
 //   d tau00 = sum_i R_i dt_i C_i + R_0 dt_0   (k_tau_grad)
 // with R_i = (M^-1)_{0i} the central block row and C_i = (G M^-1)_{i0} t_0.
 //
-// Factorization (tau_lu.hip with full_lu = 1 and every diagonal-tile inverse
-// kept): M = Lt Ut, Lt block lower with diagonal tiles P_s^T L_ss, Ut block
+// Factorization (tau_lu.hip, the last tile by k_lu_diag too, and every
+// diagonal-tile inverse kept): M = Lt Ut, Lt block lower with diagonal tiles P_s^T L_ss, Ut block
 // upper with diagonal tiles U_ss; Lt_ts (t > s) and Ut_ts (t < s) sit in M.
 // M^-1 = Ut^-1 Lt^-1 is formed in place in one Ns x Ns buffer Y:
 //   forward,  s = 0..nt-1:  Y_ss = L_ss^-1 P_s,  Y_sc = L_ss^-1 P_s Y_sc (c < s)
@@ -60,7 +60,7 @@ __device__ __forceinline__ void tile_update(const GZ *__restrict__ A, const GZ *
         q.p[1][bj][bi][r] = 0.0;
         q.p[2][bj][bi][r] = -c.x - c.y;
       }
-  wave_gemm3m_k(A + wr, B + ld * wc, ld, kTile / 4, q);
+  wave_gemm3m_k<2>(A + wr, B + ld * wc, ld, kTile / 4, q);
 #pragma unroll
   for (int bj = 0; bj < 2; bj++)
 #pragma unroll
@@ -107,13 +107,13 @@ __global__ __launch_bounds__(256) void k_inv_fwd_panel(const SolveDesc *__restri
   Acc3<double> q;
   zero_acc(q);
   // A(i,k) = L^-1(wr+i, k), unit lower; B(k,j) = (P Y_sc)(k, wc+j)
-  wave_gemm3m<double>([&](int i, int k) {
+  wave_gemm3m<double, 2>([&](int i, int k) {
                                int ii = wr + i;
                                Z v = Z{ii == k ? 1.0 : 0.0, 0.0};
                                if (ii > k) v = inv[ii + kTile * k];
                                return v;
                              },
-                             [&](int k, int j) { return Ts[wc + j][k]; }, q);
+                             [&](int k, int j) { return Ts[wc + j][k]; }, kTile / 4, q);
   store_acc(tile + wr + ld * wc, ld, q);
 }
 
@@ -152,13 +152,13 @@ __global__ __launch_bounds__(256) void k_inv_bwd_panel(const SolveDesc *__restri
   Acc3<double> q;
   zero_acc(q);
   // A(i,k) = U^-1(wr+i, k), upper incl. diagonal; B(k,j) = Y_sc(k, wc+j)
-  wave_gemm3m<double>([&](int i, int k) {
+  wave_gemm3m<double, 2>([&](int i, int k) {
                                int ii = wr + i;
                                Z v = Z{0.0, 0.0};
                                if (k >= ii) v = inv[ii + kTile * k];
                                return v;
                              },
-                             [&](int k, int j) { return Ts[wc + j][k]; }, q);
+                             [&](int k, int j) { return Ts[wc + j][k]; }, kTile / 4, q);
   store_acc(tile + wr + ld * wc, ld, q);
 }
 

@@ -39,13 +39,11 @@ __global__ void k_assemble_from_g(const SolveDesc *, const double2 *, long);
 __global__ void k_pad_identity(const SolveDesc *);
 template <class T>
 __global__ void k_lu_diag(const SolveDesc *, int);
+template <class T, int N>
+__global__ void k_lu_panel(const SolveDesc *, int, int, int);
 template <class T>
-__global__ void k_lu_panel(const SolveDesc *, int);
-template <class T>
-__global__ void k_lu_update(const SolveDesc *, int, int);
-template <class T>
-__global__ void k_lu_cross(const SolveDesc *, int, int);
-template <class T>
+__global__ void k_lu_cross_diag(const SolveDesc *, int, int);
+template <class T, int N>
 __global__ void k_lu_trail(const SolveDesc *, int, int);
 template <class T>
 __global__ void k_lu_last(const SolveDesc *);
@@ -464,103 +462,85 @@ int copy_square(void *dst, long ldd, const void *src, long lds, long n, hipMemcp
 // Steps per trailing update: with the split-FP16 update the context's
 // split_group (4, 8 or 16, default 8: the trailing matrix is read and
 // written once per group, the fused panels of a group's later steps apply
-// up to group - 1 earlier steps), two otherwise.
-inline int lu_group(const lsmsx_ctx *c, bool split_f16) { return split_f16 ? c->split_group : 2; }
+// up to group - 1 earlier steps), four otherwise: against two, the FP64
+// trailing update reads and writes C half as often (64 solves N = 2160: 29.1 ->
+// 27.0 ms, six of N = 4384: 24.1 -> 22.7; eight steps give 26.2 and 22.4), and
+// the longer cross updates cost a single solve of N = 2160 little (2.23 -> 2.29
+// ms; eight steps 2.51).
+inline int lu_group(const lsmsx_ctx *c, bool split_f16) { return split_f16 ? c->split_group : 4; }
 
-// Launch the blocked LU over a chunk of nb solves already in solver layout
-// (each descriptor's group = lu_group(c, split_f16)): steps taken in groups
-// g .. g+G-1 -- panels of g, then for each later step t of the group a cross
-// update of tile row/column t with the group's earlier steps and the panels
-// of t (on the split-FP16 path the cross update is fused into the panel
-// kernel, and only the diagonal tile's has a kernel of its own) -- then one
-// K = 64 G trailing update, so the trailing matrix is read and written once
-// per group.
+// Whether a launch over `tiles` 64x64 tiles takes a quarter of a tile per
+// workgroup, with the same arithmetic per entry: below one tile per compute
+// unit the whole tiles leave compute units idle and a launch takes as long as
+// one tile (a solve of N = 2160: 2.68 -> 2.29 ms, of n = 999: 1.59 -> 1.40 ms);
+// above, the quarters' second load of the operands costs more than it gives
+// (2.33 ms with the line at 1024 panel and 512 trailing tiles, 2.40 at twice
+// that; eight solves of N = 944: 3.14, 3.17, 3.23 ms).
+inline bool lu_small_grid(long tiles) { return tiles <= 256; }
+
+// Steps 0 .. nt_max-2 of the blocked LU over a chunk of nb solves already in
+// solver layout (each descriptor's group = lu_group(c, split_f16)), taken in
+// groups g .. g+G-1: for each step t of the group the cross update of the
+// diagonal tile (steps g .. t-1), its factorization, and the panel with the
+// cross update of its column and row fused in; then one K = 64 G trailing
+// update with the whole group, so that the trailing matrix is read and
+// written once per group.
+template <class T>
+int launch_lu_steps(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool split_f16,
+                    hipStream_t st) {
+  const int swz = (c->sched & LSMSX_SCHED_XCD_SWIZZLE) ? 1 : 0;
+  const int G = lu_group(c, split_f16);
+  for (int s = 0; s < nt_max - 1; s += G) {
+    const int b = std::min(s + G - 1, nt_max - 2);  // the group's last step, largest solve
+    for (int t = s; t <= b; t++) {
+      const int u = t - s, np = 2 * (nt_max - 1 - t);
+      if (u > 0) {
+        ProfScope p(c, 9);
+        if (split_f16)
+          hipLaunchKernelGGL(k_lu_cross_diag_h, dim3(nb), dim3(128), 0, st, dd, s, u);
+        else
+          hipLaunchKernelGGL(k_lu_cross_diag<T>, dim3(4, nb), dim3(256), 0, st, dd, s, u);
+      }
+      if (int r = check_launch("k_lu_cross_diag")) return r;
+      {
+        ProfScope p(c, 1);
+        hipLaunchKernelGGL(k_lu_diag<T>, dim3(nb), dim3(256), 0, st, dd, t);
+      }
+      {
+        ProfScope p(c, 2);
+        if (split_f16)
+          hipLaunchKernelGGL(k_lu_panel_h, dim3(np, nb), dim3(256), 0, st, dd, t, u, swz);
+        else if (lu_small_grid((long)np * nb))
+          hipLaunchKernelGGL((k_lu_panel<T, 1>), dim3(4 * np, nb), dim3(256), 0, st, dd, t, u, swz);
+        else
+          hipLaunchKernelGGL((k_lu_panel<T, 2>), dim3(np, nb), dim3(256), 0, st, dd, t, u, swz);
+      }
+      if (int r = check_launch("k_lu_diag/k_lu_panel")) return r;
+    }
+    const int nrest = nt_max - 1 - b;
+    {
+      ProfScope p(c, 3);
+      if (split_f16)
+        hipLaunchKernelGGL(k_lu_trail_h, dim3(((nrest + 1) / 2) * ((nrest + 1) / 2), nb),
+                           dim3(512), 0, st, dd, s, swz);
+      else if (lu_small_grid((long)nrest * nrest * nb))
+        hipLaunchKernelGGL((k_lu_trail<T, 1>), dim3(4 * nrest * nrest, nb), dim3(256), 0, st, dd,
+                           s, swz);
+      else
+        hipLaunchKernelGGL((k_lu_trail<T, 2>), dim3(nrest * nrest, nb), dim3(256), 0, st, dd, s,
+                           swz);
+    }
+    if (int r = check_launch("k_lu_trail")) return r;
+  }
+  return 0;
+}
+
+// The whole LU of a chunk, the last tile with k_lu_last.
 template <class T>
 int launch_lu(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool split_f16 = false,
               hipStream_t st = nullptr) {
   if (!st) st = c->stream;
-  const int swz = (c->sched & LSMSX_SCHED_XCD_SWIZZLE) ? 1 : 0;
-  const int G = lu_group(c, split_f16);
-  auto diag_panel = [&](int s) -> int {
-    const int nrest = nt_max - 1 - s;
-    if (nrest <= 0) return 0;
-    {
-      ProfScope p(c, 1);
-      hipLaunchKernelGGL(k_lu_diag<T>, dim3(nb), dim3(256), 0, st, dd, s);
-    }
-    {
-      ProfScope p(c, 2);
-      hipLaunchKernelGGL(k_lu_panel<T>, dim3(2 * nrest, nb), dim3(256), 0, st, dd, s);
-    }
-    return check_launch("k_lu_diag/k_lu_panel");
-  };
-  // the steps s .. s+n-1 of a group: n <= H, panels and crosses step by
-  // step; otherwise the first half, the strip update of the second half's
-  // columns and rows with the first half, then the second half
-  if (split_f16) {
-    // split-FP16 path: for each step t of a group, the cross update of the
-    // diagonal tile (steps g .. t-1), its factorization, and the panel with
-    // the cross update of its column and row fused in; then the trailing
-    // update with the whole group
-    for (int s = 0; s < nt_max - 1; s += G) {
-      const int b = std::min(s + G - 1, nt_max - 2);
-      for (int t = s; t <= b; t++) {
-        const int u = t - s;
-        if (u > 0) {
-          ProfScope p(c, 9);
-          hipLaunchKernelGGL(k_lu_cross_diag_h, dim3(nb), dim3(128), 0, st, dd, s, u);
-        }
-        if (int r = check_launch("k_lu_cross_diag_h")) return r;
-        {
-          ProfScope p(c, 1);
-          hipLaunchKernelGGL(k_lu_diag<T>, dim3(nb), dim3(256), 0, st, dd, t);
-        }
-        {
-          ProfScope p(c, 2);
-          hipLaunchKernelGGL(k_lu_panel_h, dim3(2 * (nt_max - 1 - t), nb), dim3(256), 0, st, dd,
-                             t, u, swz);
-        }
-        if (int r = check_launch("k_lu_diag/k_lu_panel_h")) return r;
-      }
-      const int nrest = nt_max - 1 - b;
-      if (nrest > 0) {
-        ProfScope p(c, 3);
-        hipLaunchKernelGGL(k_lu_trail_h, dim3(((nrest + 1) / 2) * ((nrest + 1) / 2), nb),
-                           dim3(512), 0, st, dd, s, swz);
-      }
-      if (int r = check_launch("k_lu_trail_h")) return r;
-    }
-    {
-      ProfScope p(c, 4);
-      hipLaunchKernelGGL(k_lu_last<T>, dim3(nb), dim3(256), 0, st, dd);
-    }
-    return check_launch("k_lu_last");
-  }
-  // steps s .. s+n-1 of a group: panels and crosses step by step
-  auto block = [&](int s, int n) -> int {
-    if (int r = diag_panel(s)) return r;
-    for (int u = 1; u < n && s + u < nt_max - 1; u++) {
-      {
-        ProfScope p(c, 9);
-        const int n1 = nt_max - s - u;
-        hipLaunchKernelGGL(k_lu_cross<T>, dim3(2 * n1 - 1, nb), dim3(256), 0, st, dd, s, u);
-      }
-      if (int r = check_launch("k_lu_cross")) return r;
-      if (int r = diag_panel(s + u)) return r;
-    }
-    return 0;
-  };
-  for (int s = 0; s < nt_max - 1; s += G) {
-    if (int r = block(s, G)) return r;
-    const int last = std::min(s + G - 1, nt_max - 2);  // the group's last step, largest solve
-    const int nrest = nt_max - 1 - last;
-    if (nrest > 0) {
-      ProfScope p(c, 3);
-      hipLaunchKernelGGL(k_lu_trail<T>, dim3(nrest * nrest, nb), dim3(256), 0, st, dd, s,
-                         swz);
-    }
-    if (int r = check_launch("k_lu_trail")) return r;
-  }
+  if (int r = launch_lu_steps<T>(c, dd, nb, nt_max, split_f16, st)) return r;
   {
     ProfScope p(c, 4);
     hipLaunchKernelGGL(k_lu_last<T>, dim3(nb), dim3(256), 0, st, dd);
@@ -1227,23 +1207,10 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
 // LU of every tile (last one included, all diagonal-tile inverses kept) and
 // the in-place explicit inverse M^-1 in d.Minv, for nb solves in solver layout.
 int launch_inverse(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max) {
-  for (int s = 0; s < nt_max; s++) {
-    int nrest = nt_max - 1 - s;
-    {
-      ProfScope p(c, 1);
-      hipLaunchKernelGGL(k_lu_diag<double>, dim3(nb), dim3(256), 0, c->stream, dd, s);
-    }
-    if (nrest > 0) {
-      {
-        ProfScope p(c, 2);
-        hipLaunchKernelGGL(k_lu_panel<double>, dim3(2 * nrest, nb), dim3(256), 0, c->stream, dd, s);
-      }
-      {
-        ProfScope p(c, 3);
-        hipLaunchKernelGGL(k_lu_update<double>, dim3(nrest * nrest, nb), dim3(256), 0, c->stream,
-                           dd, s, 0);
-      }
-    }
+  if (int r = launch_lu_steps<double>(c, dd, nb, nt_max, false, c->stream)) return r;
+  {
+    ProfScope p(c, 1);
+    hipLaunchKernelGGL(k_lu_diag<double>, dim3(nb), dim3(256), 0, c->stream, dd, kLastStep);
   }
   if (int r = check_launch("full LU")) return r;
   ProfScope p(c, 7);
@@ -1396,7 +1363,6 @@ int run_adjoint(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
       d.pad = Ns - N;
       d.nt = Ns / kTile;
       d.group = lu_group(c, false);
-      d.full_lu = 1;
       d.inv = c->inv.p + ioff;
       d.inv_stride = kTile * kTile;
       ioff += (long)d.nt * kTile * kTile;
@@ -2204,7 +2170,6 @@ int lsmsx_tau_full(lsmsx_ctx *c, int atom_id, int ispin, int iie, const double *
   d.pad = Ns - N;
   d.nt = nt;
   d.group = lu_group(c, false);
-  d.full_lu = 1;
   d.inv = c->inv.p;
   d.inv_stride = kTile * kTile;
   d.perm = c->perm.p;

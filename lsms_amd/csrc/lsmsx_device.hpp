@@ -15,6 +15,7 @@ constexpr int kTile = 64;     // LU tile / panel width
 constexpr int kMaxLmax = 3;   // tables and per-site blocks sized for lmax <= 3
 constexpr int kMaxKkr = (kMaxLmax + 1) * (kMaxLmax + 1);
 constexpr int kPlaneHalves = 4 * kTile * kTile;  // one tile's four FP16 planes
+constexpr int kLastStep = -1001;  // k_lu_diag's step value for each solve's last tile
 constexpr int kIrFirstSweep = -1000;  // k_ir_step's step value for the first forward sweep
 // k_ir_sweep (one launch per refinement sweep, kc = 16): waves per workgroup
 // and the largest number of 64-row tiles per solve it takes
@@ -86,7 +87,6 @@ struct SolveDesc {
   void *ihp;              // 2 tiles x 4 planes x 64 x 64 halves
   int *ihe;               // 2
   // explicit inverse (full tau, Lloyd term, adjoint of tau00)
-  int full_lu;            // 1: the last tile is factored by k_lu_diag like every other tile
   double2 *Minv;          // Ns x Ns (leading dim ld): M^-1 in the solver layout
   double dprel_re, dprel_im;  // d prel / dE
   double2 *gx;            // Ns x kc: the rows of site i hold (G X)_i, X = M^-1 [0; t0]

@@ -118,103 +118,88 @@ __device__ __forceinline__ long tile_ld(const SolveDesc &d) { return d.tiled ? k
 // L2/LDS into registers in MFMA layout (a-operand lane value B(k0+kq, j0+li),
 // b-operand lane value A(i0+li, k0+kq)), loaded ahead of the MFMAs; no LDS
 // staging and no barriers, so the waves of a CU run independently.
-template <class T>
+// N: a wave's block is 16N x 16N (2: the 32x32 block above; 1: 16x16, for
+// launches that would leave compute units idle otherwise).
+template <class T, int N = 2>
 struct Acc3 {
-  Acc4<T> p[3][2][2];
+  Acc4<T> p[3][N][N];
 };
 
-// One k-step (12 MFMAs) of the 3M product from operands already in registers.
-template <class T>
-__device__ __forceinline__ void gemm3m_step(CxT<T> (&av)[2], CxT<T> (&bv)[2], Acc3<T> &q) {
-  T as[2], bs[2];
+// One k-step (3 N^2 MFMAs) of the 3M product from operands already in registers.
+template <class T, int N>
+__device__ __forceinline__ void gemm3m_step(CxT<T> (&av)[N], CxT<T> (&bv)[N], Acc3<T, N> &q) {
+  T as[N], bs[N];
 #pragma unroll
-  for (int t = 0; t < 2; t++) {
+  for (int t = 0; t < N; t++) {
     as[t] = av[t].x + av[t].y;
     bs[t] = bv[t].x + bv[t].y;
   }
 #pragma unroll
-  for (int bj = 0; bj < 2; bj++)
+  for (int bj = 0; bj < N; bj++)
 #pragma unroll
-    for (int bi = 0; bi < 2; bi++) q.p[0][bj][bi] = mfma4(bv[bj].x, av[bi].x, q.p[0][bj][bi]);
+    for (int bi = 0; bi < N; bi++) q.p[0][bj][bi] = mfma4(bv[bj].x, av[bi].x, q.p[0][bj][bi]);
 #pragma unroll
-  for (int bj = 0; bj < 2; bj++)
+  for (int bj = 0; bj < N; bj++)
 #pragma unroll
-    for (int bi = 0; bi < 2; bi++) q.p[1][bj][bi] = mfma4(bv[bj].y, av[bi].y, q.p[1][bj][bi]);
+    for (int bi = 0; bi < N; bi++) q.p[1][bj][bi] = mfma4(bv[bj].y, av[bi].y, q.p[1][bj][bi]);
 #pragma unroll
-  for (int bj = 0; bj < 2; bj++)
+  for (int bj = 0; bj < N; bj++)
 #pragma unroll
-    for (int bi = 0; bi < 2; bi++) q.p[2][bj][bi] = mfma4(bs[bj], as[bi], q.p[2][bj][bi]);
+    for (int bi = 0; bi < N; bi++) q.p[2][bj][bi] = mfma4(bs[bj], as[bi], q.p[2][bj][bi]);
 }
 
-// Operand loads run PF k-steps ahead of the MFMAs: one step (768 MFMA
-// cycles) covers an L2 round trip in FP64; FP32 steps (384 cycles) with both
-// operands in L2 load three steps ahead (callers whose occupancy matters more
-// pass PF = 1).
-template <class T, int PF = (sizeof(T) == 4 ? 3 : 1), class FA, class FB>
-__device__ __forceinline__ void wave_gemm3m(FA fa, FB fb, Acc3<T> &q) {
+// q += A B over nk k-steps of four.  Operand loads run PF (3 or 7) k-steps
+// ahead of the MFMAs; nk is a multiple of PF + 1.  Three of a 32x32 block (768
+// MFMA cycles each in FP64, 432 in FP32) cover an L2 round trip; those of a
+// 16x16 block are a quarter as long.
+template <class T, int N, int PF = 3, class FA, class FB>
+__device__ __forceinline__ void wave_gemm3m(FA fa, FB fb, int nk, Acc3<T, N> &q) {
   typedef CxT<T> V;
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
-  if constexpr (PF == 1) {
-    V a[2], b[2], an[2], bn[2];
+  V a[PF + 1][N], b[PF + 1][N];
+  auto load = [&](int slot, int ks) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-      a[t] = fa(16 * t + li, kq);
-      b[t] = fb(kq, 16 * t + li);
+    for (int t = 0; t < N; t++) {
+      a[slot][t] = fa(16 * t + li, 4 * ks + kq);
+      b[slot][t] = fb(4 * ks + kq, 16 * t + li);
     }
-#pragma unroll 2
-    for (int k0 = 0; k0 < kTile; k0 += 4) {
-      if (k0 + 4 < kTile) {
+  };
+  auto step = [&](int slot) __attribute__((always_inline)) {
+    V av[N], bv[N];
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-          an[t] = fa(16 * t + li, k0 + 4 + kq);
-          bn[t] = fb(k0 + 4 + kq, 16 * t + li);
-        }
-      }
-      gemm3m_step<T>(a, b, q);
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        a[t] = an[t];
-        b[t] = bn[t];
-      }
+    for (int t = 0; t < N; t++) {
+      av[t] = a[slot][t];
+      bv[t] = b[slot][t];
     }
-    return;
+    gemm3m_step<T, N>(av, bv, q);
+  };
+#pragma unroll
+  for (int i = 0; i < PF; i++) load(i, i);
+  int ks = 0;
+#pragma unroll 1
+  for (; ks < nk - PF - 1; ks += PF + 1) {
+#pragma unroll
+    for (int i = 0; i <= PF; i++) {
+      load((i + PF) & PF, ks + i + PF);
+      step(i);
+    }
   }
-  constexpr int NS = kTile / 4;
-  V a[PF + 1][2], b[PF + 1][2];
+  load(PF, ks + PF);
 #pragma unroll
-  for (int p = 0; p < PF; p++)
-#pragma unroll
-    for (int t = 0; t < 2; t++) {
-      a[p][t] = fa(16 * t + li, 4 * p + kq);
-      b[p][t] = fb(4 * p + kq, 16 * t + li);
-    }
-#pragma unroll
-  for (int ks = 0; ks < NS; ks++) {
-    if (ks + PF < NS) {
-      const int p = (ks + PF) % (PF + 1);
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        a[p][t] = fa(16 * t + li, 4 * (ks + PF) + kq);
-        b[p][t] = fb(4 * (ks + PF) + kq, 16 * t + li);
-      }
-    }
-    const int c = ks % (PF + 1);
-    V av[2] = {a[c][0], a[c][1]}, bv[2] = {b[c][0], b[c][1]};
-    gemm3m_step<T>(av, bv, q);
-  }
+  for (int i = 0; i <= PF; i++) step(i);
 }
 
-// q += A B over 4 nk values of k in FP64 (nk a multiple of 4), A(i, k) at A[i +
-// ld k], B(k, j) at B[k + ld j], both wave-uniform.  An FP64 MFMA holds its
-// SIMD's VALU for all of its 64 cycles, whichever wave the VALU work is of, so
-// every other instruction of the loop adds to its time: the operands come by
-// buffer loads whose k offset is scalar, three k-steps ahead, and the only VALU
-// work left of a step are the four sums of the 3M form (through pointers, with
-// A negated, it was 17 instructions; 64 solves of N = 2160: trailing updates
-// 23.8 -> 22.4 ms, 75% of the MFMA cycles at the clock the card holds there,
-// the rest being the loads and stores of C at K = 128).
+// The same in FP64 for operands in global memory, nk a multiple of 8: A(i, k)
+// at A[i + ld k], B(k, j) at B[k + ld j], both wave-uniform.  An FP64 MFMA
+// holds its SIMD's VALU for all of its 64 cycles, whichever wave the VALU work
+// is of, so every other instruction of the loop adds to its time: the
+// operands come by buffer loads whose k offset is scalar, and the only VALU
+// work left of a step are the sums of the 3M form (through pointers, with A
+// negated, it was 17 instructions; 64 solves of N = 2160: trailing updates
+// 23.8 -> 22.4 ms at K = 128).
+template <int N>
 __device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<double> *B, long ld,
-                                              int nk, Acc3<double> &q) {
+                                              int nk, Acc3<double, N> &q) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef unsigned b128 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
@@ -222,51 +207,216 @@ __device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<do
   const auto ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, kRange, kFlags);
   const auto rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, kRange, kFlags);
   const int ld16 = (int)ld * 16;
-  const int va = 16 * li + ld16 * kq;           // A(li, kq), and 16 rows below
-  const int vb = 16 * kq + ld16 * li, vb2 = vb + 16 * ld16;  // B(kq, li), B(kq, 16 + li)
-  constexpr int PF = 3;
-  double2 a[PF + 1][2], b[PF + 1][2];
+  const int va = 16 * li + ld16 * kq;  // A(li, kq)
+  int vb[N];                           // B(kq, 16 t + li)
+#pragma unroll
+  for (int t = 0; t < N; t++) vb[t] = 16 * kq + ld16 * (16 * t + li);
+  constexpr int PF = N == 2 ? 3 : 7;
+  double2 a[PF + 1][N], b[PF + 1][N];
   auto get = [](b128 x) __attribute__((always_inline)) {
     return double2{__hiloint2double(x[1], x[0]), __hiloint2double(x[3], x[2])};
   };
   auto load = [&](int slot, int ks) __attribute__((always_inline)) {
     const int sa = 4 * ks * ld16, sb = 64 * ks;
-    a[slot][0] = get(__builtin_amdgcn_raw_buffer_load_b128(ra, va, sa, 0));
-    a[slot][1] = get(__builtin_amdgcn_raw_buffer_load_b128(ra, va + 256, sa, 0));
-    b[slot][0] = get(__builtin_amdgcn_raw_buffer_load_b128(rb, vb, sb, 0));
-    b[slot][1] = get(__builtin_amdgcn_raw_buffer_load_b128(rb, vb2, sb, 0));
+#pragma unroll
+    for (int t = 0; t < N; t++)
+      a[slot][t] = get(__builtin_amdgcn_raw_buffer_load_b128(ra, va + 256 * t, sa, 0));
+#pragma unroll
+    for (int t = 0; t < N; t++)
+      b[slot][t] = get(__builtin_amdgcn_raw_buffer_load_b128(rb, vb[t], sb, 0));
   };
   auto step = [&](int slot) __attribute__((always_inline)) {
-    double2 av[2] = {a[slot][0], a[slot][1]}, bv[2] = {b[slot][0], b[slot][1]};
-    gemm3m_step<double>(av, bv, q);
+    double2 av[N], bv[N];
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+      av[t] = a[slot][t];
+      bv[t] = b[slot][t];
+    }
+    gemm3m_step<double, N>(av, bv, q);
   };
 #pragma unroll
   for (int i = 0; i < PF; i++) load(i, i);
   int ks = 0;
 #pragma unroll 1
-  for (; ks < nk - 4; ks += 4) {
+  for (; ks < nk - PF - 1; ks += PF + 1) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      load((i + PF) & 3, ks + i + PF);
+    for (int i = 0; i <= PF; i++) {
+      load((i + PF) & PF, ks + i + PF);
       step(i);
     }
   }
   load(PF, ks + PF);
 #pragma unroll
-  for (int i = 0; i < 4; i++) step(i);
+  for (int i = 0; i <= PF; i++) step(i);
 #endif
 }
 
-template <class T>
-__device__ __forceinline__ void zero_acc(Acc3<T> &q) {
+// q += sum_{u < ns} A_u B_u over 64-wide tiles: A_u = A + u sa, B_u = B + u sb
+// (FP64: consecutive in k, so that ns tiles are one product).
+template <class T, int N>
+__device__ __forceinline__ void tile_products(const GCx<T> *A, long sa, const GCx<T> *B, long sb,
+                                              long ld, int ns, Acc3<T, N> &q) {
+  if constexpr (sizeof(T) == 8) {
+    if (ns > 0) wave_gemm3m_k<N>(A, B, ld, 16 * ns, q);
+  } else {
+    for (int u = 0; u < ns; u++, A += sa, B += sb)
+      wave_gemm3m<T, N, N == 2 ? 3 : 7>([&](int i, int k) { return ldg<T>(A + (i + ld * k)); },
+                                        [&](int k, int j) { return ldg<T>(B + (k + ld * j)); },
+                                        kTile / 4, q);
+  }
+}
+
+template <class T, int N>
+__device__ __forceinline__ void zero_acc(Acc3<T, N> &q) {
 #pragma unroll
   for (int m = 0; m < 3; m++)
 #pragma unroll
-    for (int bj = 0; bj < 2; bj++)
+    for (int bj = 0; bj < N; bj++)
 #pragma unroll
-      for (int bi = 0; bi < 2; bi++)
+      for (int bi = 0; bi < N; bi++)
 #pragma unroll
         for (int r = 0; r < 4; r++) q.p[m][bj][bi][r] = T(0);
+}
+
+// -C enters the 3M sums at the start (q1 = -Cre, q2 = 0, q3 = -(Cre + Cim)),
+// so that C - A B = (q2 - q1, q1 + q2 - q3) at the end: C is read and written
+// once however many products are taken, and no operand is negated.
+template <class T, int N>
+__device__ __forceinline__ void set_minus(Acc3<T, N> &q, int bj, int bi, int r, T re, T im) {
+  q.p[0][bj][bi][r] = -re;
+  q.p[1][bj][bi][r] = T(0);
+  q.p[2][bj][bi][r] = -re - im;
+}
+template <class T, int N>
+__device__ __forceinline__ CxT<T> minus_value(const Acc3<T, N> &q, int bj, int bi, int r) {
+  CxT<T> v;
+  v.x = q.p[1][bj][bi][r] - q.p[0][bj][bi][r];
+  v.y = q.p[0][bj][bi][r] + q.p[1][bj][bi][r] - q.p[2][bj][bi][r];
+  return v;
+}
+template <class T, int N>
+__device__ __forceinline__ CxT<T> plus_value(const Acc3<T, N> &q, int bj, int bi, int r) {
+  CxT<T> v;
+  v.x = q.p[0][bj][bi][r] - q.p[1][bj][bi][r];
+  v.y = q.p[2][bj][bi][r] - q.p[0][bj][bi][r] - q.p[1][bj][bi][r];
+  return v;
+}
+
+// What a panel tile does with the inverse of the step's diagonal tile.
+enum PanelOp {
+  kRightU,  // X = C' U^-1: a tile below the diagonal tile
+  kLeftL,   // X = L^-1 P C': a tile right of it, or of the inverse's forward half
+  kLeftU    // X = U^-1 C': a tile of the inverse's backward half
+};
+
+// LDS of panel_op: C' (a tile, or 16 rows or columns of one) and the pivots.
+template <class T, int N>
+struct PanelLds {
+  __align__(16) CxT<T> c[kTile * ((N == 2 ? kTile : 16) + 1)];
+  int rowpos[kTile];
+};
+
+// One panel tile or a piece of it by a 256-thread workgroup:
+//   C' = [C] - sum_{u < ns} A_u B_u,   X = C' U^-1, L^-1 P C' or U^-1 C',
+// so that the tile takes the earlier steps of its group (of the whole inverse)
+// on the way into its panel product, with no launch and no pass over C of
+// their own.  N = 2: the whole 64x64 tile, a 32x32 block per wave, A read at
+// 64 rows and B at 64 columns.  N = 1: 16 rows (kRightU) or 16 columns of it,
+// which the product with the inverse leaves independent of the others, a
+// 16x16 block per wave: a quarter of the time per tile on four times the
+// workgroups, at twice the operand loads per MFMA.  `piece` = 0..3 then.
+// perm: the pivots of kLeftL; identity: C' = the identity tile (nothing else).
+template <class T, int N, PanelOp OP>
+__device__ __forceinline__ void panel_op(GCx<T> *__restrict__ C, bool load_c, bool identity,
+                                         const GCx<T> *A, long sa, const GCx<T> *B, long sb,
+                                         long ld, int ns, const GCx<T> *__restrict__ inv,
+                                         const LSMSX_GLOBAL int *__restrict__ perm, int piece,
+                                         PanelLds<T, N> &lds) {
+  typedef CxT<T> V;
+  constexpr bool RIGHT = OP == kRightU;
+  // Ts[column][row] of C' (rows in pivot order for kLeftL)
+  constexpr int CR = N == 2 || !RIGHT ? kTile : 16, CC = N == 2 || RIGHT ? kTile : 16;
+  static_assert(sizeof(V) * CC * (CR + 1) <= sizeof(lds.c), "LDS tile");
+  V(*Ts)[CR + 1] = reinterpret_cast<V(*)[CR + 1]>(lds.c);
+  int *rowpos = lds.rowpos;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the wave's block in the piece, and the piece in the tile
+  const int wr = N == 2 ? 32 * (w & 1) : RIGHT ? 0 : 16 * w;
+  const int wc = N == 2 ? 32 * (w >> 1) : RIGHT ? 16 * w : 0;
+  const int r0 = N == 2 || !RIGHT ? 0 : 16 * piece, c0 = N == 2 || RIGHT ? 0 : 16 * piece;
+  if (OP == kLeftL) {
+    if (tid < kTile) rowpos[perm[tid]] = tid;
+    __syncthreads();
+  }
+  GCx<T> *Cw = C + (r0 + wr) + ld * (c0 + wc);
+  Acc3<T, N> q;
+#pragma unroll
+  for (int bj = 0; bj < N; bj++)
+#pragma unroll
+    for (int bi = 0; bi < N; bi++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int i = 16 * bi + li, j = 16 * bj + acc_row<T>(kq, r);
+        V c = czero<V>();
+        if (load_c) c = ldg<T>(Cw + (i + ld * j));
+        else if (identity) c.x = r0 + wr + i == c0 + wc + j ? T(1) : T(0);
+        set_minus<T, N>(q, bj, bi, r, c.x, c.y);
+      }
+  tile_products<T, N>(A + (r0 + wr), sa, B + ld * (c0 + wc), sb, ld, ns, q);
+#pragma unroll
+  for (int bj = 0; bj < N; bj++)
+#pragma unroll
+    for (int bi = 0; bi < N; bi++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int i = wr + 16 * bi + li, j = wc + 16 * bj + acc_row<T>(kq, r);
+        Ts[j][OP == kLeftL ? rowpos[i] : i] = minus_value<T, N>(q, bj, bi, r);
+      }
+  __syncthreads();
+  zero_acc(q);
+  // the triangular factor's zero blocks are left out: of a 16-column (row)
+  // strip only the k-steps up to its diagonal block, or from it on
+  const int lim = RIGHT ? wc + 16 * N : wr + 16 * N;
+  if constexpr (OP == kRightU) {
+    // A(i,k) = C'(wr+i, k); B(k,j) = U^-1(k, wc+j), upper incl. diagonal
+    wave_gemm3m<T, N>([&](int i, int k) { return Ts[k][wr + i]; },
+                      [&](int k, int j) {
+                        const int jj = wc + j;
+                        V v = ldg<T>(inv + (k + kTile * jj));
+                        if (k > jj) v = czero<V>();
+                        return v;
+                      },
+                      lim / 4, q);
+  } else if constexpr (OP == kLeftL) {
+    // A(i,k) = L^-1(wr+i, k), unit lower; B(k,j) = (P C')(k, wc+j)
+    wave_gemm3m<T, N>([&](int i, int k) {
+                        const int ii = wr + i;
+                        V v = ldg<T>(inv + (ii + kTile * k));
+                        if (ii <= k) {
+                          v.x = ii == k ? T(1) : T(0);
+                          v.y = T(0);
+                        }
+                        return v;
+                      },
+                      [&](int k, int j) { return Ts[wc + j][k]; }, lim / 4, q);
+  } else {
+    // A(i,k) = U^-1(wr+i, k), upper incl. diagonal; B(k,j) = C'(k, wc+j): k >= wr
+    wave_gemm3m<T, N>([&](int i, int k) {
+                        const int ii = wr + i;
+                        V v = ldg<T>(inv + (ii + kTile * (wr + k)));
+                        if (wr + k < ii) v = czero<V>();
+                        return v;
+                      },
+                      [&](int k, int j) { return Ts[wc + j][wr + k]; }, (kTile - wr) / 4, q);
+  }
+#pragma unroll
+  for (int bj = 0; bj < N; bj++)
+#pragma unroll
+    for (int bi = 0; bi < N; bi++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        Cw[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))] = plus_value<T, N>(q, bj, bi, r);
 }
 
 // Split-FP16 operands: eight halves of a 32-wide k chunk per lane, the

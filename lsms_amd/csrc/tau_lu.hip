@@ -12,12 +12,13 @@
 // Per step s (tile column c0 = 64 s), batched over all solves:
 //   k_lu_diag    factor A_ss = P^T L U in LDS (tile_lu.hpp); store L^-1, U^-1 and P
 //   k_lu_panel   L_is = A_is U^-1 (tiles below), U_sj = L^-1 P A_sj (right)
-//   k_lu_update  A_ij -= L_is U_sj                     <- MFMA, dominant
-// with the steps taken in groups (k_lu_cross, k_lu_trail: the trailing
-// matrix is read and written once per group; on the split-FP16 path
-// k_lu_panel_h takes the cross updates inside the panel and the trailing
-// update is k_lu_trail_h in update_f16.hip); then k_lu_last factors the last
-// tile with the pivots of its non-central
+// with the steps taken in groups: the diagonal tile (k_lu_cross_diag) and the
+// panel tiles (inside k_lu_panel) of a step first take the earlier steps of
+// its group, and one trailing update per group, A_ij -= sum_k L_ik U_kj
+// (k_lu_trail, MFMA, dominant), reads and writes the rest of the matrix once.
+// The split-FP16 path has its own k_lu_panel_h, and k_lu_trail_h and
+// k_lu_cross_diag_h in update_f16.hip.  k_lu_last then factors the last tile
+// with the pivots of its non-central
 // rows and of the central rows kept apart.  In FP64 it also solves
 // S tau00 = t0 with the Schur complement S (the plain path); in FP32 it
 // stores the last tile's factors for the refinement solves (mixed path).
@@ -169,8 +170,9 @@ __device__ __forceinline__ void store_tile(TileLds<T> &t, const SolveDesc &d, in
 template <class T>
 __global__ __launch_bounds__(256) void k_lu_diag(const SolveDesc *__restrict__ descs, int step) {
   const SolveDesc &d = descs[blockIdx.x];
-  step -= d.step0;
-  if (step < 0 || step > d.nt - 1 || (step == d.nt - 1 && !d.full_lu)) return;
+  const bool last = step == kLastStep;  // each solve's own last tile (full LU)
+  step = last ? d.nt - 1 : step - d.step0;
+  if (step < 0 || (!last && step >= d.nt - 1)) return;
   if (d.conv && *d.conv) return;
   __shared__ TileLds<T> t;
   tile_lu<T>(t, tile_ptr<T>(d, step, step), tile_ld(d), kTile, step * kTile);
@@ -321,15 +323,13 @@ __device__ __forceinline__ void cross_to_lds(const SolveDesc &d, int ti, int tj,
       }
 }
 
-// Panel of step s: x < nrest -> L_is = A_is U^-1 ; else U_sj = L^-1 P A_sj.
-// The operand tile is staged in LDS (rows gathered by the pivot permutation
-// for U_sj) before it is overwritten in place.  With CROSS (the split-FP16
-// path) the tile first takes the cross update with the ncross steps before s
-// in its group, on the way into LDS (cross_to_lds), so that no separate
-// cross kernel reads and writes it.
-template <class T, bool CROSS>
-__device__ __forceinline__ void panel_tile(const SolveDesc &d, int step, int ncross, int x) {
-  typedef CxT<T> V;
+// Panel of step s on the split-FP16 path: x < nrest -> L_is = A_is U^-1 ; else
+// U_sj = L^-1 P A_sj.  The operand tile is staged in LDS (rows gathered by the
+// pivot permutation for U_sj) before it is overwritten in place, and takes the
+// cross update with the ncross steps before s in its group on the way
+// (cross_to_lds).
+__device__ __forceinline__ void panel_tile_h(const SolveDesc &d, int step, int ncross, int x) {
+  typedef float2 V;
   const int nrest = d.nt - 1 - step;
   if (step < 0 || nrest <= 0 || x >= 2 * nrest) return;
   if (d.conv && *d.conv) return;
@@ -338,148 +338,103 @@ __device__ __forceinline__ void panel_tile(const SolveDesc &d, int step, int ncr
   const int lane = tid & 63, li = lane & 15, kq = lane >> 4;
   const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
   const long ld = tile_ld(d);
-  const GCx<T> *__restrict__ inv = (const GCx<T> *)d.inv + step * d.inv_stride;
   const bool lower = x < nrest;
   const int ti = lower ? step + 1 + x : step, tj = lower ? step : step + 1 + x - nrest;
-  GCx<T> *tile = tile_ptr<T>(d, ti, tj);
-  bool staged = false;
-  if constexpr (CROSS) {
-    if (ncross > 0) {
-      // the row of C that lands at LDS row r is perm[r] (U_sj): rowpos = perm^-1
-      __shared__ int rowpos[kTile];
-      if (!lower && tid < kTile) rowpos[d.perm[step * kTile + tid]] = tid;
-      cross_to_lds(d, ti, tj, step - ncross, ncross, tile, ld, Ts, lower ? nullptr : rowpos);
-      staged = true;
-    }
-  }
-  if (!staged) {
+  GCx<float> *tile = tile_ptr<float>(d, ti, tj);
+  if (ncross > 0) {
+    // the row of C that lands at LDS row r is perm[r] (U_sj): rowpos = perm^-1
+    __shared__ int rowpos[kTile];
+    if (!lower && tid < kTile) rowpos[d.perm[step * kTile + tid]] = tid;
+    cross_to_lds(d, ti, tj, step - ncross, ncross, tile, ld, Ts, lower ? nullptr : rowpos);
+  } else {
     if (lower) {
-      stage_tile<T>(Ts, tile, ld, [](int r) { return r; });
+      stage_tile<float>(Ts, tile, ld, [](int r) { return r; });
     } else {
       const int *perm = d.perm + step * kTile;
-      stage_tile<T>(Ts, tile, ld, [&](int r) { return perm[r]; });
+      stage_tile<float>(Ts, tile, ld, [&](int r) { return perm[r]; });
     }
   }
   __syncthreads();
   V ov[2][2][4];  // output (row wr + 16 bi + li, column wc + 16 bj + acc_row(kq, r))
-  if constexpr (CROSS) {
-    // split-FP16 product with the diagonal tile's inverse planes (written by
-    // k_lu_diag): the tile's side is split here with its own scale, the
-    // accumulators take -(A B) as in the cross update (b-operand rows with
-    // -Re, a-operand columns with +Re), two 32-wide k chunks
-    const int eC = plane_exponent([&](int a, int b) { return Ts[a][b]; });
-    const float sc = ldexpf(1.f, -eC);
-    const int g = kq, l16 = li;
-    GH8 *ip = (GH8 *)((const _Float16 *)d.ihp + (lower ? kPlaneHalves : 0));
-    const int eI = d.ihe[lower ? 1 : 0];
-    f4 cr[2][2], ci[2][2];
+  // split-FP16 product with the diagonal tile's inverse planes (written by
+  // k_lu_diag): the tile's side is split here with its own scale, the
+  // accumulators take -(A B) as in the cross update (b-operand rows with
+  // -Re, a-operand columns with +Re), two 32-wide k chunks
+  const int eC = plane_exponent([&](int a, int b) { return Ts[a][b]; });
+  const float sc = ldexpf(1.f, -eC);
+  const int g = kq, l16 = li;
+  GH8 *ip = (GH8 *)((const _Float16 *)d.ihp + (lower ? kPlaneHalves : 0));
+  const int eI = d.ihe[lower ? 1 : 0];
+  f4 cr[2][2], ci[2][2];
+#pragma unroll
+  for (int bi = 0; bi < 2; bi++)
+#pragma unroll
+    for (int bj = 0; bj < 2; bj++) {
+      cr[bi][bj] = f4{0.f, 0.f, 0.f, 0.f};
+      ci[bi][bj] = cr[bi][bj];
+    }
+#pragma unroll 1
+  for (int kh = 0; kh < 2; kh++) {
+    // b-operands (rows wr + 16 bi ..): L_is = C U^-1 takes the rows of C
+    // from Ts[k][i], U_sj = L^-1 (P C) the rows of L^-1 from its planes
+    h8 lo[2][4];
+#pragma unroll
+    for (int bi = 0; bi < 2; bi++) {
+      if (lower) {
+        float2 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = Ts[32 * kh + 8 * g + u][wr + 16 * bi + l16];
+        split8(v, -1.f, sc, lo[bi][0], lo[bi][1], lo[bi][2], lo[bi][3]);
+      } else {
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+          lo[bi][p] = ip[((p * kTile + wr + 16 * bi + l16) * kTile + 32 * kh + 8 * g) / 8];
+      }
+    }
+#pragma unroll
+    for (int bj = 0; bj < 2; bj++) {
+      // a-operand (columns wc + 16 bj ..): U^-1 from its planes, or P C from Ts[j][k]
+      h8 uo[4];
+      if (lower) {
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+          uo[p] = ip[((p * kTile + wc + 16 * bj + l16) * kTile + 32 * kh + 8 * g) / 8];
+      } else {
+        float2 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = Ts[wc + 16 * bj + l16][32 * kh + 8 * g + u];
+        split8(v, 1.f, sc, uo[0], uo[1], uo[2], uo[3]);
+      }
+      const h8 nur_h = neg8(uo[0]), nur_l = neg8(uo[1]);
+#pragma unroll
+      for (int bi = 0; bi < 2; bi++) {
+        f4 r = cr[bi][bj], m = ci[bi][bj];
+        r = mfma_h(uo[0], lo[bi][0], r);
+        r = mfma_h(uo[1], lo[bi][0], r);
+        r = mfma_h(uo[0], lo[bi][1], r);
+        r = mfma_h(uo[2], lo[bi][2], r);
+        r = mfma_h(uo[3], lo[bi][2], r);
+        r = mfma_h(uo[2], lo[bi][3], r);
+        m = mfma_h(uo[2], lo[bi][0], m);
+        m = mfma_h(uo[3], lo[bi][0], m);
+        m = mfma_h(uo[2], lo[bi][1], m);
+        m = mfma_h(nur_h, lo[bi][2], m);
+        m = mfma_h(nur_l, lo[bi][2], m);
+        m = mfma_h(nur_h, lo[bi][3], m);
+        cr[bi][bj] = r;
+        ci[bi][bj] = m;
+      }
+    }
+  }
+  const float so = -ldexpf(1.f, eC + eI);
+#pragma unroll
+  for (int bj = 0; bj < 2; bj++)
 #pragma unroll
     for (int bi = 0; bi < 2; bi++)
 #pragma unroll
-      for (int bj = 0; bj < 2; bj++) {
-        cr[bi][bj] = f4{0.f, 0.f, 0.f, 0.f};
-        ci[bi][bj] = cr[bi][bj];
-      }
-#pragma unroll 1
-    for (int kh = 0; kh < 2; kh++) {
-      // b-operands (rows wr + 16 bi ..): L_is = C U^-1 takes the rows of C
-      // from Ts[k][i], U_sj = L^-1 (P C) the rows of L^-1 from its planes
-      h8 lo[2][4];
-#pragma unroll
-      for (int bi = 0; bi < 2; bi++) {
-        if (lower) {
-          float2 v[8];
-#pragma unroll
-          for (int u = 0; u < 8; u++) v[u] = Ts[32 * kh + 8 * g + u][wr + 16 * bi + l16];
-          split8(v, -1.f, sc, lo[bi][0], lo[bi][1], lo[bi][2], lo[bi][3]);
-        } else {
-#pragma unroll
-          for (int p = 0; p < 4; p++)
-            lo[bi][p] = ip[((p * kTile + wr + 16 * bi + l16) * kTile + 32 * kh + 8 * g) / 8];
-        }
-      }
-#pragma unroll
-      for (int bj = 0; bj < 2; bj++) {
-        // a-operand (columns wc + 16 bj ..): U^-1 from its planes, or P C from Ts[j][k]
-        h8 uo[4];
-        if (lower) {
-#pragma unroll
-          for (int p = 0; p < 4; p++)
-            uo[p] = ip[((p * kTile + wc + 16 * bj + l16) * kTile + 32 * kh + 8 * g) / 8];
-        } else {
-          float2 v[8];
-#pragma unroll
-          for (int u = 0; u < 8; u++) v[u] = Ts[wc + 16 * bj + l16][32 * kh + 8 * g + u];
-          split8(v, 1.f, sc, uo[0], uo[1], uo[2], uo[3]);
-        }
-        const h8 nur_h = neg8(uo[0]), nur_l = neg8(uo[1]);
-#pragma unroll
-        for (int bi = 0; bi < 2; bi++) {
-          f4 r = cr[bi][bj], m = ci[bi][bj];
-          r = mfma_h(uo[0], lo[bi][0], r);
-          r = mfma_h(uo[1], lo[bi][0], r);
-          r = mfma_h(uo[0], lo[bi][1], r);
-          r = mfma_h(uo[2], lo[bi][2], r);
-          r = mfma_h(uo[3], lo[bi][2], r);
-          r = mfma_h(uo[2], lo[bi][3], r);
-          m = mfma_h(uo[2], lo[bi][0], m);
-          m = mfma_h(uo[3], lo[bi][0], m);
-          m = mfma_h(uo[2], lo[bi][1], m);
-          m = mfma_h(nur_h, lo[bi][2], m);
-          m = mfma_h(nur_l, lo[bi][2], m);
-          m = mfma_h(nur_h, lo[bi][3], m);
-          cr[bi][bj] = r;
-          ci[bi][bj] = m;
-        }
-      }
-    }
-    const float so = -ldexpf(1.f, eC + eI);
-#pragma unroll
-    for (int bj = 0; bj < 2; bj++)
-#pragma unroll
-      for (int bi = 0; bi < 2; bi++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) ov[bj][bi][r] = make_float2(cr[bi][bj][r] * so, ci[bi][bj][r] * so);
-  } else {
-    Acc3<T> q;
-    zero_acc(q);
-    // operand k-steps in flight: three for FP64 (the inverse's L2 latency),
-    // one for FP32, where more registers would cost a wave per SIMD
-    constexpr int kPanelPF = sizeof(T) == 8 ? 3 : 1;
-    if (lower) {
-      // A(i,k) = Ts(wr+i, k); B(k,j) = U^-1(k, wc+j), upper incl. diagonal
-      wave_gemm3m<T, kPanelPF>([&](int i, int k) { return Ts[k][wr + i]; },
-                                      [&](int k, int j) {
-                                        int jj = wc + j;
-                                        V v = czero<V>();
-                                        if (k <= jj) v = inv[k + kTile * jj];
-                                        return v;
-                                      },
-                                      q);
-    } else {
-      // A(i,k) = L^-1(wr+i, k), unit lower; B(k,j) = (P A_sj)(k, wc+j)
-      wave_gemm3m<T, kPanelPF>([&](int i, int k) {
-                                        int ii = wr + i;
-                                        V v = czero<V>();
-                                        if (ii == k) v.x = T(1);
-                                        if (ii > k) v = inv[ii + kTile * k];
-                                        return v;
-                                      },
-                                      [&](int k, int j) { return Ts[wc + j][k]; }, q);
-    }
-#pragma unroll
-    for (int bj = 0; bj < 2; bj++)
-#pragma unroll
-      for (int bi = 0; bi < 2; bi++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          ov[bj][bi][r].x = q.p[0][bj][bi][r] - q.p[1][bj][bi][r];
-          ov[bj][bi][r].y = q.p[2][bj][bi][r] - q.p[0][bj][bi][r] - q.p[1][bj][bi][r];
-        }
-  }
-  GCx<T> *C = tile + wr + ld * wc;
-  const bool planes = sizeof(T) == 4 && d.hp != nullptr;
-  if (planes) __syncthreads();  // every wave is done reading Ts
+      for (int r = 0; r < 4; r++) ov[bj][bi][r] = make_float2(cr[bi][bj][r] * so, ci[bi][bj][r] * so);
+  GCx<float> *C = tile + wr + ld * wc;
+  __syncthreads();  // every wave is done reading Ts
 #pragma unroll
   for (int bj = 0; bj < 2; bj++)
 #pragma unroll
@@ -487,32 +442,51 @@ __device__ __forceinline__ void panel_tile(const SolveDesc &d, int step, int ncr
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const V o = ov[bj][bi][r];
-        if constexpr (CROSS) {
-          // the split path's FP32 factor tile is read again only by the
-          // refinement sweeps after the whole factorization: non-temporal
-          typedef float pv2 __attribute__((ext_vector_type(2)));
-          __builtin_nontemporal_store(pv2{o.x, o.y},
-                                      (pv2 *)&C[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))]);
-        } else {
-          C[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))] = o;
-        }
-        if (planes) Ts[wc + 16 * bj + acc_row<T>(kq, r)][wr + 16 * bi + li] = o;
+        // the FP32 factor tile is read again only by the refinement sweeps
+        // after the whole factorization: non-temporal
+        typedef float pv2 __attribute__((ext_vector_type(2)));
+        __builtin_nontemporal_store(pv2{o.x, o.y},
+                                    (pv2 *)&C[(16 * bi + li) + ld * (16 * bj + acc_row<float>(kq, r))]);
+        Ts[wc + 16 * bj + acc_row<float>(kq, r)][wr + 16 * bi + li] = o;
       }
-  if constexpr (sizeof(T) == 4) {
-    if (planes) {
-      // split-FP16 planes of this panel tile for the split updates
-      const int parity = step % d.group, side = lower ? 0 : 1;
-      const int t = lower ? ti : tj;
-      write_split_planes(Ts, lower, (_Float16 *)d.hp + (long)((parity * 2 + side) * d.nt + t) * kPlaneHalves,
-                         d.he + (parity * 2 + side) * d.nt + t);
-    }
-  }
+  // split-FP16 planes of this panel tile for the split updates
+  const int parity = step % d.group, side = lower ? 0 : 1;
+  const int t = lower ? ti : tj;
+  write_split_planes(Ts, lower, (_Float16 *)d.hp + (long)((parity * 2 + side) * d.nt + t) * kPlaneHalves,
+                     d.he + (parity * 2 + side) * d.nt + t);
 }
 
-template <class T>
-__global__ __launch_bounds__(256) void k_lu_panel(const SolveDesc *__restrict__ descs, int step) {
-  const SolveDesc &d = descs[blockIdx.y];
-  panel_tile<T, false>(d, step - d.step0, 0, blockIdx.x);
+// Panel of step `step` with its cross update (panel_op): L_is = C' U^-1 for the
+// tiles below the diagonal tile, U_sj = L^-1 P C' for those right of it, where
+// C' has taken the ncross steps before s in its group.  N = 1: four
+// workgroups a tile (lu_small_grid chooses).  Bound by the MFMAs of the group's
+// steps and by the load latencies of a tile's two products (64 solves N = 2160
+// in FP64: MFMAs busy 57% of 5.7 ms).
+template <class T, int N>
+__global__ __launch_bounds__(256) void k_lu_panel(const SolveDesc *__restrict__ descs, int step,
+                                                  int ncross, int xcd_swizzle) {
+  int bx = blockIdx.x, by = blockIdx.y;
+  if (xcd_swizzle) xcd_remap(bx, by);
+  const SolveDesc &d = descs[by];
+  step -= d.step0;
+  constexpr int np = N == 2 ? 1 : 4;
+  const int nrest = d.nt - 1 - step, x = bx / np, piece = bx % np;
+  if (step < 0 || nrest <= 0 || x >= 2 * nrest) return;
+  if (d.conv && *d.conv) return;
+  const long ld = tile_ld(d);
+  const GCx<T> *inv = (const GCx<T> *)d.inv + step * d.inv_stride;
+  const LSMSX_GLOBAL int *perm = (const LSMSX_GLOBAL int *)d.perm + step * kTile;
+  const bool lower = x < nrest;
+  const int ti = lower ? step + 1 + x : step, tj = lower ? step : step + 1 + x - nrest;
+  const int g = step - ncross;
+  const GCx<T> *A = tile_ptr<T>(d, ti, g), *B = tile_ptr<T>(d, g, tj);
+  const long sa = tile_ptr<T>(d, ti, g + 1) - A, sb = tile_ptr<T>(d, g + 1, tj) - B;
+  GCx<T> *C = tile_ptr<T>(d, ti, tj);
+  __shared__ PanelLds<T, N> lds;
+  if (lower)
+    panel_op<T, N, kRightU>(C, true, false, A, sa, B, sb, ld, ncross, inv, perm, piece, lds);
+  else
+    panel_op<T, N, kLeftL>(C, true, false, A, sa, B, sb, ld, ncross, inv, perm, piece, lds);
 }
 
 // Panel of step `step` on the split-FP16 path with its cross update fused:
@@ -526,105 +500,77 @@ __global__ __launch_bounds__(256) void k_lu_panel_h(const SolveDesc *__restrict_
   int bx = blockIdx.x, by = blockIdx.y;
   if (xcd_swizzle) xcd_remap(bx, by);
   const SolveDesc &d = descs[by];
-  panel_tile<float, true>(d, step - d.step0, ncross, bx);
+  panel_tile_h(d, step - d.step0, ncross, bx);
 }
 
 // C(ti, tj) -= sum_{u < ns} L(ti, s0+u) U(s0+u, tj): one 64x64 tile per
-// workgroup, a 32x32 quarter per wave.  -C enters the 3M sums at the start
-// (q1 = -Cre, q2 = 0, q3 = -(Cre + Cim)), so C' = (q2 - q1, q1 + q2 - q3): the
-// tile is read and written once however many rank-64 panels are applied, and
-// no operand is negated.
-template <class T>
-__device__ __forceinline__ void update_tile(const SolveDesc &d, int ti, int tj, int s0, int ns) {
+// workgroup, a 32x32 quarter per wave (N = 2), or one 32x32 quarter per
+// workgroup, a 16x16 block per wave (N = 1, `piece` = the quarter).
+template <class T, int N>
+__device__ __forceinline__ void update_tile(const SolveDesc &d, int ti, int tj, int s0, int ns,
+                                            int piece) {
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
+  const int wr = N == 2 ? 32 * (w & 1) : 32 * (piece & 1) + 16 * (w & 1);
+  const int wc = N == 2 ? 32 * (w >> 1) : 32 * (piece >> 1) + 16 * (w >> 1);
   const long ld = tile_ld(d);
   GCx<T> *__restrict__ C = tile_ptr<T>(d, ti, tj) + wr + ld * wc;
   typedef T cv2 __attribute__((ext_vector_type(2)));
-  Acc3<T> q;
+  Acc3<T, N> q;
 #pragma unroll
-  for (int bj = 0; bj < 2; bj++)
+  for (int bj = 0; bj < N; bj++)
 #pragma unroll
-    for (int bi = 0; bi < 2; bi++)
+    for (int bi = 0; bi < N; bi++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         // C is read and written once per group: non-temporal, so that the
         // panels the other tiles read stay in L2
         const cv2 c = __builtin_nontemporal_load(
             (const cv2 *)&C[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))]);
-        q.p[0][bj][bi][r] = -c.x;
-        q.p[1][bj][bi][r] = T(0);
-        q.p[2][bj][bi][r] = -c.x - c.y;
+        set_minus<T, N>(q, bj, bi, r, c.x, c.y);
       }
-  if constexpr (sizeof(T) == 8) {
-    // column-major: the panels of consecutive steps are consecutive in k
-    wave_gemm3m_k(tile_ptr<T>(d, ti, s0) + wr, tile_ptr<T>(d, s0, tj) + ld * wc, ld, 16 * ns, q);
-  } else {
-    for (int u = 0; u < ns; u++) {
-      const GCx<T> *__restrict__ A = tile_ptr<T>(d, ti, s0 + u) + wr;
-      const GCx<T> *__restrict__ B = tile_ptr<T>(d, s0 + u, tj) + ld * wc;
-      wave_gemm3m<T>([&](int i, int k) { return A[i + ld * k]; },
-                            [&](int k, int j) { return B[k + ld * j]; }, q);
-    }
-  }
+  const GCx<T> *A = tile_ptr<T>(d, ti, s0), *B = tile_ptr<T>(d, s0, tj);
+  const long sa = tile_ptr<T>(d, ti, s0 + 1) - A, sb = tile_ptr<T>(d, s0 + 1, tj) - B;
+  tile_products<T, N>(A + wr, sa, B + ld * wc, sb, ld, ns, q);
 #pragma unroll
-  for (int bj = 0; bj < 2; bj++)
+  for (int bj = 0; bj < N; bj++)
 #pragma unroll
-    for (int bi = 0; bi < 2; bi++)
+    for (int bi = 0; bi < N; bi++)
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-        __builtin_nontemporal_store(
-            cv2{q.p[1][bj][bi][r] - q.p[0][bj][bi][r],
-                q.p[0][bj][bi][r] + q.p[1][bj][bi][r] - q.p[2][bj][bi][r]},
-            (cv2 *)&C[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))]);
-}
-
-// Trailing update of step s: A_ij -= L_is U_sj for all i, j > s.
-template <class T>
-__global__ __launch_bounds__(256) void k_lu_update(const SolveDesc *__restrict__ descs, int step,
-                                                   int xcd_swizzle) {
-  int bx = blockIdx.x, by = blockIdx.y;
-  if (xcd_swizzle) xcd_remap(bx, by);
-  const SolveDesc &d = descs[by];
-  step -= d.step0;
-  const int nrest = d.nt - 1 - step;
-  const int x = bx;
-  if (step < 0 || nrest <= 0 || x >= nrest * nrest) return;
-  if (d.conv && *d.conv) return;
-  update_tile<T>(d, step + 1 + x % nrest, step + 1 + x / nrest, step, 1);
+      for (int r = 0; r < 4; r++) {
+        const CxT<T> v = minus_value<T, N>(q, bj, bi, r);
+        __builtin_nontemporal_store(cv2{v.x, v.y},
+                                    (cv2 *)&C[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))]);
+      }
 }
 
 // Grouped elimination: the steps g .. g+ns-1 of a group (ns = min(group,
-// nt-1-g); step nt-1 is k_lu_last) are factored one after another, each
-// after a cross update that brings its tile column (rows >= t) and tile row
-// (columns > t) up to date with the group's earlier steps; then one trailing
-// update applies all ns steps to the tiles beyond the group.
+// nt-1-g); step nt-1 is k_lu_last) are factored one after another, the
+// diagonal tile and the panel of each first taking the group's earlier steps;
+// then one trailing update applies all ns steps to the tiles beyond the group.
 // Number of steps of the group starting at solve step g.
 __device__ __forceinline__ int group_steps(const SolveDesc &d, int g) {
   return min(d.group, d.nt - 1 - g);
 }
 
-// Cross update for step t = g + u of the group starting at global step s:
-// tile column t (rows >= t) and tile row t (columns > t) -= the products of
-// steps g .. t-1.
+// Cross update of the diagonal tile of step t = g + u of the group starting at
+// global step s with the steps g .. t-1, a quarter of the tile per workgroup
+// (the panel tiles take theirs in k_lu_panel).
 template <class T>
-__global__ __launch_bounds__(256) void k_lu_cross(const SolveDesc *__restrict__ descs, int step,
-                                                  int u) {
+__global__ __launch_bounds__(256) void k_lu_cross_diag(const SolveDesc *__restrict__ descs,
+                                                       int step, int u) {
   const SolveDesc &d = descs[blockIdx.y];
   const int g = step - d.step0, t = g + u;
   if (g < 0 || u >= group_steps(d, g)) return;
   if (d.conv && *d.conv) return;
-  const int n1 = d.nt - t, x = blockIdx.x;
-  if (x >= 2 * n1 - 1) return;
-  if (x < n1) update_tile<T>(d, t + x, t, g, u);
-  else update_tile<T>(d, t, t + 1 + (x - n1), g, u);
+  update_tile<T, 1>(d, t, t, g, u, blockIdx.x);
 }
 
 // Trailing update of the group starting at global step s: A_ij -= sum over
 // the group's steps k of L_ik U_kj for all i, j beyond the group, one pass
-// over C with K = 64 ns.
-template <class T>
+// over C with K = 64 ns.  64 solves N = 2160 in FP64: 19.2 ms with the MFMAs
+// busy 85% (22.4 ms and 75% with groups of two steps).
+template <class T, int N>
 __global__ __launch_bounds__(256) void k_lu_trail(const SolveDesc *__restrict__ descs, int step,
                                                   int xcd_swizzle) {
   int bx = blockIdx.x, by = blockIdx.y;
@@ -635,9 +581,10 @@ __global__ __launch_bounds__(256) void k_lu_trail(const SolveDesc *__restrict__ 
   const int ns = group_steps(d, g);
   if (ns <= 0) return;
   if (d.conv && *d.conv) return;
-  const int last = g + ns - 1, nrest = d.nt - 1 - last, x = bx;
+  constexpr int np = N == 2 ? 1 : 4;
+  const int last = g + ns - 1, nrest = d.nt - 1 - last, x = bx / np;
   if (x >= nrest * nrest) return;
-  update_tile<T>(d, last + 1 + x % nrest, last + 1 + x / nrest, g, ns);
+  update_tile<T, N>(d, last + 1 + x % nrest, last + 1 + x / nrest, g, ns, bx % np);
 }
 
 // Last tile (step nt-1): factor it with the non-central rows (first nd =
@@ -714,14 +661,16 @@ __global__ __launch_bounds__(256) void k_lu_last(const SolveDesc *__restrict__ d
 
 template __global__ void k_lu_diag<double>(const SolveDesc *, int);
 template __global__ void k_lu_diag<float>(const SolveDesc *, int);
-template __global__ void k_lu_panel<double>(const SolveDesc *, int);
-template __global__ void k_lu_panel<float>(const SolveDesc *, int);
-template __global__ void k_lu_update<double>(const SolveDesc *, int, int);
-template __global__ void k_lu_update<float>(const SolveDesc *, int, int);
-template __global__ void k_lu_cross<double>(const SolveDesc *, int, int);
-template __global__ void k_lu_cross<float>(const SolveDesc *, int, int);
-template __global__ void k_lu_trail<double>(const SolveDesc *, int, int);
-template __global__ void k_lu_trail<float>(const SolveDesc *, int, int);
+template __global__ void k_lu_panel<double, 2>(const SolveDesc *, int, int, int);
+template __global__ void k_lu_panel<double, 1>(const SolveDesc *, int, int, int);
+template __global__ void k_lu_panel<float, 2>(const SolveDesc *, int, int, int);
+template __global__ void k_lu_panel<float, 1>(const SolveDesc *, int, int, int);
+template __global__ void k_lu_cross_diag<double>(const SolveDesc *, int, int);
+template __global__ void k_lu_cross_diag<float>(const SolveDesc *, int, int);
+template __global__ void k_lu_trail<double, 2>(const SolveDesc *, int, int);
+template __global__ void k_lu_trail<double, 1>(const SolveDesc *, int, int);
+template __global__ void k_lu_trail<float, 2>(const SolveDesc *, int, int);
+template __global__ void k_lu_trail<float, 1>(const SolveDesc *, int, int);
 template __global__ void k_lu_last<double>(const SolveDesc *);
 template __global__ void k_lu_last<float>(const SolveDesc *);
 
