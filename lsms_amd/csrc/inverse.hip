@@ -13,10 +13,16 @@
 // diagonal-tile inverse kept): M = Lt Ut, Lt block lower with diagonal tiles P_s^T L_ss, Ut block
 // upper with diagonal tiles U_ss; Lt_ts (t > s) and Ut_ts (t < s) sit in M.
 // M^-1 = Ut^-1 Lt^-1 is formed in place in one Ns x Ns buffer Y:
-//   forward,  s = 0..nt-1:  Y_ss = L_ss^-1 P_s,  Y_sc = L_ss^-1 P_s Y_sc (c < s)
-//                           Y_tc -= Lt_ts Y_sc   (t > s, c <= s; Lt^-1 is block lower)
-//   backward, s = nt-1..0:  Y_sc = U_ss^-1 Y_sc  (all c)
-//                           Y_tc -= Ut_ts Y_sc   (t < s, all c)
+//   forward,  s = 0..nt-1:  Y_ss = L_ss^-1 P_s,
+//                           Y_sc = -L_ss^-1 P_s sum_{c <= u < s} Lt_su Y_uc  (c < s)
+//   backward, s = nt-1..0:  Y_sc = U_ss^-1 (Y_sc - sum_{u > s} Ut_su Y_uc)   (all c)
+// Both are left-looking, one launch per step and half, each tile of row s by
+// one workgroup (or four): every tile of Y is written once in each half, and
+// its sum and the product with the diagonal inverse are one pass (panel_op).
+// With a panel and an update launch per step, which read and wrote the tiles
+// of Y once for every u, eight solves of N = 944 took 1.33 ms, so 1.07 (MFMAs
+// busy 40%: the quarter tiles of such a small batch keep the L1 caches busy
+// with operands).
 // Work: Ns^3/6 (forward) + Ns^3/2 (backward) complex MACs on FP64 MFMA, 3M form.
 #include "lu_common.hpp"
 
@@ -25,156 +31,43 @@ namespace lsmsx {
 typedef CxT<double> Z;
 typedef GCx<double> GZ;
 
-// Store a wave's 32x32 3M accumulator block (rows wr.., cols wc.. of C).
-__device__ __forceinline__ void store_acc(GZ *C, long ld, const Acc3<double> &q) {
-  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
-#pragma unroll
-  for (int bj = 0; bj < 2; bj++)
-#pragma unroll
-    for (int bi = 0; bi < 2; bi++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        Z o;
-        o.x = q.p[0][bj][bi][r] - q.p[1][bj][bi][r];
-        o.y = q.p[2][bj][bi][r] - q.p[0][bj][bi][r] - q.p[1][bj][bi][r];
-        C[(16 * bi + li) + ld * (16 * bj + acc_row<double>(kq, r))] = o;
-      }
-}
-
-// C -= A B for one 64x64 tile, -C entering the 3M sums (as update_tile of the LU).
-__device__ __forceinline__ void tile_update(const GZ *__restrict__ A, const GZ *__restrict__ B,
-                                            GZ *__restrict__ C, long ld) {
-  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
-  C += wr + ld * wc;
-  Acc3<double> q;
-#pragma unroll
-  for (int bj = 0; bj < 2; bj++)
-#pragma unroll
-    for (int bi = 0; bi < 2; bi++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        Z c = C[(16 * bi + li) + ld * (16 * bj + acc_row<double>(kq, r))];
-        q.p[0][bj][bi][r] = -c.x;
-        q.p[1][bj][bi][r] = 0.0;
-        q.p[2][bj][bi][r] = -c.x - c.y;
-      }
-  wave_gemm3m_k<2>(A + wr, B + ld * wc, ld, kTile / 4, q);
-#pragma unroll
-  for (int bj = 0; bj < 2; bj++)
-#pragma unroll
-    for (int bi = 0; bi < 2; bi++)
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        C[(16 * bi + li) + ld * (16 * bj + acc_row<double>(kq, r))] =
-            Z{q.p[1][bj][bi][r] - q.p[0][bj][bi][r],
-              q.p[0][bj][bi][r] + q.p[1][bj][bi][r] - q.p[2][bj][bi][r]};
-}
-
-// Fill Y with zeros: one 64-column strip per workgroup.
-__global__ __launch_bounds__(256) void k_inv_zero(const SolveDesc *__restrict__ descs) {
+// Forward step s: Y_sc for the column tiles c = 0 .. s.
+template <int N>
+__global__ __launch_bounds__(256) void k_inv_fwd(const SolveDesc *__restrict__ descs, int step) {
   const SolveDesc &d = descs[blockIdx.y];
-  const int strip = blockIdx.x;
-  if (strip >= d.nt) return;
-  GZ *Y = (GZ *)d.Minv + d.ld * (long)(strip * kTile);
-  const long n = (long)kTile * d.ld;
-  for (long e = threadIdx.x; e < n; e += 256) Y[e] = Z{0.0, 0.0};
-}
-
-// Forward step s, diagonal part: Y_sc = L_ss^-1 P_s Y_sc for c < s and
-// Y_ss = L_ss^-1 P_s (column tile c = blockIdx.x <= s).
-__global__ __launch_bounds__(256) void k_inv_fwd_panel(const SolveDesc *__restrict__ descs,
-                                                       int step) {
-  const SolveDesc &d = descs[blockIdx.y];
-  const int c = blockIdx.x;
+  constexpr int np = N == 2 ? 1 : 4;
+  const int c = blockIdx.x / np, piece = blockIdx.x % np;
   if (step >= d.nt || c > step) return;
-  __shared__ Z Ts[kTile][kTile + 1];  // Ts[col][row]
-  const int tid = threadIdx.x, w = tid >> 6;
-  const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
+  __shared__ PanelLds<double, N> lds;
   const long ld = d.ld;
-  GZ *tile = (GZ *)d.Minv + (long)(step * kTile) + ld * (c * kTile);
-  const int *perm = d.perm + step * kTile;
-  const GZ *__restrict__ inv = (const GZ *)d.inv + step * d.inv_stride;
-  for (int e = tid; e < kTile * kTile; e += 256) {
-    int r = e & 63, col = e >> 6;
-    Z v;
-    if (c == step) v = Z{perm[r] == col ? 1.0 : 0.0, 0.0};
-    else v = tile[perm[r] + ld * col];
-    Ts[col][r] = v;
-  }
-  __syncthreads();
-  Acc3<double> q;
-  zero_acc(q);
-  // A(i,k) = L^-1(wr+i, k), unit lower; B(k,j) = (P Y_sc)(k, wc+j)
-  wave_gemm3m<double, 2>([&](int i, int k) {
-                               int ii = wr + i;
-                               Z v = Z{ii == k ? 1.0 : 0.0, 0.0};
-                               if (ii > k) v = inv[ii + kTile * k];
-                               return v;
-                             },
-                             [&](int k, int j) { return Ts[wc + j][k]; }, kTile / 4, q);
-  store_acc(tile + wr + ld * wc, ld, q);
+  GZ *M = (GZ *)d.M, *Y = (GZ *)d.Minv;
+  panel_op<double, N, kLeftL>(Y + kTile * (step + ld * c), false, c == step,
+                              M + kTile * (step + ld * c), 0, Y + kTile * (c + ld * c), 0, ld,
+                              step - c, (const GZ *)d.inv + step * d.inv_stride,
+                              (const LSMSX_GLOBAL int *)d.perm + step * kTile, piece, lds);
 }
 
-// Forward step s, update: Y_tc -= Lt_ts Y_sc for t > s, c <= s.
-__global__ __launch_bounds__(256) void k_inv_fwd_update(const SolveDesc *__restrict__ descs,
-                                                        int step) {
+// Backward step s: Y_sc for every column tile c; the forward half left rows
+// s >= c, the others are zero.
+template <int N>
+__global__ __launch_bounds__(256) void k_inv_bwd(const SolveDesc *__restrict__ descs, int step) {
   const SolveDesc &d = descs[blockIdx.y];
-  const int nrest = d.nt - 1 - step;
-  const int x = blockIdx.x;
-  if (nrest <= 0 || x >= nrest * (step + 1)) return;
-  const int t = step + 1 + x % nrest, c = x / nrest;
-  const long ld = d.ld;
-  const GZ *M = (const GZ *)d.M;
-  GZ *Y = (GZ *)d.Minv;
-  tile_update(M + (long)(kTile * t) + ld * (kTile * step), Y + (long)(kTile * step) + ld * (kTile * c),
-              Y + (long)(kTile * t) + ld * (kTile * c), ld);
-}
-
-// Backward step s, diagonal part: Y_sc = U_ss^-1 Y_sc for every column tile c.
-__global__ __launch_bounds__(256) void k_inv_bwd_panel(const SolveDesc *__restrict__ descs,
-                                                       int step) {
-  const SolveDesc &d = descs[blockIdx.y];
-  const int c = blockIdx.x;
+  constexpr int np = N == 2 ? 1 : 4;
+  const int c = blockIdx.x / np, piece = blockIdx.x % np;
   if (step >= d.nt || c >= d.nt) return;
-  __shared__ Z Ts[kTile][kTile + 1];
-  const int tid = threadIdx.x, w = tid >> 6;
-  const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
+  __shared__ PanelLds<double, N> lds;
   const long ld = d.ld;
-  GZ *tile = (GZ *)d.Minv + (long)(step * kTile) + ld * (c * kTile);
-  const GZ *__restrict__ inv = (const GZ *)d.inv + step * d.inv_stride;
-  for (int e = tid; e < kTile * kTile; e += 256) {
-    int r = e & 63, col = e >> 6;
-    Ts[col][r] = tile[r + ld * col];
-  }
-  __syncthreads();
-  Acc3<double> q;
-  zero_acc(q);
-  // A(i,k) = U^-1(wr+i, k), upper incl. diagonal; B(k,j) = Y_sc(k, wc+j)
-  wave_gemm3m<double, 2>([&](int i, int k) {
-                               int ii = wr + i;
-                               Z v = Z{0.0, 0.0};
-                               if (k >= ii) v = inv[ii + kTile * k];
-                               return v;
-                             },
-                             [&](int k, int j) { return Ts[wc + j][k]; }, kTile / 4, q);
-  store_acc(tile + wr + ld * wc, ld, q);
+  const int s1 = min(step + 1, d.nt - 1);
+  GZ *M = (GZ *)d.M, *Y = (GZ *)d.Minv;
+  panel_op<double, N, kLeftU>(Y + kTile * (step + ld * c), step >= c, false,
+                              M + kTile * (step + ld * s1), 0, Y + kTile * (s1 + ld * c), 0, ld,
+                              d.nt - 1 - step, (const GZ *)d.inv + step * d.inv_stride, nullptr,
+                              piece, lds);
 }
-
-// Backward step s, update: Y_tc -= Ut_ts Y_sc for t < s, all c.
-__global__ __launch_bounds__(256) void k_inv_bwd_update(const SolveDesc *__restrict__ descs,
-                                                        int step) {
-  const SolveDesc &d = descs[blockIdx.y];
-  const int x = blockIdx.x;
-  if (step >= d.nt || step == 0 || x >= step * d.nt) return;
-  const int t = x % step, c = x / step;
-  const long ld = d.ld;
-  const GZ *M = (const GZ *)d.M;
-  GZ *Y = (GZ *)d.Minv;
-  tile_update(M + (long)(kTile * t) + ld * (kTile * step), Y + (long)(kTile * step) + ld * (kTile * c),
-              Y + (long)(kTile * t) + ld * (kTile * c), ld);
-}
+template __global__ void k_inv_fwd<1>(const SolveDesc *, int);
+template __global__ void k_inv_fwd<2>(const SolveDesc *, int);
+template __global__ void k_inv_bwd<1>(const SolveDesc *, int);
+template __global__ void k_inv_bwd<2>(const SolveDesc *, int);
 
 // X = M^-1 [0; t0] = Y[:, central] t0 (one 64-row tile per workgroup) and
 // tau00 = X_c, the central rows.

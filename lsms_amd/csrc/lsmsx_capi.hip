@@ -81,11 +81,10 @@ __global__ void k_ir_extract(const SolveDesc *);
 __global__ void k_count_conv(const SolveDesc *, int, int *);
 __global__ void k_lloyd(const SolveDesc *, const double2 *, const double2 *, long, const double *,
                         const double2 *, int);
-__global__ void k_inv_zero(const SolveDesc *);
-__global__ void k_inv_fwd_panel(const SolveDesc *, int);
-__global__ void k_inv_fwd_update(const SolveDesc *, int);
-__global__ void k_inv_bwd_panel(const SolveDesc *, int);
-__global__ void k_inv_bwd_update(const SolveDesc *, int);
+template <int N>
+__global__ void k_inv_fwd(const SolveDesc *, int);
+template <int N>
+__global__ void k_inv_bwd(const SolveDesc *, int);
 __global__ void k_inv_x(const SolveDesc *);
 __global__ void k_tau_full_out(const SolveDesc *, const double2 *, long, const int *, const int *,
                                double2 *, long);
@@ -1214,18 +1213,17 @@ int launch_inverse(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max) {
   }
   if (int r = check_launch("full LU")) return r;
   ProfScope p(c, 7);
-  hipLaunchKernelGGL(k_inv_zero, dim3(nt_max, nb), dim3(256), 0, c->stream, dd);
   for (int s = 0; s < nt_max; s++) {
-    hipLaunchKernelGGL(k_inv_fwd_panel, dim3(s + 1, nb), dim3(256), 0, c->stream, dd, s);
-    int nrest = nt_max - 1 - s;
-    if (nrest > 0)
-      hipLaunchKernelGGL(k_inv_fwd_update, dim3(nrest * (s + 1), nb), dim3(256), 0, c->stream, dd,
-                         s);
+    if (lu_small_grid((long)(s + 1) * nb))
+      hipLaunchKernelGGL(k_inv_fwd<1>, dim3(4 * (s + 1), nb), dim3(256), 0, c->stream, dd, s);
+    else
+      hipLaunchKernelGGL(k_inv_fwd<2>, dim3(s + 1, nb), dim3(256), 0, c->stream, dd, s);
   }
   for (int s = nt_max - 1; s >= 0; s--) {
-    hipLaunchKernelGGL(k_inv_bwd_panel, dim3(nt_max, nb), dim3(256), 0, c->stream, dd, s);
-    if (s > 0)
-      hipLaunchKernelGGL(k_inv_bwd_update, dim3(s * nt_max, nb), dim3(256), 0, c->stream, dd, s);
+    if (lu_small_grid((long)nt_max * nb))
+      hipLaunchKernelGGL(k_inv_bwd<1>, dim3(4 * nt_max, nb), dim3(256), 0, c->stream, dd, s);
+    else
+      hipLaunchKernelGGL(k_inv_bwd<2>, dim3(nt_max, nb), dim3(256), 0, c->stream, dd, s);
   }
   return check_launch("explicit inverse");
 }
