@@ -62,6 +62,7 @@ __global__ void k_ir_residual_g(const SolveDesc *);
 __global__ void k_ir_residual_g_finish(const SolveDesc *);
 __global__ void k_copy_m(const SolveDesc *);
 __global__ void k_fitpot(const double *, const double *, const int *, int, int, double *);
+template <int NQ>
 __global__ void k_single_site(const double *, const double *, const SingleSitePot *,
                               const double2 *, const double2 *, int, int, int, int, int,
                               double2 *, double2 *, double2 *, int *);
@@ -2386,7 +2387,13 @@ int lsmsx_single_site_nonrel(lsmsx_ctx *c, int nrelv, int lmax, int npot, int ip
                      c->ss_v.p, c->ss_iend.p, iprpts, npot, c->ss_coef.p);
   HIPCHK(hipGetLastError());
   const size_t nthr = (want_j ? 2 : 1) * ntask;  // inward integrations in threads of their own
-  hipLaunchKernelGGL(k_single_site, dim3((unsigned)((nthr + 63) / 64)), dim3(64), 0, st,
+  // a quad of lanes per integration while those are one wave per SIMD at most
+  // and the time is one wave's chain (4096 integrations 3.74 -> 3.02 ms a
+  // call, 8192: 4.58 -> 3.91; at 32768 both take 13.0 ms, at 65536 one thread
+  // each is the faster, 23 against 38 ms)
+  const bool quad = nthr <= 16384;
+  const auto kernel = quad ? k_single_site<4> : k_single_site<1>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((nthr * (quad ? 4 : 1) + 63) / 64)), dim3(64), 0, st,
                      c->ss_r.p, c->ss_coef.p, c->ss_pot.p, c->ss_e.p, c->ss_prel.p, npot, ne,
                      lmax, iprpts, nrelv == 0 ? 1 : 0, c->ss_matom.p,
                      want_z ? c->ss_zlr.p : nullptr, want_j ? c->ss_jlr.p : nullptr,

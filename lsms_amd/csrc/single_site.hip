@@ -74,7 +74,7 @@ __device__ inline zd zexp_i(zd z) {  // e^{i z}
 }
 
 // Bulirsch-Stoer step-count sequence n_j = 2 n_{j-2} (bulirschStoerIntegrator.cpp:66-67)
-__constant__ int kSeq[12] = {2, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
+__device__ constexpr int kSeq[12] = {2, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
 constexpr int kBsSteps = 11;
 constexpr int kBsTarget = 7;
 constexpr double kBsEps = 1.0e-12;
@@ -97,100 +97,159 @@ struct RhsPar {
   double er, ei, b, allp1;
 };
 
-// derivatives of (Re g, Im g, Re f, Im f) (dfv_new.f, nv = 4, eunit = 1)
-__device__ inline void rhs4(double r, const double *y, double *dy, double rn, const double *pc,
-                            const RhsPar &p) {
-  const double s1or = fdiv(1.0, r), s1or2 = s1or * s1or;
+// derivatives of (Re g, Im g, Re f, Im f) (dfv_new.f, nv = 4, eunit = 1):
+// the coefficients at r, and the derivative from them
+struct RhsCoef {
+  double s1or, frelr, freli, facr, faci;
+};
+__device__ inline RhsCoef rhs_coef(double r, double rn, const double *pc, const RhsPar &p) {
+  RhsCoef c;
+  c.s1or = fdiv(1.0, r);
+  const double s1or2 = c.s1or * c.s1or;
   const double r1 = r - rn;
   const double v = fdiv(pc[0] * r1 + pc[1], 1.0 + pc[2] * r1 * r1) + pc[3];
-  const double s2vmer = v * s1or - p.er;
-  const double frelr = 1.0 - p.b * s2vmer;
+  const double s2vmer = v * c.s1or - p.er;
+  c.frelr = 1.0 - p.b * s2vmer;
   const double s2vmei = -p.ei;
-  const double freli = -p.b * s2vmei;
-  const double den = fdiv(p.allp1, frelr * frelr + freli * freli) * s1or2;
-  const double facr = den * frelr + s2vmer;
-  const double faci = -den * freli + s2vmei;
-  dy[0] = frelr * y[2] - freli * y[3] + s1or * y[0];
-  dy[1] = freli * y[2] + frelr * y[3] + s1or * y[1];
-  dy[2] = facr * y[0] - faci * y[1] - y[2] * s1or;
-  dy[3] = faci * y[0] + facr * y[1] - y[3] * s1or;
+  c.freli = -p.b * s2vmei;
+  const double den = fdiv(p.allp1, c.frelr * c.frelr + c.freli * c.freli) * s1or2;
+  c.facr = den * c.frelr + s2vmer;
+  c.faci = -den * c.freli + s2vmei;
+  return c;
+}
+__device__ inline void rhs_apply(const RhsCoef &c, const double *y, double *dy) {
+  dy[0] = c.frelr * y[2] - c.freli * y[3] + c.s1or * y[0];
+  dy[1] = c.freli * y[2] + c.frelr * y[3] + c.s1or * y[1];
+  dy[2] = c.facr * y[0] - c.faci * y[1] - y[2] * c.s1or;
+  dy[3] = c.faci * y[0] + c.facr * y[1] - y[3] * c.s1or;
+}
+__device__ inline void rhs4(double r, const double *y, double *dy, double rn, const double *pc,
+                            const RhsPar &p) {
+  rhs_apply(rhs_coef(r, rn, pc, p), y, dy);
 }
 
-// modified midpoint rule with `steps` substeps over [x0, x1]
+// modified midpoint rule with `steps` (even) substeps over [x0, x1].  The
+// coefficients depend on r alone and are most of a derivative's chain: those
+// of the next substep are formed beside this substep's update of y.  Two
+// substeps per turn, so that nothing is moved between registers.
 __device__ inline void midpoint4(double x0, double x1, const double *y0, double *y1, int steps,
                                  double rn, const double *pc, const RhsPar &p) {
   double y2[4], dy[4];
   const double h = fdiv(x1 - x0, (double)steps), h2 = 2.0 * h;
-  double x = x0;
-  rhs4(x, y0, dy, rn, pc, p);
+  double x = x0 + h;
+  RhsCoef ca = rhs_coef(x0, rn, pc, p), cb = rhs_coef(x, rn, pc, p);
+  rhs_apply(ca, y0, dy);
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     y1[i] = y0[i];
     y2[i] = y0[i] + h * dy[i];
   }
-  for (int j = 1; j < steps; j++) {
-    x += h;
-    rhs4(x, y2, dy, rn, pc, p);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const double t = y1[i] + h2 * dy[i];
-      y1[i] = y2[i];
-      y2[i] = t;
-    }
-  }
   x += h;
-  rhs4(x, y2, dy, rn, pc, p);
+  ca = rhs_coef(x, rn, pc, p);
+  rhs_apply(cb, y2, dy);
 #pragma unroll
-  for (int i = 0; i < 4; i++) y1[i] = 0.5 * (y1[i] + y2[i] + h * dy[i]);
+  for (int i = 0; i < 4; i++) y1[i] = y1[i] + h2 * dy[i];
+  for (int j = 2; j < steps; j += 2) {
+    x += h;
+    cb = rhs_coef(x, rn, pc, p);
+    rhs_apply(ca, y1, dy);
+#pragma unroll
+    for (int i = 0; i < 4; i++) y2[i] = y2[i] + h2 * dy[i];
+    x += h;
+    ca = rhs_coef(x, rn, pc, p);
+    rhs_apply(cb, y2, dy);
+#pragma unroll
+    for (int i = 0; i < 4; i++) y1[i] = y1[i] + h2 * dy[i];
+  }
+  rhs_apply(ca, y1, dy);
+#pragma unroll
+  for (int i = 0; i < 4; i++) y1[i] = 0.5 * (y2[i] + y1[i] + h * dy[i]);
+}
+
+// Value of lane Q0 of each quad of lanes, in all four of them.
+template <int Q0>
+__device__ inline double quad_value(double v) {
+  constexpr int perm = Q0 * 0x55;  // quad_perm [Q0, Q0, Q0, Q0]
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), perm, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), perm, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
 }
 
 // Adaptive Bulirsch-Stoer over [x0, x1] with polynomial extrapolation in h^2,
 // one tableau row kept in registers (T[i][k] needs only T[i][k-1] and
 // T[i-1][k-1]).  y is advanced in place; dy returns the derivative at x1.
 // Returns 1 if the step size underflowed (y then holds the last estimate).
+// NQ = 4: the four lanes of a quad take one task together.  The midpoint
+// values of four tableau rows (first those of 2, 4, 6 and 8 substeps) depend
+// on the start of the step alone, so each lane runs one row and all four then
+// extrapolate with all rows; the row that ends the step is the first that
+// passes the test, as when they are formed one by one.  A step that ends at
+// row 4 (94% of them on the radial meshes of the single-site problem) is a
+// chain of 9 derivatives, not of 24.
+template <int NQ>
 __device__ int bs_interval(double x0, double x1, double *y, double *dy, double rn,
-                           const double *pc, const RhsPar &p) {
+                           const double *pc, const RhsPar &p, int q) {
   const double xeps = 1.0e-12 * fabs(x0);
   double x = x0;
   const double h0 = x1 - x0;
   double h = h0;
   double row[kBsSteps][4] = {};
-  double hh[kBsSteps] = {};
-  int last = 0;  // diagonal index of the last tableau
+  double best[4];  // T[i][i] of the last row
   int rc = 0;
   do {
-    double err = HUGE_VAL;
+    bool more = true, ok = false;
     int step = 0;
 #pragma unroll
-    for (int i = 0; i < kBsSteps; i++) {
-      if (err > kBsEps) {
-        double y1[4];
-        midpoint4(x, x + h, y, y1, kSeq[i], rn, pc, p);
-        hh[i] = fdiv(h, (double)kSeq[i]);
-        double e = 0.0, mag = 0.0;
+    for (int ib = 0; ib < kBsSteps; ib += 4) {
+      if (more) {
+        double yb[4][4];  // the midpoint values of rows ib .. ib+3
+        if (NQ == 4) {
+          double y1[4];
+          const int n = q == 0 ? kSeq[ib] : q == 1 ? kSeq[ib + 1] : q == 2 ? kSeq[ib + 2] : kSeq[ib + 3];
+          midpoint4(x, x + h, y, y1, ib + q < kBsSteps ? n : kSeq[ib], rn, pc, p);
 #pragma unroll
-        for (int d = 0; d < 4; d++) {
-          double old = row[0][d];  // T[i-1][0]
-          row[0][d] = y1[d];
-#pragma unroll
-          for (int k = 1; k <= i; k++) {
-            const double rr = fdiv(hh[i - k], hh[i]);
-            const double den = fdiv(1.0, rr * rr - 1.0);
-            const double keep = row[k][d];  // T[i-1][k] (unused when k == i)
-            row[k][d] = row[k - 1][d] + (row[k - 1][d] - old) * den;
-            if (k == i) e += fabs(row[i][d] - old);  // old = T[i-1][i-1]
-            old = keep;
+          for (int d = 0; d < 4; d++) {
+            yb[0][d] = quad_value<0>(y1[d]);
+            yb[1][d] = quad_value<1>(y1[d]);
+            yb[2][d] = quad_value<2>(y1[d]);
+            yb[3][d] = quad_value<3>(y1[d]);
           }
-          mag += fabs(row[i][d]);
         }
-        if (i == 0) e = 4.0;
-        if (mag == 0.0) mag = 1.0e-15;
-        err = fdiv(e, mag);
-        step = i + 1;
-        last = i;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int i = ib + u;
+          if (i < kBsSteps && (NQ == 4 || more)) {
+            if (NQ == 1) midpoint4(x, x + h, y, yb[u], kSeq[i], rn, pc, p);
+            double e = 0.0, mag = 0.0;
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+              double old = row[0][d];  // T[i-1][0]
+              row[0][d] = yb[u][d];
+#pragma unroll
+              for (int k = 1; k <= i; k++) {
+                // 1 / ((h_{i-k} / h_i)^2 - 1), h_i = h / n_i
+                const double n1 = kSeq[i], n0 = kSeq[i - k];
+                const double den = n0 * n0 / (n1 * n1 - n0 * n0);
+                const double keep = row[k][d];  // T[i-1][k] (unused when k == i)
+                row[k][d] = row[k - 1][d] + (row[k - 1][d] - old) * den;
+                if (k == i) e += fabs(row[i][d] - old);  // old = T[i-1][i-1]
+                old = keep;
+              }
+              mag += fabs(row[i][d]);
+            }
+            if (i == 0) e = 4.0;
+            if (mag == 0.0) mag = 1.0e-15;
+            // selects, not branches: the rows' chains overlap
+            step = more ? i + 1 : step;
+            ok = more ? e < kBsEps * mag : ok;
+#pragma unroll
+            for (int d = 0; d < 4; d++) best[d] = more ? row[i][d] : best[d];
+            more = more && e > kBsEps * mag;
+          }
+        }
       }
     }
-    if (err < kBsEps) {
+    if (ok) {
       x = x + h;
       if (step < kBsTarget)
         h *= 1.25;
@@ -199,11 +258,7 @@ __device__ int bs_interval(double x0, double x1, double *y, double *dy, double r
       const double lim = fabs(x1 - x);
       h = copysign(fabs(h) < lim ? fabs(h) : lim, h0);
 #pragma unroll
-      for (int k = 0; k < kBsSteps; k++)
-        if (k == last) {
-#pragma unroll
-          for (int d = 0; d < 4; d++) y[d] = row[k][d];
-        }
+      for (int d = 0; d < 4; d++) y[d] = best[d];
     } else {
       h = 0.25 * h;
       if (h + x == x) {
@@ -213,11 +268,7 @@ __device__ int bs_interval(double x0, double x1, double *y, double *dy, double r
     }
   } while (fabs(x - x1) > xeps);
 #pragma unroll
-  for (int k = 0; k < kBsSteps; k++)
-    if (k == last) {
-#pragma unroll
-      for (int d = 0; d < 4; d++) y[d] = row[k][d];
-    }
+  for (int d = 0; d < 4; d++) y[d] = best[d];
   rhs4(x1, y, dy, rn, pc, p);
   return rc;
 }
@@ -460,9 +511,13 @@ __global__ void k_fitpot(const double *__restrict__ rmesh, const double *__restr
   c[3] = 0.0;
 }
 
-// One thread per (energy e, potential p, l): rwave.f with the outputs of
-// semrel_c.f (solver 2).  matom[(e*npot + p)*(lmax+1) + l];
+// One thread (NQ = 1) or one quad of lanes (NQ = 4) per (energy e, potential
+// p, l): rwave.f with the outputs of semrel_c.f (solver 2).  The time is one
+// thread's chain of dependent FP64 operations over the mesh as long as the
+// threads do not fill the chip: 16 potentials x 32 energies x 4 l are 64 waves
+// at one thread each, 2.41 ms, and 256 at four, 1.27.  matom[(e*npot + p)*(lmax+1) + l];
 // zlr/jlr (may be null) columns of iprpts at ((e*npot + p)*(lmax+1) + l)*iprpts.
+template <int NQ>
 __global__ void __launch_bounds__(64) k_single_site(
     const double *__restrict__ rmesh, const double *__restrict__ coef,
     const SingleSitePot *__restrict__ pots, const double2 *__restrict__ energy,
@@ -476,7 +531,8 @@ __global__ void __launch_bounds__(64) k_single_site(
   // solution.  k_jlr_scale divides their raw values by matom afterwards.
   const int nl = lmax + 1;
   const long ntask = (long)ne * npot * nl;
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  long t = ((long)blockIdx.x * blockDim.x + threadIdx.x) / NQ;
+  const int q = threadIdx.x % NQ;  // lane of the quad; it writes the points j % NQ == q
   if (t >= (jlr ? 2 : 1) * ntask) return;
   const bool inward = t >= ntask;
   if (inward) t -= ntask;
@@ -547,8 +603,8 @@ __global__ void __launch_bounds__(64) k_single_site(
     rhs4(P.r_sph, y, dy, P.r_sph, cf + 4 * (jmt - 1), rp);
     for (int j = jmt - 2; j >= 0; j--) {
       const double rfrom = (j + 1 == jmt - 1) ? P.r_sph : rad[j + 1];
-      rc |= bs_interval(rfrom, rad[j], y, dy, rad[j], cf + 4 * j, rp);
-      if (j < jws) jcol[j] = make_double2(y[0], y[1]);
+      rc |= bs_interval<NQ>(rfrom, rad[j], y, dy, rad[j], cf + 4 * j, rp, q);
+      if (j < jws && j % NQ == q) jcol[j] = make_double2(y[0], y[1]);
     }
     if (rc) atomicOr(status, 1);
     return;
@@ -565,11 +621,11 @@ __global__ void __launch_bounds__(64) k_single_site(
     if (j == wi) { wr[1] = g; wd[1] = d; }
     if (j == P.ip1) { wr[2] = g; wd[2] = d; }
     if (j == P.i2) { wr[3] = g; wd[3] = d; }
-    if (zcol && j < jws) zcol[j] = make_double2(y[0], y[1]);
+    if (zcol && j < jws && j % NQ == q) zcol[j] = make_double2(y[0], y[1]);
   };
   capture(0);
   for (int j = 1; j < jmt; j++) {
-    rc |= bs_interval(rad[j - 1], rad[j], y, dy, rad[j - 1], cf + 4 * (j - 1), rp);
+    rc |= bs_interval<NQ>(rad[j - 1], rad[j], y, dy, rad[j - 1], cf + 4 * (j - 1), rp, q);
     capture(j);
   }
 
@@ -586,13 +642,13 @@ __global__ void __launch_bounds__(64) k_single_site(
   const zd cnorm = (bj + cdum * bh1) / fi;
   const zd tatoml = r_sph * cdum;
   const zd matom = -(times_i(ka) / tatoml);
-  matom_out[t] = make_double2(matom.x, matom.y);
+  if (q == 0) matom_out[t] = make_double2(matom.x, matom.y);
   const zd iprel = times_i(mk(prel[e].x, prel[e].y));
 
   // zlr = (cnorm g) matom / r inside the sphere
   if (zcol) {
     const int jend = jmt - 1 < jws ? jmt - 1 : jws;
-    for (int j = 0; j < jend; j++) {
+    for (int j = q; j < jend; j += NQ) {
       const double2 g = zcol[j];
       const zd gn = cnorm * mk(g.x, g.y);
       const zd z = (gn * matom) / rad[j];
@@ -601,7 +657,7 @@ __global__ void __launch_bounds__(64) k_single_site(
   }
 
   // outside the sphere: Bessel and Hankel forms (rwave.f:225-240)
-  for (int j = jmt - 1; j < jws; j++) {
+  for (int j = jmt - 1 + (q - (jmt - 1) % NQ + NQ) % NQ; j < jws; j += NQ) {
     kar = ka * rad[j];
     b = bessel_pick(kar, l);
     outside(b, ka, kar, l, bj, dbj, bh1, dbh1);
@@ -617,6 +673,12 @@ __global__ void __launch_bounds__(64) k_single_site(
   }
   if (rc) atomicOr(status, 1);
 }
+template __global__ void k_single_site<1>(const double *, const double *, const SingleSitePot *,
+                                          const double2 *, const double2 *, int, int, int, int, int,
+                                          double2 *, double2 *, double2 *, int *);
+template __global__ void k_single_site<4>(const double *, const double *, const SingleSitePot *,
+                                          const double2 *, const double2 *, int, int, int, int, int,
+                                          double2 *, double2 *, double2 *, int *);
 
 // jlr = i prel g_irr / (r matom) (semrel_c.f:214-217) for the points the
 // inward threads of k_single_site left raw (j < min(jmt-1, jws)); one
