@@ -103,7 +103,8 @@ __global__ void k_rel_tstore(double2 *, long, long, int, const double *, const d
 __global__ void k_rel_tau(double2 *, int, const double *, const double2 *);
 __global__ void k_rel_blocks(double2 *, long, int, const double *);
 __global__ void k_lu_cross_diag_h(const SolveDesc *, int, int);
-__global__ void k_lu_panel_h(const SolveDesc *, int, int, int);
+__global__ void k_lu_panel_h(const SolveDesc *, int, int, int, int);
+__global__ void k_lu_strip_h(const SolveDesc *, int);
 
 // Copy a caller matrix (central block first, n x n) into the solver layout;
 // rowperm (or null) reorders the n - k non-central rows: solver row xr takes
@@ -492,6 +493,13 @@ int launch_lu_steps(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool 
   const int G = lu_group(c, split_f16);
   for (int s = 0; s < nt_max - 1; s += G) {
     const int b = std::min(s + G - 1, nt_max - 2);  // the group's last step, largest solve
+    const int nrest = nt_max - 1 - b;
+    // strips (k_lu_strip_h) where there are many to a compute unit: a strip is
+    // as long as its group's steps together, and so is the launch's end (248
+    // solves of N = 2160, 12896 to 4960 strips a group: 52.6 -> 51.5 ms; 96
+    // uneven ones of an alloy, up to 4224: 19.2 -> 19.4; 32 of N = 864, 384:
+    // 3.45 -> 3.5)
+    const bool strips = split_f16 && 2L * nrest * nb >= 4864;
     for (int t = s; t <= b; t++) {
       const int u = t - s, np = 2 * (nt_max - 1 - t);
       if (u > 0) {
@@ -508,16 +516,21 @@ int launch_lu_steps(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool 
       }
       {
         ProfScope p(c, 2);
-        if (split_f16)
-          hipLaunchKernelGGL(k_lu_panel_h, dim3(np, nb), dim3(256), 0, st, dd, t, u, swz);
-        else if (lu_small_grid((long)np * nb))
+        if (split_f16) {
+          if (!strips || t < b)
+            hipLaunchKernelGGL(k_lu_panel_h, dim3(strips ? 2 * (b - t) : np, nb), dim3(256), 0, st,
+                               dd, t, u, strips ? 0 : 1, swz);
+        } else if (lu_small_grid((long)np * nb))
           hipLaunchKernelGGL((k_lu_panel<T, 1>), dim3(4 * np, nb), dim3(256), 0, st, dd, t, u, swz);
         else
           hipLaunchKernelGGL((k_lu_panel<T, 2>), dim3(np, nb), dim3(256), 0, st, dd, t, u, swz);
       }
       if (int r = check_launch("k_lu_diag/k_lu_panel")) return r;
     }
-    const int nrest = nt_max - 1 - b;
+    if (strips) {
+      ProfScope p(c, 2);
+      hipLaunchKernelGGL(k_lu_strip_h, dim3(2 * nrest, nb), dim3(256), 0, st, dd, s);
+    }
     {
       ProfScope p(c, 3);
       if (split_f16)
@@ -750,7 +763,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
     if (plain) bytes[i] += kTile * kTile * 16;
     if (mixed) bytes[i] += Ns * Ns * 8 + nt * kTile * kTile * 8 + Ns * kc * 24;
     if (refined64) bytes[i] += Ns * Ns * 16 + nt * kTile * kTile * 16 + Ns * kc * 32;
-    if (split) bytes[i] += (2 * lu_group(c, true) * nt + 2) * ((long)kPlaneHalves * 2 + 4);
+    if (split) bytes[i] += 2 * lu_group(c, true) * (nt + 1) * ((long)kPlaneHalves * 2 + 4);
   }
   // the explicit-inverse route's buffers are not used here: give them back
   // before sizing the chunks by the free memory
@@ -780,7 +793,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
       mtot += Ns * Ns;
       xtot += Ns * kc;
       ivtot += refining ? (Ns / kTile) * kTile * kTile : kTile * kTile;
-      htot += 2 * lu_group(c, split) * (Ns / kTile) + 2;
+      htot += 2 * lu_group(c, split) * (Ns / kTile + 1);
       maxliz = std::max(maxliz, a.numLIZ);
       nt_max = std::max(nt_max, (int)(Ns / kTile));
       if (gmode) {
@@ -837,7 +850,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
         hoff += 2 * lu_group(c, split) * (Ns / kTile);
         d.ihp = c->hp.p + hoff * kPlaneHalves;
         d.ihe = c->he.p + hoff;
-        hoff += 2;
+        hoff += 2 * lu_group(c, split);
       }
       d.pos = a.d_pos;
       d.lmax = a.d_lmax;

@@ -84,8 +84,8 @@ struct SolveDesc {
   // the current diagonal tile's inverses as split planes for the fused panel:
   // L^-1 (unit lower, as an L tile) then U^-1 (upper, as a U tile), and
   // their two exponents; written by k_lu_diag<float> when set
-  void *ihp;              // 2 tiles x 4 planes x 64 x 64 halves
-  int *ihe;               // 2
+  void *ihp;              // (step % group) x 2 tiles x 4 planes x 64 x 64 halves
+  int *ihe;               // (step % group) x 2
   // explicit inverse (full tau, Lloyd term, adjoint of tau00)
   double2 *Minv;          // Ns x Ns (leading dim ld): M^-1 in the solver layout
   double dprel_re, dprel_im;  // d prel / dE

@@ -30,13 +30,22 @@
 
 namespace lsmsx {
 
+// threadIdx.x as a value the compiler does not carry over from elsewhere: a
+// kernel that loops over panel tiles would otherwise keep every address and
+// index of the loop body in registers across it (237 VGPRs, not 150).
+__device__ __forceinline__ int fresh_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // Stage a 64 x 64 tile (column stride ld) in LDS, S[col][row] =
 // src[rowmap(row) + ld col]: the 16 loads of a thread are all issued before
 // its first LDS write, so staging costs one memory round trip, not sixteen.
 template <class T, class RM>
 __device__ __forceinline__ void stage_tile(CxT<T> (*S)[kTile + 1], const GCx<T> *src, long ld,
                                            RM rowmap) {
-  const int tid = threadIdx.x, r = tid & 63, c0 = tid >> 6;
+  const int tid = fresh_tid(), r = tid & 63, c0 = tid >> 6;
   const int rr = rowmap(r);
   CxT<T> v[kTile / 4];
 #pragma unroll
@@ -51,7 +60,7 @@ __device__ __forceinline__ void stage_tile(CxT<T> (*S)[kTile + 1], const GCx<T> 
 template <class F>
 __device__ int plane_exponent(F get) {
   __shared__ float wmax[4];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const int tid = fresh_tid(), w = tid >> 6, lane = tid & 63;
   __syncthreads();  // the values were written by all four waves
   float m = 0.f;
   for (int e = tid; e < kTile * kTile; e += 256) {
@@ -93,7 +102,7 @@ __device__ __forceinline__ void split8(const float2 (&v)[8], float sgn, float sc
 // The L planes carry the sign of the update C -= L U.
 template <class F>
 __device__ void write_planes(F get, bool lower, _Float16 *out, int *eout) {
-  const int tid = threadIdx.x;
+  const int tid = fresh_tid();
   const int ex = plane_exponent(get);
   if (tid == 0) *eout = ex;
   const float sc = ldexpf(1.f, -ex);
@@ -144,8 +153,10 @@ __device__ __forceinline__ void store_tile(TileLds<T> &t, const SolveDesc &d, in
   }
   if constexpr (sizeof(T) == 4) {
     if (d.ihp) {
-      // L^-1 (unit lower, L layout) and U^-1 (U layout)
-      _Float16 *ip = (_Float16 *)d.ihp;
+      // L^-1 (unit lower, L layout) and U^-1 (U layout), in the step's slot
+      const int slot = step % d.group;
+      _Float16 *ip = (_Float16 *)d.ihp + slot * (2 * kPlaneHalves);
+      int *ie = d.ihe + 2 * slot;
       write_planes(
           [&](int i, int k) {
             V v = t.get(k, i);
@@ -153,9 +164,9 @@ __device__ __forceinline__ void store_tile(TileLds<T> &t, const SolveDesc &d, in
             v.y = i > k ? v.y : 0.f;
             return v;
           },
-          true, ip, d.ihe);
+          true, ip, ie);
       write_planes([&](int j, int k) { return upper_at<T>(t, k, j); }, false, ip + kPlaneHalves,
-                   d.ihe + 1);
+                   ie + 1);
     }
   }
 }
@@ -198,7 +209,7 @@ __device__ __forceinline__ void cross_to_lds(const SolveDesc &d, int ti, int tj,
                                              int ns, const GCx<float> *A, long ld,
                                              float2 (*Ts)[kTile + 1], const int *rowpos) {
   __shared__ int exs[16];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int tid = fresh_tid(), w = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
   const int nt = d.nt, gmask = d.group - 1;
   const _Float16 *hp = (const _Float16 *)d.hp;
@@ -323,23 +334,20 @@ __device__ __forceinline__ void cross_to_lds(const SolveDesc &d, int ti, int tj,
       }
 }
 
-// Panel of step s on the split-FP16 path: x < nrest -> L_is = A_is U^-1 ; else
-// U_sj = L^-1 P A_sj.  The operand tile is staged in LDS (rows gathered by the
-// pivot permutation for U_sj) before it is overwritten in place, and takes the
-// cross update with the ncross steps before s in its group on the way
-// (cross_to_lds).
-__device__ __forceinline__ void panel_tile_h(const SolveDesc &d, int step, int ncross, int x) {
+// Panel tile t of step s on the split-FP16 path: lower -> L_ts = A_ts U^-1 ;
+// else U_st = L^-1 P A_st.  The operand tile is staged in LDS (rows gathered
+// by the pivot permutation for U_st) before it is overwritten in place, and
+// takes the cross update with the ncross steps before s in its group on the
+// way (cross_to_lds).
+__device__ __forceinline__ void panel_tile_h(const SolveDesc &d, int step, int ncross, bool lower,
+                                             int t) {
   typedef float2 V;
-  const int nrest = d.nt - 1 - step;
-  if (step < 0 || nrest <= 0 || x >= 2 * nrest) return;
-  if (d.conv && *d.conv) return;
   __shared__ __align__(16) V Ts[kTile][kTile + 1];  // Ts[col][row]
-  const int tid = threadIdx.x, w = tid >> 6;
+  const int tid = fresh_tid(), w = tid >> 6;
   const int lane = tid & 63, li = lane & 15, kq = lane >> 4;
   const int wr = 32 * (w & 1), wc = 32 * (w >> 1);
   const long ld = tile_ld(d);
-  const bool lower = x < nrest;
-  const int ti = lower ? step + 1 + x : step, tj = lower ? step : step + 1 + x - nrest;
+  const int ti = lower ? t : step, tj = lower ? step : t;
   GCx<float> *tile = tile_ptr<float>(d, ti, tj);
   if (ncross > 0) {
     // the row of C that lands at LDS row r is perm[r] (U_sj): rowpos = perm^-1
@@ -363,8 +371,9 @@ __device__ __forceinline__ void panel_tile_h(const SolveDesc &d, int step, int n
   const int eC = plane_exponent([&](int a, int b) { return Ts[a][b]; });
   const float sc = ldexpf(1.f, -eC);
   const int g = kq, l16 = li;
-  GH8 *ip = (GH8 *)((const _Float16 *)d.ihp + (lower ? kPlaneHalves : 0));
-  const int eI = d.ihe[lower ? 1 : 0];
+  const int slot = step % d.group;
+  GH8 *ip = (GH8 *)((const _Float16 *)d.ihp + slot * (2 * kPlaneHalves) + (lower ? kPlaneHalves : 0));
+  const int eI = d.ihe[2 * slot + (lower ? 1 : 0)];
   f4 cr[2][2], ci[2][2];
 #pragma unroll
   for (int bi = 0; bi < 2; bi++)
@@ -450,10 +459,9 @@ __device__ __forceinline__ void panel_tile_h(const SolveDesc &d, int step, int n
         Ts[wc + 16 * bj + acc_row<float>(kq, r)][wr + 16 * bi + li] = o;
       }
   // split-FP16 planes of this panel tile for the split updates
-  const int parity = step % d.group, side = lower ? 0 : 1;
-  const int t = lower ? ti : tj;
-  write_split_planes(Ts, lower, (_Float16 *)d.hp + (long)((parity * 2 + side) * d.nt + t) * kPlaneHalves,
-                     d.he + (parity * 2 + side) * d.nt + t);
+  const int side = lower ? 0 : 1;
+  write_split_planes(Ts, lower, (_Float16 *)d.hp + (long)((slot * 2 + side) * d.nt + t) * kPlaneHalves,
+                     d.he + (slot * 2 + side) * d.nt + t);
 }
 
 // Panel of step `step` with its cross update (panel_op): L_is = C' U^-1 for the
@@ -489,18 +497,52 @@ __global__ __launch_bounds__(256) void k_lu_panel(const SolveDesc *__restrict__ 
     panel_op<T, N, kLeftL>(C, true, false, A, sa, B, sb, ld, ncross, inv, perm, piece, lds);
 }
 
-// Panel of step `step` on the split-FP16 path with its cross update fused:
-// the tiles of column and row `step` first take the ncross steps before it
-// in its group (planes in the group's slots), then the panel.  With
-// xcd_swizzle the workgroups of one solve run on one XCD (xcd_remap), so the
-// planes its tiles share (the U planes of the step's column, the L planes of
-// its row) are fetched into one L2.
+// Panels of a group on the split-FP16 path.  k_lu_panel_h takes the tiles of
+// one step: all of its column and row, or in large launches (launch_lu_steps)
+// those inside the group's diagonal block alone (rows and columns up to its
+// last step), which the next diagonal tiles wait for; then each tile row below
+// the block, and each tile column right of it, runs through all the group's
+// steps in one workgroup (k_lu_strip_h).  Both read a tile's planes of every
+// earlier step of the group again, from HBM mostly; a strip shares the block's
+// planes with the others at the same step through L2, and saves the launches'
+// ends (248 solves N = 2160: 14.7 -> 13.4 ms a pass for the panels).
+// The workgroups of one solve run on one XCD (xcd_remap; for k_lu_panel_h with
+// xcd_swizzle), so that the planes they share are fetched into one L2.
+
+// the last step of the group starting at solve step g
+__device__ __forceinline__ int group_last(const SolveDesc &d, int g) {
+  return min(g + d.group, d.nt - 1) - 1;
+}
+
 __global__ __launch_bounds__(256) void k_lu_panel_h(const SolveDesc *__restrict__ descs, int step,
-                                                      int ncross, int xcd_swizzle) {
+                                                    int ncross, int whole, int xcd_swizzle) {
   int bx = blockIdx.x, by = blockIdx.y;
   if (xcd_swizzle) xcd_remap(bx, by);
   const SolveDesc &d = descs[by];
-  panel_tile_h(d, step - d.step0, ncross, bx);
+  const int s = step - d.step0;
+  if (s - ncross < 0) return;
+  const int n = (whole ? d.nt - 1 : group_last(d, s - ncross)) - s;
+  if (bx >= 2 * n) return;
+  if (d.conv && *d.conv) return;
+  panel_tile_h(d, s, ncross, bx < n, s + 1 + (bx < n ? bx : bx - n));
+}
+
+__global__ __launch_bounds__(256, 3) void k_lu_strip_h(const SolveDesc *__restrict__ descs, int step) {
+  int bx = blockIdx.x, by = blockIdx.y;
+  xcd_remap(bx, by);
+  const SolveDesc &d = descs[by];
+  const int g = step - d.step0;
+  if (g < 0) return;
+  const int last = group_last(d, g), n = d.nt - 1 - last;
+  if (last < g || bx >= 2 * n) return;
+  if (d.conv && *d.conv) return;
+  const bool lower = bx < n;
+  const int t = last + 1 + (lower ? bx : bx - n);
+#pragma unroll 1
+  for (int s = g; s <= last; s++) {
+    if (s > g) __syncthreads();  // the planes of step s-1 are written, Ts is read
+    panel_tile_h(d, s, s - g, lower, t);
+  }
 }
 
 // C(ti, tj) -= sum_{u < ns} L(ti, s0+u) U(s0+u, tj): one 64x64 tile per
