@@ -3,6 +3,8 @@
 // 16x16x4 MFMA wrappers with their accumulator layout, and the 3M complex
 // wave product used by every trailing update.
 #pragma once
+#include <type_traits>
+
 #include "lsmsx_device.hpp"
 
 namespace lsmsx {
@@ -345,10 +347,7 @@ __device__ __forceinline__ void panel_op(GCx<T> *__restrict__ C, bool load_c, bo
   const int wr = N == 2 ? 32 * (w & 1) : RIGHT ? 0 : 16 * w;
   const int wc = N == 2 ? 32 * (w >> 1) : RIGHT ? 16 * w : 0;
   const int r0 = N == 2 || !RIGHT ? 0 : 16 * piece, c0 = N == 2 || RIGHT ? 0 : 16 * piece;
-  if (OP == kLeftL) {
-    if (tid < kTile) rowpos[perm[tid]] = tid;
-    __syncthreads();
-  }
+  if (OP == kLeftL && tid < kTile) rowpos[perm[tid]] = tid;
   GCx<T> *Cw = C + (r0 + wr) + ld * (c0 + wc);
   Acc3<T, N> q;
 #pragma unroll
@@ -364,6 +363,7 @@ __device__ __forceinline__ void panel_op(GCx<T> *__restrict__ C, bool load_c, bo
         set_minus<T, N>(q, bj, bi, r, c.x, c.y);
       }
   tile_products<T, N>(A + (r0 + wr), sa, B + ld * (c0 + wc), sb, ld, ns, q);
+  if (OP == kLeftL) __syncthreads();  // rowpos
 #pragma unroll
   for (int bj = 0; bj < N; bj++)
 #pragma unroll
@@ -375,48 +375,87 @@ __device__ __forceinline__ void panel_op(GCx<T> *__restrict__ C, bool load_c, bo
       }
   __syncthreads();
   zero_acc(q);
-  // the triangular factor's zero blocks are left out: of a 16-column (row)
-  // strip only the k-steps up to its diagonal block, or from it on
-  const int lim = RIGHT ? wc + 16 * N : wr + 16 * N;
-  if constexpr (OP == kRightU) {
-    // A(i,k) = C'(wr+i, k); B(k,j) = U^-1(k, wc+j), upper incl. diagonal
-    wave_gemm3m<T, N>([&](int i, int k) { return Ts[k][wr + i]; },
-                      [&](int k, int j) {
-                        const int jj = wc + j;
-                        V v = ldg<T>(inv + (k + kTile * jj));
-                        if (k > jj) v = czero<V>();
-                        return v;
-                      },
-                      lim / 4, q);
-  } else if constexpr (OP == kLeftL) {
-    // A(i,k) = L^-1(wr+i, k), unit lower; B(k,j) = (P C')(k, wc+j)
-    wave_gemm3m<T, N>([&](int i, int k) {
-                        const int ii = wr + i;
-                        V v = ldg<T>(inv + (ii + kTile * k));
-                        if (ii <= k) {
-                          v.x = ii == k ? T(1) : T(0);
-                          v.y = T(0);
-                        }
-                        return v;
-                      },
-                      [&](int k, int j) { return Ts[wc + j][k]; }, lim / 4, q);
+  // Second product, by 16-wide strips of the triangular side (columns of U^-1,
+  // rows of the left factors).  Strip t takes the k-steps up to its diagonal
+  // block, or from it on: for N = 2 a wave has strips t and 3 - t, so that all
+  // waves have the same work and none is done on the zero blocks.
+  const int t0 = N == 2 ? (RIGHT ? w >> 1 : w & 1) : w;
+  auto strip = [&](int b) { return 16 * (N == 2 && b ? 3 - t0 : t0); };
+  // element k of the triangular factor at offset x of strip b
+  auto tri = [&](int b, int x, int k) __attribute__((always_inline)) {
+    const int ii = strip(b) + x;
+    V v = ldg<T>(inv + (OP == kRightU ? k + kTile * ii : ii + kTile * k));
+    if (OP == kLeftL) {
+      if (ii <= k) {
+        v.x = ii == k ? T(1) : T(0);
+        v.y = T(0);
+      }
+    } else if (OP == kRightU ? k > ii : k < ii) {
+      v = czero<V>();
+    }
+    return v;
+  };
+  const int pr = N == 2 ? wr : 0, pc = N == 2 ? wc : 0;  // the wave's rows (columns) of C'
+  auto full = [&](int k0, int nk) __attribute__((always_inline)) {
+    if constexpr (RIGHT)
+      wave_gemm3m<T, N>([&](int i, int k) { return Ts[k0 + k][pr + i]; },
+                        [&](int k, int j) { return tri(j >> 4, j & 15, k0 + k); }, nk, q);
+    else
+      wave_gemm3m<T, N>([&](int i, int k) { return tri(i >> 4, i & 15, k0 + k); },
+                        [&](int k, int j) { return Ts[pc + j][k0 + k]; }, nk, q);
+  };
+  // k-steps of one strip alone, b the one that is longer
+  auto half = [&](auto bc, int k0, int nk) __attribute__((always_inline)) {
+    constexpr int b = decltype(bc)::value;
+    for (int ks = 0; ks < nk; ks += 4) {
+      V av[4][2], bv[4][2];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int k = k0 + 4 * (ks + u) + kq;
+        if constexpr (RIGHT) {
+          bv[u][b] = tri(b, li, k);
+          av[u][0] = Ts[k][pr + li];
+          av[u][1] = Ts[k][pr + 16 + li];
+        } else {
+          av[u][b] = tri(b, li, k);
+          bv[u][0] = Ts[pc + li][k];
+          bv[u][1] = Ts[pc + 16 + li][k];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+          const int bi = RIGHT ? o : b, bj = RIGHT ? b : o;
+          const V x = av[u][bi], y = bv[u][bj];
+          q.p[0][bj][bi] = mfma4(y.x, x.x, q.p[0][bj][bi]);
+          q.p[1][bj][bi] = mfma4(y.y, x.y, q.p[1][bj][bi]);
+          q.p[2][bj][bi] = mfma4(y.x + y.y, x.x + x.y, q.p[2][bj][bi]);
+        }
+    }
+  };
+  if constexpr (N == 1) {
+    if (OP == kLeftU) full(16 * t0, 16 - 4 * t0);
+    else full(0, 4 * t0 + 4);
+  } else if constexpr (OP == kLeftU) {
+    // strip 3 - t starts at its own block, strip t before it
+    half(std::integral_constant<int, 0>(), 16 * t0, 4 * (3 - 2 * t0));
+    full(16 * (3 - t0), 4 * t0 + 4);
   } else {
-    // A(i,k) = U^-1(wr+i, k), upper incl. diagonal; B(k,j) = C'(k, wc+j): k >= wr
-    wave_gemm3m<T, N>([&](int i, int k) {
-                        const int ii = wr + i;
-                        V v = ldg<T>(inv + (ii + kTile * (wr + k)));
-                        if (wr + k < ii) v = czero<V>();
-                        return v;
-                      },
-                      [&](int k, int j) { return Ts[wc + j][wr + k]; }, (kTile - wr) / 4, q);
+    full(0, 4 * t0 + 4);
+    half(std::integral_constant<int, 1>(), 16 * (t0 + 1), 4 * (3 - 2 * t0));
   }
+  GCx<T> *Cp = C + (RIGHT ? r0 + pr : 0) + ld * (RIGHT ? 0 : c0 + pc);
 #pragma unroll
   for (int bj = 0; bj < N; bj++)
 #pragma unroll
     for (int bi = 0; bi < N; bi++)
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-        Cw[(16 * bi + li) + ld * (16 * bj + acc_row<T>(kq, r))] = plus_value<T, N>(q, bj, bi, r);
+      for (int r = 0; r < 4; r++) {
+        const int i = (RIGHT ? 16 * bi : strip(bi)) + li;
+        const int j = (RIGHT ? strip(bj) : 16 * bj) + acc_row<T>(kq, r);
+        Cp[i + ld * j] = plus_value<T, N>(q, bj, bi, r);
+      }
 }
 
 // Split-FP16 operands: eight halves of a 32-wide k chunk per lane, the
