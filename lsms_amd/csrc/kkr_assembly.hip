@@ -247,8 +247,8 @@ __device__ __forceinline__ void load_tables(const double *__restrict__ cgnt_g,
                                             int *lofk) {
   const int tid = threadIdx.x;
   const int kkr_tab = (lmax_tab + 1) * (lmax_tab + 1);
-  for (int t = tid; t < (lmax_tab + 1) * kkr_tab * kkr_tab; t += 256) cg[t] = cgnt_g[t];
-  for (int t = tid; t < kkr_tab * kkr_tab; t += 256) il[t] = illp_g[t];
+  for (int t = tid; t < (lmax_tab + 1) * kkr_tab * kkr_tab; t += blockDim.x) cg[t] = cgnt_g[t];
+  for (int t = tid; t < kkr_tab * kkr_tab; t += blockDim.x) il[t] = illp_g[t];
   if (tid < (kLmaxD + 1) * (kLmaxD + 1)) {
     int l = tid / (kLmaxD + 1), m = tid % (kLmaxD + 1);
     double a = 0.0, b = 0.0;
@@ -275,7 +275,7 @@ __device__ __forceinline__ void load_tables(const double *__restrict__ cgnt_g,
 // 16-aligned offset and zero-padded for the MFMA products.
 __device__ __forceinline__ void load_tpack(const double2 *__restrict__ T, int nsc, int kkrsz,
                                            int ldt, int kkri, double2 (*tn)[2 * kMaxKkr + 1]) {
-  for (int t = threadIdx.x; t < 4 * kMaxKkr * kMaxKkr; t += 256) {
+  for (int t = threadIdx.x; t < 4 * kMaxKkr * kMaxKkr; t += blockDim.x) {
     int r = t % (2 * kMaxKkr), c = t / (2 * kMaxKkr);
     int rs = r / kMaxKkr, ri = r % kMaxKkr, cs = c / kMaxKkr, ci = c % kMaxKkr;
     double2 v = make_double2(0.0, 0.0);
@@ -762,8 +762,13 @@ template __global__ void k_assemble_from_g<kAsmGW>(const SolveDesc *, const doub
 //   gx(site i rows) = sum_j diag_spin(G_ij) X_j,   X = M^-1 [0; t0]  (d.X)
 // tdot = dt/dE from the derivative store dtmat (same layout as tmat); with
 // dtmat == nullptr only gx is formed.  The (i, i) blocks are constant (M_ii =
-// 1, G_ii = 0) and contribute nothing.
-__global__ __launch_bounds__(256) void k_lloyd(const SolveDesc *__restrict__ descs,
+// 1, G_ii = 0) and contribute nothing.  A wave takes every eighth site j, one
+// after another, and each is a chain of latencies (special functions, Gaunt
+// sums through LDS); the tables leave room for one workgroup per compute unit,
+// so its eight waves are what overlaps (472 sites of eight solves: 278 us with
+// four, 177 with eight).
+constexpr int kLloydWaves = 8;
+__global__ __launch_bounds__(kLloydWaves * 64) void k_lloyd(const SolveDesc *__restrict__ descs,
                                                const double2 *__restrict__ tmat,
                                                const double2 *__restrict__ dtmat, long ldT,
                                                const double *__restrict__ cgnt_g,
@@ -780,10 +785,10 @@ __global__ __launch_bounds__(256) void k_lloyd(const SolveDesc *__restrict__ des
   __shared__ double pa[kLmaxD + 1][kLmaxD + 1], pb[kLmaxD + 1][kLmaxD + 1];
   __shared__ double pmmf[kLmaxD + 1], pm1f[kLmaxD + 1];
   __shared__ int lofk[kNd];
-  __shared__ double2 dl[4][kNd], ddl[4][kNd];
-  __shared__ double2 gs[4][kMaxKkr * kMaxKkr], gds[4][kMaxKkr * kMaxKkr];
+  __shared__ double2 dl[kLloydWaves][kNd], ddl[kLloydWaves][kNd];
+  __shared__ double2 gs[kLloydWaves][kMaxKkr * kMaxKkr], gds[kLloydWaves][kMaxKkr * kMaxKkr];
   __shared__ double2 red[2 * kMaxKkr][2 * kMaxKkr + 1];
-  __shared__ double2 trs[4];
+  __shared__ double2 trs[kLloydWaves];
 
   const int nsc = d.n_spin_cant, kc = d.kc, Ns = d.Ns;
   const int lmi = d.lmax[i], kkri = (lmi + 1) * (lmi + 1), kkri_ns = kkri * nsc;
@@ -812,7 +817,7 @@ __global__ __launch_bounds__(256) void k_lloyd(const SolveDesc *__restrict__ des
 #pragma unroll
       for (int m = 0; m < 3; m++) gq[bs][cb][m] = d4{0.0, 0.0, 0.0, 0.0};
 
-  for (int j = w; j < d.numLIZ; j += 4) {
+  for (int j = w; j < d.numLIZ; j += kLloydWaves) {
     if (j == i) continue;
     const int lmj = d.lmax[j], kkrj = (lmj + 1) * (lmj + 1);
     const int offj = d.site_off[j];
@@ -893,7 +898,7 @@ __global__ __launch_bounds__(256) void k_lloyd(const SolveDesc *__restrict__ des
     tr.y += __shfl_xor(tr.y, off, 64);
   }
   if (lane == 0) trs[w] = tr;
-  for (int ww = 0; ww < 4; ww++) {
+  for (int ww = 0; ww < kLloydWaves; ww++) {
     if (w == ww) {
 #pragma unroll
       for (int bs = 0; bs < 2; bs++)
@@ -913,38 +918,39 @@ __global__ __launch_bounds__(256) void k_lloyd(const SolveDesc *__restrict__ des
   }
   if (threadIdx.x == 0) {
     double2 s = make_double2(0.0, 0.0);
-    for (int ww = 0; ww < 4; ww++) {
+    for (int ww = 0; ww < kLloydWaves; ww++) {
       s.x += trs[ww].x;
       s.y += trs[ww].y;
     }
     d.lpart[i] = s;
   }
-  for (int e = threadIdx.x; e < kkri_ns * kc; e += 256) {
+  for (int e = threadIdx.x; e < kkri_ns * kc; e += kLloydWaves * 64) {
     const int p = e % kkri_ns, col = e / kkri_ns;
     const int bs = p / kkri, a = p % kkri;
     d.gx[(offi + p) + (long)Ns * col] = red[bs * kMaxKkr + a][col];
   }
 }
 
-// Identity in the leading pad rows/columns of the solver layout.
+// Identity in the leading pad rows/columns of the solver layout: workgroup t
+// takes rows 64t .. of the pad columns and the pad rows of columns 64t .. (one
+// workgroup per solve took 42 us for N = 2160, 159 for N = 4384).
 __global__ __launch_bounds__(256) void k_pad_identity(const SolveDesc *__restrict__ descs) {
-  const SolveDesc &d = descs[blockIdx.x];
-  const int pad = d.pad;
-  if (pad == 0) return;
+  const SolveDesc &d = descs[blockIdx.y];
+  const int pad = d.pad, t = blockIdx.x;
+  if (pad == 0 || t >= d.nt) return;
   double2 *M = d.M;
   float2 *W = d.w32;
   const long ld = d.ld;
-  // columns 0..pad-1: full columns; columns pad..Ns-1: rows 0..pad-1
-  for (long e = threadIdx.x; e < (long)pad * d.Ns; e += blockDim.x) {
-    int rr = (int)(e % d.Ns), cc = (int)(e / d.Ns);
-    if (M) M[rr + ld * cc] = make_double2(rr == cc ? 1.0 : 0.0, 0.0);
-    if (W) W[tiled_index(rr, cc, d.nt)] = make_float2(rr == cc ? 1.f : 0.f, 0.f);
-  }
-  for (long e = threadIdx.x; e < (long)pad * (d.Ns - pad); e += blockDim.x) {
-    int rr = (int)(e % pad), cc = pad + (int)(e / pad);
-    if (M) M[rr + ld * cc] = make_double2(0.0, 0.0);
-    if (W) W[tiled_index(rr, cc, d.nt)] = make_float2(0.f, 0.f);
-  }
+  auto put = [&](int r, int c) {
+    const double v = r == c ? 1.0 : 0.0;
+    if (M) M[r + ld * c] = make_double2(v, 0.0);
+    if (W) W[tiled_index(r, c, d.nt)] = make_float2((float)v, 0.f);
+  };
+  const int a = threadIdx.x & 63;
+  for (int c = threadIdx.x >> 6; c < pad; c += 4) put(kTile * t + a, c);
+  if (a < pad)
+    for (int c = kTile * t + (threadIdx.x >> 6); c < kTile * (t + 1); c += 4)
+      if (c >= pad) put(a, c);
 }
 
 }  // namespace lsmsx

@@ -568,7 +568,7 @@ int launch_lu(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool split_
 template <class T>
 int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int max_sweeps,
            double tol, int *left) {
-  hipLaunchKernelGGL(k_ir_init<T>, dim3(nb), dim3(256), 0, c->stream, dd);
+  hipLaunchKernelGGL(k_ir_init<T>, dim3(nt_max, nb), dim3(256), 0, c->stream, dd);
   if (int r = check_launch("k_ir_init")) return r;
   int done = 0;
   for (int it = 0; it < max_sweeps; it++) {
@@ -624,7 +624,7 @@ int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int ma
 // part's refinement can then run beside another part's factorization.
 int refine_async(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int max_sweeps,
                  double tol, hipStream_t st, int nbands_max) {
-  hipLaunchKernelGGL(k_ir_init<float>, dim3(nb), dim3(256), 0, st, dd);
+  hipLaunchKernelGGL(k_ir_init<float>, dim3(nt_max, nb), dim3(256), 0, st, dd);
   for (int it = 0; it < max_sweeps; it++) {
     if (it > 0) {
       ProfScope p(c, 5);
@@ -1010,7 +1010,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
       if (int r = check_launch("k_init_status")) return r;
       {
         ProfScope p(c, 0);
-        hipLaunchKernelGGL(k_pad_identity, dim3(n), dim3(256), 0, st, dd);
+        hipLaunchKernelGGL(k_pad_identity, dim3(ntm, n), dim3(256), 0, st, dd);
         if (share)
           launch_assemble_from_g(c, dim3(mliz, n), st, dd, asm_mode);
         else
@@ -1394,7 +1394,7 @@ int run_adjoint(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
     hipLaunchKernelGGL(k_init_status, dim3((nb + 255) / 256), dim3(256), 0, c->stream, c->desc.p, nb);
     {
       ProfScope p(c, 0);
-      hipLaunchKernelGGL(k_pad_identity, dim3(nb), dim3(256), 0, c->stream, c->desc.p);
+      hipLaunchKernelGGL(k_pad_identity, dim3(nt_max, nb), dim3(256), 0, c->stream, c->desc.p);
       launch_assemble(c, nsc, dim3(maxliz, nb), c->stream, c->desc.p);
     }
     if (int r = check_launch("k_assemble")) return r;
@@ -1402,7 +1402,7 @@ int run_adjoint(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
     {
       ProfScope p(c, 8);
       hipLaunchKernelGGL(k_inv_x, dim3(nt_max, nb), dim3(256), 0, c->stream, c->desc.p);
-      hipLaunchKernelGGL(k_lloyd, dim3(maxliz, nb), dim3(256), 0, c->stream, c->desc.p, c->tmat.p,
+      hipLaunchKernelGGL(k_lloyd, dim3(maxliz, nb), dim3(512), 0, c->stream, c->desc.p, c->tmat.p,
                          lloyd_out ? c->dtmat.p : nullptr, c->ldT, c->cgnt.p, c->illp.p,
                          c->lmax_tab);
       hipLaunchKernelGGL(k_lloyd_reduce, dim3((nb + 63) / 64), dim3(64), 0, c->stream, c->desc.p,
@@ -2191,7 +2191,7 @@ int lsmsx_tau_full(lsmsx_ctx *c, int atom_id, int ispin, int iie, const double *
   hipLaunchKernelGGL(k_init_status, dim3(1), dim3(64), 0, c->stream, c->desc.p, 1);
   {
     ProfScope p(c, 0);
-    hipLaunchKernelGGL(k_pad_identity, dim3(1), dim3(256), 0, c->stream, c->desc.p);
+    hipLaunchKernelGGL(k_pad_identity, dim3(nt), dim3(256), 0, c->stream, c->desc.p);
     launch_assemble(c, nsc, dim3(a.numLIZ, 1), c->stream, c->desc.p);
   }
   if (int r = check_launch("k_assemble")) return r;
