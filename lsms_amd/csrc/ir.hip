@@ -635,41 +635,49 @@ __global__ void k_ir_decide(const SolveDesc *__restrict__ descs, int n, double t
 // central rows between the forward and the backward halves, and X += dX.  It
 // does the work of k_ir_step, k_ir_accum and k_ir_decide for one sweep.
 //
-// Left-looking by tile row, with the tile rows dealt round-robin to the
-// waves of the workgroup: wave w takes t = w, w+8, ... (forward, ascending)
-// and computes
-//   y_t = L_tt^-1 P_t (r_t - sum_{s<t} L_ts y_s)
-// with the 64 x 16 block in MFMA accumulators (4M form), then publishes y_t
-// (in place of r_t in R) by a workgroup-scope flag in LDS; the waves that
-// need y_s wait on its flag.  The backward half runs the same way from the
-// last tile down (x_t = U_tt^-1 (y_t - sum_{s>t} U_ts x_s)).  Every wave
-// waits only for tiles below its own (above, backward) and takes its tiles
-// in order, so the waits always end.  The diagonal-tile inverse is applied
-// as one more 64 x 64 operand, its input staged in the wave's LDS slot.
+// Left-looking by tile row, with the tile rows dealt round-robin to teams of
+// NW = 4/RB waves (one wave, or a pair): team p of n takes t = p, p+n, ...
+// (forward, ascending) and computes
+//   y_t = L_tt^-1 P_t (r_t - sum_{s<t} L_ts y_s),
+// 16 RB rows by each wave, with its block in MFMA accumulators (3M form), then
+// publishes y_t (in place of r_t in R) by a workgroup-scope count in LDS; the
+// waves that need y_s wait on it.  The backward half runs the same way from
+// the last tile down (x_t = U_tt^-1 (y_t - sum_{s>t} U_ts x_s)).  Every wave
+// waits only for tiles below its own (above, backward) and, before the
+// diagonal product, for its partner at the same tile, and takes its tiles in
+// order, so the waits always end.  The diagonal-tile inverse is applied as one
+// more operand, its input staged in the team's LDS slot (a pair has two in
+// turn: a wave writes one while its partner may still read the other).
 // All operand tiles (L_ts, U_ts, the inverses) stream from HBM through a
-// ring of kSweepD k-steps per wave that runs on across tiles; the published
-// y_s / x_s come from L2, one item ahead when its flag is already set.
+// ring of k-steps per wave that runs on across tiles; the published y_s / x_s
+// come from L2, one item ahead when its count is already full.
 // HBM traffic per sweep: the factors once, R and X; no launch per tile
 // column.  The first sweep (R = B, zero outside the last tile, so y_t = 0
 // for t < nt-1 under tile-local pivoting) runs only the last tile forward.
-constexpr int kSweepD = 4;  // k-steps (4 columns of a 64 x 64 operand) in flight per wave
+// With few tiles the sweep is the chain of its diagonal tiles (update with
+// the last y, diagonal product, publish), half as long by pairs; with many it
+// is HBM or a compute unit's MFMAs, and single waves read y half as often
+// (sweep_pairs has both sides).  The arithmetic of both is the same.
 
-template <bool FIRST>
+template <bool FIRST, int RB>
 __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *__restrict__ descs,
                                                                double tol) {
   typedef float2 V;
+  constexpr int NW = 4 / RB, NT = kSweepWaves / NW;  // waves of a team, teams
+  // k-steps (4 columns of a 16 RB x 64 operand) in flight per wave
+  constexpr int kSweepD = 16 / RB;
   const SolveDesc &d = descs[blockIdx.x];
   if (*d.conv) return;
   const int nt = d.nt, Ns = d.Ns;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  __shared__ V slot[kSweepWaves][kTile][17];  // a wave's block, input of its diagonal step
-  __shared__ int pslot[kSweepWaves][kTile];
-  __shared__ int ready[kSweepMaxTiles], done[kSweepMaxTiles];
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), team = w / NW, half = w % NW;
+  __shared__ V slot[NT][NW][kTile][17];  // a team's block, input of its diagonal step
+  __shared__ int ready[kSweepMaxTiles], done[kSweepMaxTiles], arrived[NT];
   __shared__ int conv_flag;
   for (int i = tid; i < kSweepMaxTiles; i += kSweepWaves * 64) {
     ready[i] = 0;
     done[i] = 0;
+    if (i < NT) arrived[i] = 0;
   }
   __syncthreads();
   GCx<float> *R = (GCx<float> *)d.R;
@@ -678,16 +686,18 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   const GCx<float> *__restrict__ Inv = (const GCx<float> *)d.inv;
   const LSMSX_GLOBAL int *Perm = (const LSMSX_GLOBAL int *)d.perm;
   const long istr = d.inv_stride;
-  const int loff = li + kTile * kq;
+  const int row0 = 16 * RB * half;  // the wave's rows of a tile
+  const int loff = row0 + li + kTile * kq;
 
-  f4 cr[4], ci[4];  // the current tile row's 64 x 16 block: (16 rb + li, 4 kq + r)
-  V ycur[16], ynext[16];  // y_s / x_s operand: (4 kk + kq, li)
+  f4 q1[RB], q2[RB], q3[RB];  // 3M sums of the wave's block: (16 rb + li, 4 kq + r)
+  V ycur[16], ynext[16];   // y_s / x_s operand: (4 kk + kq, li)
+  int phase = 0;           // diagonal products of the team so far
 
-  // ---- operand stream.  Items are 64 x 64 column-major operands, consumed
-  // 4 columns (one k-step) at a time.  Forward items of tile t: s < t: L_ts,
-  // s == t: the inverse (lower part), s == t+1: the inverse again (upper
-  // part; last tile only).  Backward items of tile t: s > t: U_ts, s == t:
-  // the inverse (upper part).
+  // ---- operand stream.  Items are the wave's rows of 64 x 64 column-major
+  // operands, consumed 4 columns (one k-step) at a time.  Forward items of
+  // tile t: s < t: L_ts, s == t: the inverse (lower part), s == t+1: the
+  // inverse again (upper part; last tile only).  Backward items of tile t:
+  // s > t: U_ts, s == t: the inverse (upper part).
   auto item_base = [&](bool fwd, int t, int s) __attribute__((always_inline)) -> const GCx<float> * {
     const bool inv = fwd ? s >= t : s == t;
     return inv ? Inv + t * istr : F + ((long)s * nt + t) * (kTile * kTile);
@@ -699,7 +709,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
         return true;
       }
       if (FIRST) return false;
-      t += kSweepWaves;
+      t += NT;
       s = 0;
       return t < nt;
     }
@@ -707,11 +717,11 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
       s--;
       return true;
     }
-    t -= kSweepWaves;
+    t -= NT;
     s = nt - 1;
     return t >= 0;
   };
-  V rg[kSweepD][4];
+  V rg[kSweepD][RB];
   const GCx<float> *cb = F;
   int pt = 0, ps = 0, pk = 0;
   bool pok = false;
@@ -721,7 +731,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   auto load_slot = [&](bool fwd, int u) __attribute__((always_inline)) {
     const GCx<float> *src = cb + kTile * 4 * pk + loff;
 #pragma unroll
-    for (int rb = 0; rb < 4; rb++) {
+    for (int rb = 0; rb < RB; rb++) {
       // the factor streams through once per sweep: non-temporal, so that the
       // published y_s / x_s blocks the waves read from L2 stay there
       typedef float sv2 __attribute__((ext_vector_type(2)));
@@ -747,99 +757,36 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
 #pragma unroll
     for (int u = 0; u < kSweepD; u++) load_slot(fwd, u);
   };
-  // block -= operand * ycur
+  // sums += operand * v, v in the MFMA's a-operand layout
+  auto step = [&](int rb, V l, V v, float vs) __attribute__((always_inline)) {
+    q1[rb] = mfma4(v.x, l.x, q1[rb]);
+    q2[rb] = mfma4(v.y, l.y, q2[rb]);
+    q3[rb] = mfma4(vs, l.x + l.y, q3[rb]);
+  };
   auto consume_update = [&](bool fwd) __attribute__((always_inline)) {
 #pragma unroll
     for (int kk = 0; kk < 16; kk++) {
       const int u = kk % kSweepD;
       const V yv = ycur[kk];
+      const float ys = yv.x + yv.y;
 #pragma unroll
-      for (int rb = 0; rb < 4; rb++) {
-        const V l = rg[u][rb];
-        cr[rb] = mfma4(yv.x, -l.x, cr[rb]);
-        cr[rb] = mfma4(yv.y, l.y, cr[rb]);
-        ci[rb] = mfma4(yv.y, -l.x, ci[rb]);
-        ci[rb] = mfma4(yv.x, -l.y, ci[rb]);
-      }
+      for (int rb = 0; rb < RB; rb++) step(rb, rg[u][rb], yv, ys);
       load_slot(fwd, u);
     }
   };
-  // block = operand * In, In = the wave's slot (rows permuted by pslot for
-  // the unit lower L^-1; as stored for the upper U^-1, diagonal included)
-  auto consume_diag = [&](bool fwd, bool upper) __attribute__((always_inline)) {
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++) {
-      cr[rb] = f4{0.f, 0.f, 0.f, 0.f};
-      ci[rb] = cr[rb];
-    }
-#pragma unroll
-    for (int kk = 0; kk < 16; kk++) {
-      const int u = kk % kSweepD, k = 4 * kk + kq;
-      const V in = upper ? slot[w][k][li] : slot[w][pslot[w][k]][li];
-#pragma unroll
-      for (int rb = 0; rb < 4; rb++) {
-        const int i = 16 * rb + li;
-        V op = rg[u][rb];
-        if (upper ? k < i : k >= i) {
-          op.x = (!upper && k == i) ? 1.f : 0.f;
-          op.y = 0.f;
-        }
-        cr[rb] = mfma4(in.x, op.x, cr[rb]);
-        cr[rb] = mfma4(in.y, -op.y, cr[rb]);
-        ci[rb] = mfma4(in.y, op.x, ci[rb]);
-        ci[rb] = mfma4(in.x, op.y, ci[rb]);
-      }
-      load_slot(fwd, u);
-    }
+  // block - sums of the updates (set by load_block) and plain sums
+  auto minus = [&](int rb, int r) __attribute__((always_inline)) {
+    return make_float2(q2[rb][r] - q1[rb][r], q1[rb][r] + q2[rb][r] - q3[rb][r]);
   };
-  auto block_to_slot = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) slot[w][16 * rb + li][4 * kq + r] = make_float2(cr[rb][r], ci[rb][r]);
-  };
-  auto load_block = [&](int t) __attribute__((always_inline)) {
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const V v = ldg<float>(R + (t * kTile + 16 * rb + li) + (long)Ns * (4 * kq + r));
-        cr[rb][r] = v.x;
-        ci[rb][r] = v.y;
-      }
-  };
-  auto store_block = [&](int t) __attribute__((always_inline)) {
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        R[(t * kTile + 16 * rb + li) + (long)Ns * (4 * kq + r)] = make_float2(cr[rb][r], ci[rb][r]);
-  };
-  // X += the block of tile t; returns the central-row sums (rb = 3 of the
-  // last tile: rows Ns-16 .. Ns-1)
-  auto add_to_x = [&](int t, double &dn, double &xn) __attribute__((always_inline)) {
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const long idx = (t * kTile + 16 * rb + li) + (long)Ns * (4 * kq + r);
-        const float dr = cr[rb][r], di = ci[rb][r];
-        double2 x = X[idx];
-        x.x += dr;
-        x.y += di;
-        X[idx] = x;
-        if (rb == 3) {
-          dn += (double)dr * dr + (double)di * di;
-          xn += x.x * x.x + x.y * x.y;
-        }
-      }
+  auto plus = [&](int rb, int r) __attribute__((always_inline)) {
+    return make_float2(q1[rb][r] - q2[rb][r], q3[rb][r] - q1[rb][r] - q2[rb][r]);
   };
   // Every wait ends (see above); the spin bound (about half a second) only
   // guards the GPU against a broken invariant: the solve then reports
   // kInfoSweepStall and the wave goes on, so the kernel still exits.
-  auto wait_flag = [&](int *flag) __attribute__((always_inline)) {
+  auto wait_count = [&](int *count, int n) __attribute__((always_inline)) {
     unsigned spins = 0;
-    while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) {
+    while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < n) {
       if (++spins > kSweepSpinLimit) {
         if (lane == 0) *d.info = kInfoSweepStall;
         break;
@@ -848,32 +795,111 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   };
-  auto flag_set = [&](int *flag) __attribute__((always_inline)) {
-    return __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0;
+  auto count_full = [&](int *count) __attribute__((always_inline)) {
+    return __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= NW;
   };
-  auto publish = [&](int *flag) __attribute__((always_inline)) {
+  auto publish = [&](int *count) __attribute__((always_inline)) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    if (lane == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (lane == 0)
+      __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  // block = operand * In, In = the team's slot (rows in pivot order for the
+  // unit lower L^-1; as stored for the upper U^-1, diagonal included): the
+  // wave's half of In is already in the slot
+  auto consume_diag = [&](bool fwd, bool upper, const int (&prow)[16]) __attribute__((always_inline)) {
+    const V(*in_slot)[17] = slot[team][phase % NW];
+    phase++;
+    if (NW > 1) {
+      publish(arrived + team);
+      wait_count(arrived + team, NW * phase);
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++) {
+      q1[rb] = f4{0.f, 0.f, 0.f, 0.f};
+      q2[rb] = q1[rb];
+      q3[rb] = q1[rb];
+    }
+#pragma unroll
+    for (int kk = 0; kk < 16; kk++) {
+      const int u = kk % kSweepD, k = 4 * kk + kq;
+      const V in = in_slot[upper ? k : prow[kk]][li];
+      const float is = in.x + in.y;
+#pragma unroll
+      for (int rb = 0; rb < RB; rb++) {
+        const int i = row0 + 16 * rb + li;
+        V op = rg[u][rb];
+        if (upper ? k < i : k >= i) {
+          op.x = (!upper && k == i) ? 1.f : 0.f;
+          op.y = 0.f;
+        }
+        step(rb, op, in, is);
+      }
+      load_slot(fwd, u);
+    }
+  };
+  auto load_block = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const V v = ldg<float>(R + (t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r));
+        q1[rb][r] = -v.x;
+        q2[rb][r] = 0.f;
+        q3[rb][r] = -v.x - v.y;
+      }
+  };
+  auto block_to_slot = [&](auto value) __attribute__((always_inline)) {
+    V(*out)[17] = slot[team][phase % NW];
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) out[row0 + 16 * rb + li][4 * kq + r] = value(rb, r);
+  };
+  auto store_block = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        R[(t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r)] = plus(rb, r);
+  };
+  // X += the block of tile t; returns the sums over the last 16 rows (the
+  // central rows Ns-16 .. Ns-1 for the last wave of the last tile's team)
+  auto add_to_x = [&](int t, double &dn, double &xn) __attribute__((always_inline)) {
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const long idx = (t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r);
+        const V dx = plus(rb, r);
+        double2 x = X[idx];
+        x.x += dx.x;
+        x.y += dx.y;
+        X[idx] = x;
+        if (rb == RB - 1) {
+          dn += (double)dx.x * dx.x + (double)dx.y * dx.y;
+          xn += x.x * x.x + x.y * x.y;
+        }
+      }
   };
   auto load_y = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int kk = 0; kk < 16; kk++) ynext[kk] = ldg<float>(R + (s * kTile + 4 * kk + kq) + (long)Ns * li);
   };
   // the update items of a tile: steps s = first, first + dir, ..., last
-  // (inclusive), operand y_s / x_s published under flag[s]
-  auto run_updates = [&](bool fwd, int first, int last, int *flag) __attribute__((always_inline)) {
+  // (inclusive), operand y_s / x_s published under count[s]
+  auto run_updates = [&](bool fwd, int first, int last, int *count) __attribute__((always_inline)) {
     const int dir = fwd ? 1 : -1;
     bool have = false;
     for (int s = first; fwd ? s <= last : s >= last; s += dir) {
       if (!have) {
-        wait_flag(flag + s);
+        wait_count(count + s, NW);
         load_y(s);
       }
 #pragma unroll
       for (int kk = 0; kk < 16; kk++) ycur[kk] = ynext[kk];
       have = false;
       const int sn = s + dir;
-      if ((fwd ? sn <= last : sn >= last) && flag_set(flag + sn)) {
+      if ((fwd ? sn <= last : sn >= last) && count_full(count + sn)) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         load_y(sn);
         have = true;
@@ -883,21 +909,23 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   };
 
   // ---- forward half
-  const int tl = nt - 1, wl = tl % kSweepWaves;
+  const int tl = nt - 1, pl = tl % NT;
+  int prow[16] = {};
   {
-    const int t0 = FIRST ? tl : w;
-    const bool mine = FIRST ? w == wl : w < nt;
+    const int t0 = FIRST ? tl : team;
+    const bool mine = FIRST ? team == pl : team < nt;
     prime(true, t0, FIRST ? tl : 0, mine);
     if (mine) {
-      for (int t = t0; t < nt; t += kSweepWaves) {
+      for (int t = t0; t < nt; t += NT) {
         load_block(t);
+#pragma unroll
+        for (int kk = 0; kk < 16; kk++) prow[kk] = Perm[t * kTile + 4 * kk + kq];
         if (!FIRST && t > 0) run_updates(true, 0, t - 1, ready);
-        block_to_slot();
-        if (lane < kTile) pslot[w][lane] = Perm[t * kTile + lane];
-        consume_diag(true, false);
+        block_to_slot(minus);
+        consume_diag(true, false, prow);
         if (t == tl) {
-          block_to_slot();
-          consume_diag(true, true);
+          block_to_slot(plus);
+          consume_diag(true, true, prow);
           store_block(t);
           double dn = 0.0, xn = 0.0;
           add_to_x(t, dn, xn);
@@ -905,7 +933,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
             dn += __shfl_xor(dn, off, 64);
             xn += __shfl_xor(xn, off, 64);
           }
-          if (lane == 0) {
+          if (half == NW - 1 && lane == 0) {
             ir_decide_one(d, dn, xn, tol);
             conv_flag = *d.conv;
           }
@@ -920,15 +948,15 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   __syncthreads();
   if (conv_flag) return;
 
-  // ---- backward half: this wave's tiles below the last, descending
+  // ---- backward half: this team's tiles below the last, descending
   {
-    const int t0 = w <= nt - 2 ? w + kSweepWaves * ((nt - 2 - w) / kSweepWaves) : -1;
+    const int t0 = team <= nt - 2 ? team + NT * ((nt - 2 - team) / NT) : -1;
     prime(false, t0 < 0 ? 0 : t0, tl, t0 >= 0);
-    for (int t = t0; t >= 0; t -= kSweepWaves) {
+    for (int t = t0; t >= 0; t -= NT) {
       load_block(t);
       run_updates(false, tl, t + 1, done);
-      block_to_slot();
-      consume_diag(false, true);
+      block_to_slot(minus);
+      consume_diag(false, true, prow);
       store_block(t);
       double dn = 0.0, xn = 0.0;
       add_to_x(t, dn, xn);
@@ -985,7 +1013,9 @@ template __global__ void k_ir_step<double, true>(const SolveDesc *, int);
 template __global__ void k_ir_step<double, false>(const SolveDesc *, int);
 template __global__ void k_ir_accum<float>(const SolveDesc *, int);
 template __global__ void k_ir_accum<double>(const SolveDesc *, int);
-template __global__ void k_ir_sweep<true>(const SolveDesc *, double);
-template __global__ void k_ir_sweep<false>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<true, 2>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<true, 4>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<false, 2>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<false, 4>(const SolveDesc *, double);
 
 }  // namespace lsmsx

@@ -56,7 +56,7 @@ __global__ void k_ir_step(const SolveDesc *, int);
 template <class T>
 __global__ void k_ir_accum(const SolveDesc *, int);
 __global__ void k_ir_decide(const SolveDesc *, int, double);
-template <bool FIRST>
+template <bool FIRST, int RB>
 __global__ void k_ir_sweep(const SolveDesc *, double);
 __global__ void k_ir_residual_g(const SolveDesc *);
 __global__ void k_ir_residual_g_finish(const SolveDesc *);
@@ -617,6 +617,13 @@ int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int ma
   return 0;
 }
 
+// Whether the refinement sweeps take a tile row by a pair of waves: up to a
+// dozen tiles the chain of the diagonal tiles bounds a sweep (16 solves of four
+// tiles: 52.6 us a first sweep with single waves, 41.5 with pairs; 64 of ten
+// tiles: 154 and 125), beyond that HBM and the reads of y (96 solves of up to
+// 30 tiles: 682 and 812; 248 of 34: 1125 and 1161).
+inline bool sweep_pairs(int nt_max) { return nt_max <= 12; }
+
 // Refinement of a chunk part on stream st with no host round trip (mixed
 // path, kc = 16, k_ir_sweep): max_sweeps sweeps are enqueued up front; the
 // residual and sweep kernels return at once for solves already converged,
@@ -636,10 +643,10 @@ int refine_async(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int max_
       }
     }
     ProfScope p(c, 6);
-    if (it == 0)
-      hipLaunchKernelGGL(k_ir_sweep<true>, dim3(nb), dim3(kSweepWaves * 64), 0, st, dd, tol);
-    else
-      hipLaunchKernelGGL(k_ir_sweep<false>, dim3(nb), dim3(kSweepWaves * 64), 0, st, dd, tol);
+    const auto sweep = sweep_pairs(nt_max)
+                           ? (it == 0 ? k_ir_sweep<true, 2> : k_ir_sweep<false, 2>)
+                           : (it == 0 ? k_ir_sweep<true, 4> : k_ir_sweep<false, 4>);
+    hipLaunchKernelGGL(sweep, dim3(nb), dim3(kSweepWaves * 64), 0, st, dd, tol);
   }
   hipLaunchKernelGGL(k_ir_extract, dim3(nb), dim3(256), 0, st, dd);
   return check_launch("refine_async");
