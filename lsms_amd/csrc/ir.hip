@@ -649,8 +649,9 @@ __global__ void k_ir_decide(const SolveDesc *__restrict__ descs, int n, double t
 // more operand, its input staged in the team's LDS slot (a pair has two in
 // turn: a wave writes one while its partner may still read the other).
 // All operand tiles (L_ts, U_ts, the inverses) stream from HBM through a
-// ring of k-steps per wave that runs on across tiles; the published y_s / x_s
-// come from L2, one item ahead when its count is already full.
+// ring of k-steps per wave that runs on across tiles.  The published y_s / x_s
+// are kept in LDS with pairs (up to kSweepPairTiles tiles); with single waves
+// they go through R and come from L2, one item ahead when the count is full.
 // HBM traffic per sweep: the factors once, R and X; no launch per tile
 // column.  The first sweep (R = B, zero outside the last tile, so y_t = 0
 // for t < nt-1 under tile-local pivoting) runs only the last tile forward.
@@ -664,6 +665,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
                                                                double tol) {
   typedef float2 V;
   constexpr int NW = 4 / RB, NT = kSweepWaves / NW;  // waves of a team, teams
+  constexpr bool YL = NW > 1;                        // y_s / x_s in LDS
   // k-steps (4 columns of a 16 RB x 64 operand) in flight per wave
   constexpr int kSweepD = 16 / RB;
   const SolveDesc &d = descs[blockIdx.x];
@@ -674,6 +676,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   __shared__ V slot[NT][NW][kTile][17];  // a team's block, input of its diagonal step
   __shared__ int ready[kSweepMaxTiles], done[kSweepMaxTiles], arrived[NT];
   __shared__ int conv_flag;
+  __shared__ __align__(16) V ybuf[YL ? kSweepPairTiles : 1][kTile][16];
   for (int i = tid; i < kSweepMaxTiles; i += kSweepWaves * 64) {
     ready[i] = 0;
     done[i] = 0;
@@ -690,7 +693,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   const int loff = row0 + li + kTile * kq;
 
   f4 q1[RB], q2[RB], q3[RB];  // 3M sums of the wave's block: (16 rb + li, 4 kq + r)
-  V ycur[16], ynext[16];   // y_s / x_s operand: (4 kk + kq, li)
+  V ycur[16], ynext[16];   // y_s / x_s operand: (4 kk + kq, li); ynext not with ybuf
   int phase = 0;           // diagonal products of the team so far
 
   // ---- operand stream.  Items are the wave's rows of 64 x 64 column-major
@@ -721,41 +724,44 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     s = nt - 1;
     return t >= 0;
   };
+  // The ring holds the next kSweepD k-steps.  Every item is 16 of them, so a
+  // consumer's loads are the rest of its own item and the first of the next,
+  // at fixed offsets from the two bases (cb, nb) and without a branch; past
+  // the last item they read it again (never consumed), so that the wait
+  // counts stay static.
   V rg[kSweepD][RB];
-  const GCx<float> *cb = F;
-  int pt = 0, ps = 0, pk = 0;
+  const GCx<float> *cb = F, *nb = F;
+  int pt = 0, ps = 0;
   bool pok = false;
-  // load the cursor's k-step into a ring slot and advance; the loads are
-  // unconditional (an exhausted cursor re-reads its last k-step, never
-  // consumed) so that the wait counts stay static
-  auto load_slot = [&](bool fwd, int u) __attribute__((always_inline)) {
-    const GCx<float> *src = cb + kTile * 4 * pk + loff;
+  auto load_slot = [&](const GCx<float> *base, int k) __attribute__((always_inline)) {
+    const GCx<float> *src = base + kTile * 4 * k + loff;
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
       // the factor streams through once per sweep: non-temporal, so that the
       // published y_s / x_s blocks the waves read from L2 stay there
       typedef float sv2 __attribute__((ext_vector_type(2)));
       const sv2 v = __builtin_nontemporal_load((const sv2 *)(src + 16 * rb));
-      rg[u][rb] = make_float2(v.x, v.y);
-    }
-    if (pok && ++pk == 16) {
-      pok = next_item(fwd, pt, ps);
-      if (pok) {
-        pk = 0;
-        cb = item_base(fwd, pt, ps);
-      } else {
-        pk = 15;
-      }
+      rg[k % kSweepD][rb] = make_float2(v.x, v.y);
     }
   };
   auto prime = [&](bool fwd, int t0, int s0, bool ok) __attribute__((always_inline)) {
     pt = t0;
     ps = s0;
-    pk = 0;
     pok = ok;
     cb = ok ? item_base(fwd, t0, s0) : F;
 #pragma unroll
-    for (int u = 0; u < kSweepD; u++) load_slot(fwd, u);
+    for (int u = 0; u < kSweepD; u++) load_slot(cb, u);
+  };
+  auto begin_item = [&](bool fwd) __attribute__((always_inline)) {
+    pok = pok && next_item(fwd, pt, ps);
+    nb = pok ? item_base(fwd, pt, ps) : cb;
+  };
+  auto refill = [&](int kk) __attribute__((always_inline)) {
+    if (kk + kSweepD < 16) load_slot(cb, kk + kSweepD);
+    else load_slot(nb, kk + kSweepD - 16);
+    if (kk == 15) cb = nb;
+    // the loads stay here, kSweepD k-steps before their use
+    __builtin_amdgcn_sched_barrier(0);
   };
   // sums += operand * v, v in the MFMA's a-operand layout
   auto step = [&](int rb, V l, V v, float vs) __attribute__((always_inline)) {
@@ -764,6 +770,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     q3[rb] = mfma4(vs, l.x + l.y, q3[rb]);
   };
   auto consume_update = [&](bool fwd) __attribute__((always_inline)) {
+    begin_item(fwd);
 #pragma unroll
     for (int kk = 0; kk < 16; kk++) {
       const int u = kk % kSweepD;
@@ -771,7 +778,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
       const float ys = yv.x + yv.y;
 #pragma unroll
       for (int rb = 0; rb < RB; rb++) step(rb, rg[u][rb], yv, ys);
-      load_slot(fwd, u);
+      refill(kk);
     }
   };
   // block - sums of the updates (set by load_block) and plain sums
@@ -780,6 +787,17 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   };
   auto plus = [&](int rb, int r) __attribute__((always_inline)) {
     return make_float2(q1[rb][r] - q2[rb][r], q3[rb][r] - q1[rb][r] - q2[rb][r]);
+  };
+  // What is published: LDS alone (ybuf, the slots), whose fences leave the
+  // operand loads in flight, or y_s / x_s in R, whose release waits for all of
+  // the wave's memory operations.
+  auto release = [&]() __attribute__((always_inline)) {
+    if constexpr (YL) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  };
+  auto acquire = [&]() __attribute__((always_inline)) {
+    if constexpr (YL) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   };
   // Every wait ends (see above); the spin bound (about half a second) only
   // guards the GPU against a broken invariant: the solve then reports
@@ -793,13 +811,13 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
       }
       __builtin_amdgcn_s_sleep(1);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    acquire();
   };
   auto count_full = [&](int *count) __attribute__((always_inline)) {
     return __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= NW;
   };
   auto publish = [&](int *count) __attribute__((always_inline)) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    release();
     if (lane == 0)
       __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
@@ -807,6 +825,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   // unit lower L^-1; as stored for the upper U^-1, diagonal included): the
   // wave's half of In is already in the slot
   auto consume_diag = [&](bool fwd, bool upper, const int (&prow)[16]) __attribute__((always_inline)) {
+    begin_item(fwd);
     const V(*in_slot)[17] = slot[team][phase % NW];
     phase++;
     if (NW > 1) {
@@ -820,9 +839,11 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
       q3[rb] = q1[rb];
     }
 #pragma unroll
+    for (int kk = 0; kk < 16; kk++) ycur[kk] = in_slot[upper ? 4 * kk + kq : prow[kk]][li];
+#pragma unroll
     for (int kk = 0; kk < 16; kk++) {
       const int u = kk % kSweepD, k = 4 * kk + kq;
-      const V in = in_slot[upper ? k : prow[kk]][li];
+      const V in = ycur[kk];
       const float is = in.x + in.y;
 #pragma unroll
       for (int rb = 0; rb < RB; rb++) {
@@ -834,15 +855,18 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
         }
         step(rb, op, in, is);
       }
-      load_slot(fwd, u);
+      refill(kk);
     }
   };
-  auto load_block = [&](int t) __attribute__((always_inline)) {
+  auto load_block = [&](int t, bool fwd) __attribute__((always_inline)) {
 #pragma unroll
     for (int rb = 0; rb < RB; rb++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const V v = ldg<float>(R + (t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r));
+        // (the first sweep's y are zero but for the last tile)
+        const V v = YL && !fwd ? (FIRST ? make_float2(0.f, 0.f)
+                                        : ybuf[YL ? t : 0][row0 + 16 * rb + li][4 * kq + r])
+                               : ldg<float>(R + (t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r));
         q1[rb][r] = -v.x;
         q2[rb][r] = 0.f;
         q3[rb][r] = -v.x - v.y;
@@ -859,8 +883,10 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
 #pragma unroll
     for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-        R[(t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r)] = plus(rb, r);
+      for (int r = 0; r < 4; r++) {
+        if (YL) ybuf[YL ? t : 0][row0 + 16 * rb + li][4 * kq + r] = plus(rb, r);
+        else R[(t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r)] = plus(rb, r);
+      }
   };
   // X += the block of tile t; returns the sums over the last 16 rows (the
   // central rows Ns-16 .. Ns-1 for the last wave of the last tile's team)
@@ -891,6 +917,13 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     const int dir = fwd ? 1 : -1;
     bool have = false;
     for (int s = first; fwd ? s <= last : s >= last; s += dir) {
+      if (YL) {
+        wait_count(count + s, NW);
+#pragma unroll
+        for (int kk = 0; kk < 16; kk++) ycur[kk] = ybuf[YL ? s : 0][4 * kk + kq][li];
+        consume_update(fwd);
+        continue;
+      }
       if (!have) {
         wait_count(count + s, NW);
         load_y(s);
@@ -900,7 +933,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
       have = false;
       const int sn = s + dir;
       if ((fwd ? sn <= last : sn >= last) && count_full(count + sn)) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        acquire();
         load_y(sn);
         have = true;
       }
@@ -917,7 +950,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     prime(true, t0, FIRST ? tl : 0, mine);
     if (mine) {
       for (int t = t0; t < nt; t += NT) {
-        load_block(t);
+        load_block(t, true);
 #pragma unroll
         for (int kk = 0; kk < 16; kk++) prow[kk] = Perm[t * kTile + 4 * kk + kq];
         if (!FIRST && t > 0) run_updates(true, 0, t - 1, ready);
@@ -953,14 +986,14 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     const int t0 = team <= nt - 2 ? team + NT * ((nt - 2 - team) / NT) : -1;
     prime(false, t0 < 0 ? 0 : t0, tl, t0 >= 0);
     for (int t = t0; t >= 0; t -= NT) {
-      load_block(t);
+      load_block(t, false);
       run_updates(false, tl, t + 1, done);
       block_to_slot(minus);
       consume_diag(false, true, prow);
       store_block(t);
+      publish(done + t);  // the other tiles wait for it, not for X
       double dn = 0.0, xn = 0.0;
       add_to_x(t, dn, xn);
-      publish(done + t);
     }
   }
 }

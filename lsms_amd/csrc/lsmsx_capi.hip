@@ -617,12 +617,13 @@ int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int ma
   return 0;
 }
 
-// Whether the refinement sweeps take a tile row by a pair of waves: up to a
-// dozen tiles the chain of the diagonal tiles bounds a sweep (16 solves of four
-// tiles: 52.6 us a first sweep with single waves, 41.5 with pairs; 64 of ten
-// tiles: 154 and 125), beyond that HBM and the reads of y (96 solves of up to
-// 30 tiles: 682 and 812; 248 of 34: 1125 and 1161).
-inline bool sweep_pairs(int nt_max) { return nt_max <= 12; }
+// Whether the refinement sweeps take a tile row by a pair of waves, their y in
+// LDS: as far as those fit.  The chain of the diagonal tiles bounds such a
+// sweep (a first sweep of 16 solves of four tiles: 52.6 us with single waves,
+// 30 with pairs; 64 of ten tiles: 154 and 78).  Beyond it is HBM and the reads
+// of y, which pairs do twice (96 solves of up to 30 tiles: 682 with single
+// waves, 812 with pairs; 248 of 34: 1125 and 1161, all with y in R).
+inline bool sweep_pairs(int nt_max) { return nt_max <= kSweepPairTiles; }
 
 // Refinement of a chunk part on stream st with no host round trip (mixed
 // path, kc = 16, k_ir_sweep): max_sweeps sweeps are enqueued up front; the

@@ -21,6 +21,7 @@ constexpr int kIrFirstSweep = -1000;  // k_ir_step's step value for the first fo
 // and the largest number of 64-row tiles per solve it takes
 constexpr int kSweepWaves = 8;
 constexpr int kSweepMaxTiles = 128;
+constexpr int kSweepPairTiles = 11;  // tiles a sweep by pairs of waves takes (its y are in LDS)
 constexpr unsigned kSweepSpinLimit = 1u << 24;  // bound of one k_ir_sweep flag wait
 constexpr int kInfoSweepStall = -2;             // per-solve info when that bound is hit
 // per-solve info of a solve whose FP64 refinement did not converge: its

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("precision", [capi.PREC_MIXED_FP32, capi.PREC_MIXED_F16])
-@pytest.mark.parametrize("nsites", [1, 4, 5, 20, 47, 48, 49])
+@pytest.mark.parametrize("nsites", [1, 4, 5, 20, 43, 44, 45, 48, 49])
 def test_alone_and_beside_a_large_solve(precision, nsites):
     s = CF.config_c4()
     small, big = pick(s, 2)
