@@ -595,6 +595,8 @@ __global__ __launch_bounds__(256) void k_ir_accum(const SolveDesc *__restrict__ 
   if (tid == 0) {
     d.nrm[0] = red[0][0];
     d.nrm[1] = red[1][0];
+    d.nrm[2] = 0.0;
+    d.nrm[3] = 0.0;
   }
 }
 
@@ -626,7 +628,7 @@ __global__ void k_ir_decide(const SolveDesc *__restrict__ descs, int n, double t
   if (b >= n) return;
   const SolveDesc &d = descs[b];
   if (*d.conv) return;
-  ir_decide_one(d, d.nrm[0], d.nrm[1], tol);
+  ir_decide_one(d, d.nrm[0] + d.nrm[2], d.nrm[1] + d.nrm[3], tol);
 }
 
 // ---------------------------------------------------------------------------
@@ -634,6 +636,8 @@ __global__ void k_ir_decide(const SolveDesc *__restrict__ descs, int n, double t
 // FP32 factors, tile-major): dX = (P^T L U)^-1 R, the convergence test on the
 // central rows between the forward and the backward halves, and X += dX.  It
 // does the work of k_ir_step, k_ir_accum and k_ir_decide for one sweep.
+// With kc = 32 a workgroup takes 16 of the columns, and the halves are
+// launches of their own (kSweepFwd, kSweepBwd) with k_ir_decide between them.
 //
 // Left-looking by tile row, with the tile rows dealt round-robin to teams of
 // NW = 4/RB waves (one wave, or a pair): team p of n takes t = p, p+n, ...
@@ -646,8 +650,8 @@ __global__ void k_ir_decide(const SolveDesc *__restrict__ descs, int n, double t
 // waits only for tiles below its own (above, backward) and, before the
 // diagonal product, for its partner at the same tile, and takes its tiles in
 // order, so the waits always end.  The diagonal-tile inverse is applied as one
-// more operand, its input staged in the team's LDS slot (a pair has two in
-// turn: a wave writes one while its partner may still read the other).
+// more operand, its input staged in the team's LDS slot (a wave of a pair
+// writes it once its partner has read the last one).
 // All operand tiles (L_ts, U_ts, the inverses) stream from HBM through a
 // ring of k-steps per wave that runs on across tiles.  The published y_s / x_s
 // are kept in LDS with pairs (up to kSweepPairTiles tiles); with single waves
@@ -660,7 +664,7 @@ __global__ void k_ir_decide(const SolveDesc *__restrict__ descs, int n, double t
 // is HBM or a compute unit's MFMAs, and single waves read y half as often
 // (sweep_pairs has both sides).  The arithmetic of both is the same.
 
-template <bool FIRST, int RB>
+template <bool FIRST, int RB, SweepPart PART>
 __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *__restrict__ descs,
                                                                double tol) {
   typedef float2 V;
@@ -673,18 +677,24 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   const int nt = d.nt, Ns = d.Ns;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), team = w / NW, half = w % NW;
-  __shared__ V slot[NT][NW][kTile][17];  // a team's block, input of its diagonal step
-  __shared__ int ready[kSweepMaxTiles], done[kSweepMaxTiles], arrived[NT];
+  __shared__ V slot[NT][kTile][17];  // a team's block, input of its diagonal step
+  __shared__ int ready[kSweepMaxTiles], done[kSweepMaxTiles], arrived[NT], taken[NT];
   __shared__ int conv_flag;
   __shared__ __align__(16) V ybuf[YL ? kSweepPairTiles : 1][kTile][16];
   for (int i = tid; i < kSweepMaxTiles; i += kSweepWaves * 64) {
     ready[i] = 0;
     done[i] = 0;
-    if (i < NT) arrived[i] = 0;
+    if (i < NT) {
+      arrived[i] = 0;
+      taken[i] = 0;
+    }
   }
   __syncthreads();
-  GCx<float> *R = (GCx<float> *)d.R;
-  gd2 *X = (gd2 *)d.X;
+  // kSweepFwd, kSweepBwd: the workgroup's 16 columns of 32
+  const long c0 = PART == kSweepAll ? 0 : (long)Ns * (16 * blockIdx.y);
+  const int central = kTile - d.kc;  // first central row in the last tile
+  GCx<float> *R = (GCx<float> *)d.R + c0;
+  gd2 *X = (gd2 *)d.X + c0;
   const GCx<float> *__restrict__ F = (const GCx<float> *)d.A;  // tile-major factors
   const GCx<float> *__restrict__ Inv = (const GCx<float> *)d.inv;
   const LSMSX_GLOBAL int *Perm = (const LSMSX_GLOBAL int *)d.perm;
@@ -826,7 +836,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   // wave's half of In is already in the slot
   auto consume_diag = [&](bool fwd, bool upper, const int (&prow)[16]) __attribute__((always_inline)) {
     begin_item(fwd);
-    const V(*in_slot)[17] = slot[team][phase % NW];
+    const V(*in_slot)[17] = slot[team];
     phase++;
     if (NW > 1) {
       publish(arrived + team);
@@ -840,6 +850,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     }
 #pragma unroll
     for (int kk = 0; kk < 16; kk++) ycur[kk] = in_slot[upper ? 4 * kk + kq : prow[kk]][li];
+    if (NW > 1) publish(taken + team);
 #pragma unroll
     for (int kk = 0; kk < 16; kk++) {
       const int u = kk % kSweepD, k = 4 * kk + kq;
@@ -864,7 +875,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         // (the first sweep's y are zero but for the last tile)
-        const V v = YL && !fwd ? (FIRST ? make_float2(0.f, 0.f)
+        const V v = YL && !fwd && PART == kSweepAll ? (FIRST ? make_float2(0.f, 0.f)
                                         : ybuf[YL ? t : 0][row0 + 16 * rb + li][4 * kq + r])
                                : ldg<float>(R + (t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r));
         q1[rb][r] = -v.x;
@@ -873,7 +884,8 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
       }
   };
   auto block_to_slot = [&](auto value) __attribute__((always_inline)) {
-    V(*out)[17] = slot[team][phase % NW];
+    V(*out)[17] = slot[team];
+    if (NW > 1) wait_count(taken + team, NW * phase);  // the partner has read the last block
 #pragma unroll
     for (int rb = 0; rb < RB; rb++)
 #pragma unroll
@@ -885,11 +897,12 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         if (YL) ybuf[YL ? t : 0][row0 + 16 * rb + li][4 * kq + r] = plus(rb, r);
-        else R[(t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r)] = plus(rb, r);
+        if (!YL || PART == kSweepFwd)
+          R[(t * kTile + row0 + 16 * rb + li) + (long)Ns * (4 * kq + r)] = plus(rb, r);
       }
   };
-  // X += the block of tile t; returns the sums over the last 16 rows (the
-  // central rows Ns-16 .. Ns-1 for the last wave of the last tile's team)
+  // X += the block of tile t; returns the sums over the rows that are central
+  // if t is the last tile (all of them in the last wave of a team)
   auto add_to_x = [&](int t, double &dn, double &xn) __attribute__((always_inline)) {
 #pragma unroll
     for (int rb = 0; rb < RB; rb++)
@@ -901,7 +914,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
         x.x += dx.x;
         x.y += dx.y;
         X[idx] = x;
-        if (rb == RB - 1) {
+        if (row0 + 16 * rb >= central) {
           dn += (double)dx.x * dx.x + (double)dx.y * dx.y;
           xn += x.x * x.x + x.y * x.y;
         }
@@ -941,10 +954,10 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     }
   };
 
-  // ---- forward half
   const int tl = nt - 1, pl = tl % NT;
   int prow[16] = {};
-  {
+  // ---- forward half
+  if constexpr (PART != kSweepBwd) {
     const int t0 = FIRST ? tl : team;
     const bool mine = FIRST ? team == pl : team < nt;
     prime(true, t0, FIRST ? tl : 0, mine);
@@ -967,8 +980,13 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
             xn += __shfl_xor(xn, off, 64);
           }
           if (half == NW - 1 && lane == 0) {
-            ir_decide_one(d, dn, xn, tol);
-            conv_flag = *d.conv;
+            if constexpr (PART == kSweepFwd) {  // k_ir_decide adds up the column halves
+              d.nrm[2 * blockIdx.y] = dn;
+              d.nrm[2 * blockIdx.y + 1] = xn;
+            } else {
+              ir_decide_one(d, dn, xn, tol);
+              conv_flag = *d.conv;
+            }
           }
           publish(done + t);
         } else {
@@ -978,8 +996,15 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
       }
     }
   }
+  if constexpr (PART == kSweepFwd) return;
+  if constexpr (PART == kSweepBwd) {
+    if (YL)  // the last tile's x
+      for (int e = tid; e < 16 * kTile; e += kSweepWaves * 64)
+        ybuf[YL ? tl : 0][e & 63][e >> 6] = ldg<float>(R + (tl * kTile + (e & 63)) + (long)Ns * (e >> 6));
+    if (tid == 0) done[tl] = NW;
+  }
   __syncthreads();
-  if (conv_flag) return;
+  if (PART == kSweepAll && conv_flag) return;
 
   // ---- backward half: this team's tiles below the last, descending
   {
@@ -1046,9 +1071,12 @@ template __global__ void k_ir_step<double, true>(const SolveDesc *, int);
 template __global__ void k_ir_step<double, false>(const SolveDesc *, int);
 template __global__ void k_ir_accum<float>(const SolveDesc *, int);
 template __global__ void k_ir_accum<double>(const SolveDesc *, int);
-template __global__ void k_ir_sweep<true, 2>(const SolveDesc *, double);
-template __global__ void k_ir_sweep<true, 4>(const SolveDesc *, double);
-template __global__ void k_ir_sweep<false, 2>(const SolveDesc *, double);
-template __global__ void k_ir_sweep<false, 4>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<true, 2, kSweepAll>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<true, 4, kSweepAll>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<false, 2, kSweepAll>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<false, 4, kSweepAll>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<true, 2, kSweepFwd>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<false, 2, kSweepFwd>(const SolveDesc *, double);
+template __global__ void k_ir_sweep<false, 2, kSweepBwd>(const SolveDesc *, double);
 
 }  // namespace lsmsx

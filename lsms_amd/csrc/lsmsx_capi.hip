@@ -56,7 +56,7 @@ __global__ void k_ir_step(const SolveDesc *, int);
 template <class T>
 __global__ void k_ir_accum(const SolveDesc *, int);
 __global__ void k_ir_decide(const SolveDesc *, int, double);
-template <bool FIRST, int RB>
+template <bool FIRST, int RB, SweepPart PART>
 __global__ void k_ir_sweep(const SolveDesc *, double);
 __global__ void k_ir_residual_g(const SolveDesc *);
 __global__ void k_ir_residual_g_finish(const SolveDesc *);
@@ -561,9 +561,20 @@ int launch_lu(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool split_
   return check_launch("k_lu_last");
 }
 
-// Refinement sweeps, one launch per tile column (k_ir_step), on a chunk whose
-// factors (T = float: mixed path with 32 right-hand sides; T = double:
-// FP64-refined path) are in place.  Returns the number of
+// Whether the refinement sweeps take a tile row by a pair of waves, their y in
+// LDS: as far as those fit.  The chain of the diagonal tiles bounds such a
+// sweep (a first sweep of 16 solves of four tiles: 52.6 us with single waves,
+// 30 with pairs; 64 of ten tiles: 154 and 78).  Beyond it is HBM and the reads
+// of y, which pairs do twice (96 solves of up to 30 tiles: 682 with single
+// waves, 812 with pairs; 248 of 34: 1125 and 1161, all with y in R).
+inline bool sweep_pairs(int nt_max) { return nt_max <= kSweepPairTiles; }
+
+// Refinement sweeps on a chunk whose factors (T = float: mixed path with 32
+// right-hand sides; T = double: FP64-refined path) are in place: one launch
+// per tile column (k_ir_step), or, for FP32 factors as far as a pair of waves
+// takes them (sweep_pairs), one per half sweep: a k_ir_step launch is 10 to 14
+// us long whatever its size, and the sweeps of 32 solves of 14 tiles took 1.19
+// ms, so 0.79.  Returns the number of
 // unconverged solves left in *left.
 template <class T>
 int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int max_sweeps,
@@ -580,7 +591,14 @@ int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int ma
         hipLaunchKernelGGL((k_ir_residual<T, 1>), dim3(nt_max, nb), dim3(256), 0, c->stream, dd);
     }
     if (int r = check_launch("k_ir_residual")) return r;
-    {
+    if (sizeof(T) == 4 && kc == 32 && sweep_pairs(nt_max)) {
+      ProfScope p(c, 6);
+      const dim3 grid(nb, 2), block(kSweepWaves * 64);
+      const auto fwd = it == 0 ? k_ir_sweep<true, 2, kSweepFwd> : k_ir_sweep<false, 2, kSweepFwd>;
+      hipLaunchKernelGGL(fwd, grid, block, 0, c->stream, dd, tol);
+      hipLaunchKernelGGL(k_ir_decide, dim3((nb + 255) / 256), dim3(256), 0, c->stream, dd, nb, tol);
+      hipLaunchKernelGGL((k_ir_sweep<false, 2, kSweepBwd>), grid, block, 0, c->stream, dd, tol);
+    } else {
       ProfScope p(c, 6);
       if (it == 0) {  // R = B: only the last tile of each solve (kIrFirstSweep)
         hipLaunchKernelGGL((k_ir_step<T, true>), dim3(1, nb), dim3(256), 0, c->stream, dd,
@@ -617,14 +635,6 @@ int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int ma
   return 0;
 }
 
-// Whether the refinement sweeps take a tile row by a pair of waves, their y in
-// LDS: as far as those fit.  The chain of the diagonal tiles bounds such a
-// sweep (a first sweep of 16 solves of four tiles: 52.6 us with single waves,
-// 30 with pairs; 64 of ten tiles: 154 and 78).  Beyond it is HBM and the reads
-// of y, which pairs do twice (96 solves of up to 30 tiles: 682 with single
-// waves, 812 with pairs; 248 of 34: 1125 and 1161, all with y in R).
-inline bool sweep_pairs(int nt_max) { return nt_max <= kSweepPairTiles; }
-
 // Refinement of a chunk part on stream st with no host round trip (mixed
 // path, kc = 16, k_ir_sweep): max_sweeps sweeps are enqueued up front; the
 // residual and sweep kernels return at once for solves already converged,
@@ -645,8 +655,8 @@ int refine_async(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int max_
     }
     ProfScope p(c, 6);
     const auto sweep = sweep_pairs(nt_max)
-                           ? (it == 0 ? k_ir_sweep<true, 2> : k_ir_sweep<false, 2>)
-                           : (it == 0 ? k_ir_sweep<true, 4> : k_ir_sweep<false, 4>);
+                           ? (it == 0 ? k_ir_sweep<true, 2, kSweepAll> : k_ir_sweep<false, 2, kSweepAll>)
+                           : (it == 0 ? k_ir_sweep<true, 4, kSweepAll> : k_ir_sweep<false, 4, kSweepAll>);
     hipLaunchKernelGGL(sweep, dim3(nb), dim3(kSweepWaves * 64), 0, st, dd, tol);
   }
   hipLaunchKernelGGL(k_ir_extract, dim3(nb), dim3(256), 0, st, dd);
@@ -837,7 +847,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
       if (int r = c->X.ensure(xtot)) return r;
       if (int r = c->conv.ensure((size_t)nb)) return r;
       if (int r = c->iters.ensure((size_t)nb)) return r;
-      if (int r = c->dxn.ensure((size_t)4 * nb)) return r;
+      if (int r = c->dxn.ensure((size_t)6 * nb)) return r;
       if (int r = c->count.ensure(1)) return r;
     }
     if (split) {
@@ -907,7 +917,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
         d.iters = c->iters.p + b;
         d.dxn = c->dxn.p + b;
         d.dxn_rho2 = c->dxn.p + nb + b;
-        d.nrm = c->dxn.p + 2 * nb + 2 * b;
+        d.nrm = c->dxn.p + 2 * nb + 4 * b;
       }
       if (mixed) {
         d.A = c->W.p + moff;

@@ -17,11 +17,12 @@ constexpr int kMaxKkr = (kMaxLmax + 1) * (kMaxLmax + 1);
 constexpr int kPlaneHalves = 4 * kTile * kTile;  // one tile's four FP16 planes
 constexpr int kLastStep = -1001;  // k_lu_diag's step value for each solve's last tile
 constexpr int kIrFirstSweep = -1000;  // k_ir_step's step value for the first forward sweep
-// k_ir_sweep (one launch per refinement sweep, kc = 16): waves per workgroup
+// k_ir_sweep (refinement sweeps): waves per workgroup
 // and the largest number of 64-row tiles per solve it takes
 constexpr int kSweepWaves = 8;
 constexpr int kSweepMaxTiles = 128;
-constexpr int kSweepPairTiles = 11;  // tiles a sweep by pairs of waves takes (its y are in LDS)
+constexpr int kSweepPairTiles = 15;  // tiles a sweep by pairs of waves takes (its y are in LDS)
+enum SweepPart { kSweepAll, kSweepFwd, kSweepBwd };
 constexpr unsigned kSweepSpinLimit = 1u << 24;  // bound of one k_ir_sweep flag wait
 constexpr int kInfoSweepStall = -2;             // per-solve info when that bound is hit
 // per-solve info of a solve whose FP64 refinement did not converge: its
@@ -77,7 +78,7 @@ struct SolveDesc {
   int *iters;             // refinement sweeps used
   double *dxn;            // ||dX_c||^2 of the previous sweep
   double *dxn_rho2;       // the contraction (||dX_c|| ratio)^2 observed at the previous sweep
-  double *nrm;            // ||dX_c||^2, ||X_c||^2 of the current sweep
+  double *nrm;            // ||dX_c||^2, ||X_c||^2 of the current sweep, of two column halves
   // split-FP16 trailing updates (mixed path): the FP32 panels of the steps
   // of a group as hi/lo FP16 planes with one power-of-2 scale per tile
   void *hp;               // (step % group) x (L, U) x nt tiles x 4 planes x 64 x 64 halves
