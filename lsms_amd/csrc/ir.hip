@@ -841,6 +841,8 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
     if (NW > 1) {
       publish(arrived + team);
       wait_count(arrived + team, NW * phase);
+    } else {
+      wave_lds_fence();
     }
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {

@@ -191,7 +191,7 @@ __device__ __forceinline__ void wave_gemm3m(FA fa, FB fb, int nk, Acc3<T, N> &q)
   for (int i = 0; i <= PF; i++) step(i);
 }
 
-// The same in FP64 for operands in global memory, nk a multiple of 8: A(i, k)
+// The same in FP64 for operands in global memory, nk a multiple of 4: A(i, k)
 // at A[i + ld k], B(k, j) at B[k + ld j], both wave-uniform.  An FP64 MFMA
 // holds its SIMD's VALU for all of its 64 cycles, whichever wave the VALU work
 // is of, so every other instruction of the loop adds to its time: the
@@ -199,9 +199,8 @@ __device__ __forceinline__ void wave_gemm3m(FA fa, FB fb, int nk, Acc3<T, N> &q)
 // work left of a step are the sums of the 3M form (through pointers, with A
 // negated, it was 17 instructions; 64 solves of N = 2160: trailing updates
 // 23.8 -> 22.4 ms at K = 128).
-template <int N>
 __device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<double> *B, long ld,
-                                              int nk, Acc3<double, N> &q) {
+                                              int nk, Acc3<double, 2> &q) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef unsigned b128 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
@@ -209,11 +208,11 @@ __device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<do
   const auto ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, kRange, kFlags);
   const auto rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, kRange, kFlags);
   const int ld16 = (int)ld * 16;
+  constexpr int N = 2, PF = 3;
   const int va = 16 * li + ld16 * kq;  // A(li, kq)
   int vb[N];                           // B(kq, 16 t + li)
 #pragma unroll
   for (int t = 0; t < N; t++) vb[t] = 16 * kq + ld16 * (16 * t + li);
-  constexpr int PF = N == 2 ? 3 : 7;
   double2 a[PF + 1][N], b[PF + 1][N];
   auto get = [](b128 x) __attribute__((always_inline)) {
     return double2{__hiloint2double(x[1], x[0]), __hiloint2double(x[3], x[2])};
@@ -253,13 +252,101 @@ __device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<do
 #endif
 }
 
+// Wave-scope ordering of LDS traffic: what any lane has written before is there
+// for the others' reads after, and what they read before is not overwritten.
+// (The hardware keeps a wave's LDS operations in order; without the fence the
+// compiler may still move a lane's read over its own write elsewhere.)
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// LDS of one wave for the operand B of wave_gemm3m_staged: two chunks of 16 k.
+struct BStage {
+  __align__(16) double2 b[2][16][17];  // [chunk][column][k]
+};
+
+// The same for a 16 x 16 block, nk a multiple of 8; `st` is the wave's own
+// LDS.  A's rows are contiguous over the lanes; B's are not (a lane's column,
+// four k over the lane groups), and read straight into that layout every lane
+// is an L1 access of its own, 64 a load.  A 16 x 16 block has a load of each a
+// k-step of 192 MFMA cycles, and L1 was busy 82% of the time (the MFMAs 40%)
+// in the inverse of eight solves of N = 944.  So B is read 16 k by 4 columns a
+// load, 16 accesses, and turned in LDS: 1.06 -> 0.87 ms there.  A 32 x 32
+// block, with half the loads to an MFMA, gains nothing (64 solves of N = 2160:
+// trailing updates 18.4 ms either way, six of N = 4384 16.2 and 16.5), and
+// neither do loads further ahead.
+__device__ __forceinline__ void wave_gemm3m_staged(const GCx<double> *A, const GCx<double> *B,
+                                                   long ld, int nk, Acc3<double, 1> &q,
+                                                   BStage &st) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef unsigned b128 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
+  constexpr int kRange = 0x7fffffff, kFlags = 0x00027000;  // raw buffer, byte offsets
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, kRange, kFlags);
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, kRange, kFlags);
+  const int ld16 = (int)ld * 16;
+  const int v0 = 16 * li + ld16 * kq;  // A(li, kq); B(li, kq): 16 k, columns kq + 4 m
+  double2 a[8], b[4];
+  auto get = [](b128 x) __attribute__((always_inline)) {
+    return double2{__hiloint2double(x[1], x[0]), __hiloint2double(x[3], x[2])};
+  };
+  auto load_a = [&](int slot, int ks) __attribute__((always_inline)) {
+    a[slot] = get(__builtin_amdgcn_raw_buffer_load_b128(ra, v0, 4 * ks * ld16, 0));
+  };
+  auto load_b = [&](int c) __attribute__((always_inline)) {  // chunk c: k-steps 4c .. 4c+3
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+      b[m] = get(__builtin_amdgcn_raw_buffer_load_b128(rb, v0, 256 * c + 4 * m * ld16, 0));
+  };
+  auto put_b = [&](int buf) __attribute__((always_inline)) {
+    wave_lds_fence();
+#pragma unroll
+    for (int m = 0; m < 4; m++) st.b[buf][kq + 4 * m][li] = b[m];
+    wave_lds_fence();
+  };
+  // chunk c from LDS buffer `buf` (c mod 2); the A k-steps 4c+4 .. 4c+7 are
+  // loaded on the way when `next`
+  auto chunk = [&](int c, int buf, bool next) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (next) load_a((4 * buf + u + 4) & 7, 4 * c + u + 4);
+      double2 av[1] = {a[4 * buf + u]}, bv[1] = {st.b[buf][li][4 * u + kq]};
+      gemm3m_step<double, 1>(av, bv, q);
+    }
+  };
+  const int nc = nk / 4;
+  load_b(0);
+#pragma unroll
+  for (int i = 0; i < 4; i++) load_a(i, i);
+  put_b(0);
+  load_b(1);
+  int c = 0;
+#pragma unroll 1
+  for (; c < nc - 2; c += 2) {
+    put_b(1);
+    load_b(c + 2);
+    chunk(c, 0, true);
+    put_b(0);
+    load_b(c + 3);
+    chunk(c + 1, 1, true);
+  }
+  put_b(1);
+  chunk(c, 0, true);
+  chunk(c + 1, 1, false);
+#endif
+}
+
 // q += sum_{u < ns} A_u B_u over 64-wide tiles: A_u = A + u sa, B_u = B + u sb
 // (FP64: consecutive in k, so that ns tiles are one product).
 template <class T, int N>
 __device__ __forceinline__ void tile_products(const GCx<T> *A, long sa, const GCx<T> *B, long sb,
-                                              long ld, int ns, Acc3<T, N> &q) {
-  if constexpr (sizeof(T) == 8) {
-    if (ns > 0) wave_gemm3m_k<N>(A, B, ld, 16 * ns, q);
+                                              long ld, int ns, Acc3<T, N> &q, BStage *st) {
+  if constexpr (sizeof(T) == 8 && N == 1) {
+    if (ns > 0) wave_gemm3m_staged(A, B, ld, 16 * ns, q, st[threadIdx.x >> 6]);
+  } else if constexpr (sizeof(T) == 8) {
+    if (ns > 0) wave_gemm3m_k(A, B, ld, 16 * ns, q);
   } else {
     for (int u = 0; u < ns; u++, A += sa, B += sb)
       wave_gemm3m<T, N, N == 2 ? 3 : 7>([&](int i, int k) { return ldg<T>(A + (i + ld * k)); },
@@ -314,8 +401,12 @@ enum PanelOp {
 // LDS of panel_op: C' (a tile, or 16 rows or columns of one) and the pivots.
 template <class T, int N>
 struct PanelLds {
-  __align__(16) CxT<T> c[kTile * ((N == 2 ? kTile : 16) + 1)];
+  union {
+    __align__(16) CxT<T> c[kTile * ((N == 2 ? kTile : 16) + 1)];
+    BStage st[sizeof(T) == 8 && N == 1 ? 4 : 1];  // before that: B of the earlier steps
+  };
   int rowpos[kTile];
+  __device__ PanelLds() {}
 };
 
 // One panel tile or a piece of it by a 256-thread workgroup:
@@ -362,8 +453,9 @@ __device__ __forceinline__ void panel_op(GCx<T> *__restrict__ C, bool load_c, bo
         else if (identity) c.x = r0 + wr + i == c0 + wc + j ? T(1) : T(0);
         set_minus<T, N>(q, bj, bi, r, c.x, c.y);
       }
-  tile_products<T, N>(A + (r0 + wr), sa, B + ld * (c0 + wc), sb, ld, ns, q);
-  if (OP == kLeftL) __syncthreads();  // rowpos
+  tile_products<T, N>(A + (r0 + wr), sa, B + ld * (c0 + wc), sb, ld, ns, q, lds.st);
+  // rowpos is there, the staged operands are read
+  if (OP == kLeftL || (sizeof(T) == 8 && N == 1)) __syncthreads();
 #pragma unroll
   for (int bj = 0; bj < N; bj++)
 #pragma unroll
