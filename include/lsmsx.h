@@ -263,7 +263,8 @@ int lsmsx_tau00_adjoint(lsmsx_ctx *ctx, int nsolve, const int *atom_ids,
  *                            updates, the panels with their fused cross
  *                            updates) are remapped so that each of the 8 XCDs
  *                            works on whole solves and reads their panels
- *                            into its own L2;
+ *                            into its own L2 (split-FP16 batches of one size
+ *                            always are);
  *   LSMSX_SCHED_TWO_STREAMS  the two halves of a chunk run on two streams (of
  *                            default priority), so one half's diagonal-tile
  *                            and panel steps overlap the other's updates.
