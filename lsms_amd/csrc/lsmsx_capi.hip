@@ -102,7 +102,7 @@ __global__ void k_interstitial(int, int, const double2 *, const double2 *, const
 __global__ void k_rel_tstore(double2 *, long, long, int, const double *, const double2 *);
 __global__ void k_rel_tau(double2 *, int, const double *, const double2 *);
 __global__ void k_rel_blocks(double2 *, long, int, const double *);
-__global__ void k_lu_cross_diag_h(const SolveDesc *, int, int);
+__global__ void k_lu_diag_h(const SolveDesc *, int, int);
 __global__ void k_lu_panel_h(const SolveDesc *, int, int, int, int);
 __global__ void k_lu_strip_h(const SolveDesc *, int);
 
@@ -508,17 +508,17 @@ int launch_lu_steps(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool 
     const bool strips = split_f16 && 2L * nrest * nb >= 4864;
     for (int t = s; t <= b; t++) {
       const int u = t - s, np = 2 * (nt_max - 1 - t);
-      if (u > 0) {
+      if (u > 0 && !split_f16) {
         ProfScope p(c, 9);
-        if (split_f16)
-          hipLaunchKernelGGL(k_lu_cross_diag_h, dim3(nb), dim3(128), 0, st, dd, s, u);
-        else
-          hipLaunchKernelGGL(k_lu_cross_diag<T>, dim3(4, nb), dim3(256), 0, st, dd, s, u);
+        hipLaunchKernelGGL(k_lu_cross_diag<T>, dim3(4, nb), dim3(256), 0, st, dd, s, u);
       }
       if (int r = check_launch("k_lu_cross_diag")) return r;
       {
         ProfScope p(c, 1);
-        hipLaunchKernelGGL(k_lu_diag<T>, dim3(nb), dim3(256), 0, st, dd, t);
+        if (u > 0 && split_f16)
+          hipLaunchKernelGGL(k_lu_diag_h, dim3(nb), dim3(256), 0, st, dd, t, u);
+        else
+          hipLaunchKernelGGL(k_lu_diag<T>, dim3(nb), dim3(256), 0, st, dd, t);
       }
       {
         ProfScope p(c, 2);

@@ -16,8 +16,8 @@
 // panel tiles (inside k_lu_panel) of a step first take the earlier steps of
 // its group, and one trailing update per group, A_ij -= sum_k L_ik U_kj
 // (k_lu_trail, MFMA, dominant), reads and writes the rest of the matrix once.
-// The split-FP16 path has its own k_lu_panel_h, and k_lu_trail_h and
-// k_lu_cross_diag_h in update_f16.hip.  k_lu_last then factors the last tile
+// The split-FP16 path has its own k_lu_diag_h, k_lu_panel_h and k_lu_strip_h,
+// and k_lu_trail_h in update_f16.hip.  k_lu_last then factors the last tile
 // with the pivots of its non-central
 // rows and of the central rows kept apart.  In FP64 it also solves
 // S tau00 = t0 with the Schur complement S (the plain path); in FP32 it
@@ -332,6 +332,25 @@ __device__ __forceinline__ void cross_to_lds(const SolveDesc &d, int ti, int tj,
         Ts[col][rowpos ? rowpos[row] : row] =
             make_float2(av[bi][bj][r].x + cr[bi][bj][r] * sc2, av[bi][bj][r].y + ci[bi][bj][r] * sc2);
       }
+}
+
+// Diagonal tile of step s on the split-FP16 path, after its cross update with
+// the ncross (> 0) steps before s in its group, on the way into the
+// factorization: a few microseconds of FP16 MFMAs, where a launch of its own
+// took 14 (32 solves) to 21 (248).
+__global__ __launch_bounds__(256) void k_lu_diag_h(const SolveDesc *__restrict__ descs, int step,
+                                                   int ncross) {
+  const SolveDesc &d = descs[blockIdx.x];
+  const int s = step - d.step0;
+  if (s - ncross < 0 || s >= d.nt - 1) return;
+  if (d.conv && *d.conv) return;
+  __shared__ TileLds<float> t;
+  __shared__ __align__(16) float2 Ts[kTile][kTile + 1];
+  cross_to_lds(d, s, s, s - ncross, ncross, tile_ptr<float>(d, s, s), tile_ld(d), Ts, nullptr);
+  __syncthreads();
+  tile_lu<float>(t, [&](int r, int c) { return Ts[c][r]; }, kTile, s * kTile);
+  tile_invert_upper<float>(t);
+  store_tile<float>(t, d, s);
 }
 
 // Panel tile t of step s on the split-FP16 path: lower -> L_ts = A_ts U^-1 ;

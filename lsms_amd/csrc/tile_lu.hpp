@@ -300,16 +300,15 @@ __device__ __forceinline__ void tile_invert_upper(TileLds<T> &t) {
   __syncthreads();
 }
 
-// Factor the tile at src (column stride ld), P A = L U: on return t holds L^-1
+// Factor the tile load(row, column), P A = L U: on return t holds L^-1
 // below the diagonal (which is 1) and U on and above it, dinv the reciprocals of
 // U's diagonal, prow the permutation (row r of P A is row prow[r] of A).  info:
 // col_base + the first column with a zero pivot (1-based), or 0; minpiv: the
 // smallest |pivot|.  The pivots of columns below nd come from the rows below nd,
 // so the rows from nd on (the central site of the last tile) never pivot into
 // the rest.  256 threads; ends with a barrier.
-template <class T>
-__device__ __forceinline__ void tile_lu(TileLds<T> &t, const GCx<T> *src, long ld, int nd,
-                                        int col_base) {
+template <class T, class LD>
+__device__ __forceinline__ void tile_lu(TileLds<T> &t, LD load, int nd, int col_base) {
   typedef CxT<T> V;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -317,7 +316,7 @@ __device__ __forceinline__ void tile_lu(TileLds<T> &t, const GCx<T> *src, long l
     T re[kTile / 4], im[kTile / 4];  // (an array of structs would go to scratch)
 #pragma unroll
     for (int q = 0; q < kTile / 4; q++) {
-      const V x = ldg<T>(src + lane + ld * (w + 4 * q));
+      const V x = load(lane, w + 4 * q);
       re[q] = x.x;
       im[q] = x.y;
     }
@@ -455,6 +454,13 @@ __device__ __forceinline__ void tile_lu(TileLds<T> &t, const GCx<T> *src, long l
     }
   }
   __syncthreads();
+}
+
+// The same for the tile at src, column stride ld.
+template <class T>
+__device__ __forceinline__ void tile_lu(TileLds<T> &t, const GCx<T> *src, long ld, int nd,
+                                        int col_base) {
+  tile_lu<T>(t, [=](int r, int c) { return ldg<T>(src + r + ld * c); }, nd, col_base);
 }
 
 }  // namespace lsmsx

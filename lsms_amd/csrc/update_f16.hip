@@ -310,20 +310,4 @@ __global__ __launch_bounds__(512) void k_lu_trail_h(const SolveDesc *__restrict_
                  min(2, nrest - 2 * sc), g0, ns, Ls, Us);
 }
 
-// Cross update of the diagonal tile of step t = g + u of the group starting
-// at global step `step` (g local), before the tile is factored: the steps
-// g .. t-1 on their split planes, one 64 x 64 region of 128 threads per
-// solve.  The other tiles of column and row t take the same update inside
-// the fused panel (k_lu_panel_h).
-__global__ __launch_bounds__(128) void k_lu_cross_diag_h(const SolveDesc *__restrict__ descs,
-                                                         int step, int u) {
-  __shared__ h8 Ls[1][1][4][kTile][4];
-  __shared__ h8 Us[1][1][4][kTile][4];
-  const SolveDesc &d = descs[blockIdx.x];
-  const int g0 = step - d.step0, t = g0 + u;
-  if (g0 < 0 || u <= 0 || t > d.nt - 2) return;
-  if (d.conv && *d.conv) return;
-  region_h<1, 1, 1>(d, t, 1, t, 1, g0, u, Ls, Us);
-}
-
 }  // namespace lsmsx
