@@ -338,21 +338,116 @@ __device__ __forceinline__ void wave_gemm3m_staged(const GCx<double> *A, const G
 #endif
 }
 
+// LDS of one wave for the operand B of tile_products_f32: two chunks of 16 k.
+template <int N>
+struct BStage32 {
+  __align__(16) float2 b[2][16 * N][18];  // [chunk][column][k]
+};
+
+// The FP32 form: q += sum_{u < ns} A_u B_u over 64-wide tiles, A_u = A + u sa,
+// B_u = B + u sb, wave-uniform.  Here B read in the MFMA's layout is 128 L1
+// accesses a k-step (one per lane and column block) of 432 MFMA cycles, for
+// each of four waves: L1 was the bound.  Read 16 k by 8 columns a load and
+// turned in LDS it is 16 (64 solves of ten tiles: panels and trailing updates
+// 660 -> 495 us).
+template <int N>
+__device__ __forceinline__ void tile_products_f32(const GCx<float> *A, long sa,
+                                                  const GCx<float> *B, long sb, long ld, int ns,
+                                                  Acc3<float, N> &q, BStage32<N> &st) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef unsigned b64 __attribute__((ext_vector_type(2)));
+  typedef unsigned b128 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
+  constexpr int kRange = 0x7fffffff, kFlags = 0x00027000;  // raw buffer, byte offsets
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, kRange, kFlags);
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, kRange, kFlags);
+  const int ld8 = (int)ld * 8, sa8 = (int)sa * 8, sb8 = (int)sb * 8;
+  const int va = 8 * li + ld8 * kq;                     // A(li, kq)
+  const int bk = 2 * (lane & 7), bc = lane >> 3;        // B(bk, bc): 16 k, columns bc + 8 m
+  const int vb = 8 * bk + ld8 * bc;
+  constexpr int NB = 2 * N;
+  float2 a[8][N];
+  b128 b[NB];
+  auto load_a = [&](int slot, int c, int u) __attribute__((always_inline)) {  // k-step u of chunk c
+    const int off = (c >> 2) * sa8 + (16 * (c & 3) + 4 * u) * ld8;
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+      const b64 x = __builtin_amdgcn_raw_buffer_load_b64(ra, va + 128 * t, off, 0);
+      a[slot][t] = make_float2(__uint_as_float(x[0]), __uint_as_float(x[1]));
+    }
+  };
+  auto load_b = [&](int c) __attribute__((always_inline)) {
+    const int off = (c >> 2) * sb8 + 128 * (c & 3);
+#pragma unroll
+    for (int m = 0; m < NB; m++)
+      b[m] = __builtin_amdgcn_raw_buffer_load_b128(rb, vb, off + 8 * m * ld8, 0);
+  };
+  auto put_b = [&](int buf) __attribute__((always_inline)) {
+    wave_lds_fence();
+#pragma unroll
+    for (int m = 0; m < NB; m++) *(b128 *)&st.b[buf][bc + 8 * m][bk] = b[m];
+    wave_lds_fence();
+  };
+  auto chunk = [&](int c, int buf, bool next) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (next) load_a((4 * buf + u + 4) & 7, c + 1, u);
+      float2 av[N], bv[N];
+#pragma unroll
+      for (int t = 0; t < N; t++) {
+        av[t] = a[4 * buf + u][t];
+        bv[t] = st.b[buf][16 * t + li][4 * u + kq];
+      }
+      gemm3m_step<float, N>(av, bv, q);
+    }
+  };
+  const int nc = 4 * ns;
+  load_b(0);
+#pragma unroll
+  for (int u = 0; u < 4; u++) load_a(u, 0, u);
+  put_b(0);
+  load_b(1);
+  int c = 0;
+#pragma unroll 1
+  for (; c < nc - 2; c += 2) {
+    put_b(1);
+    load_b(c + 2);
+    chunk(c, 0, true);
+    put_b(0);
+    load_b(c + 3);
+    chunk(c + 1, 1, true);
+  }
+  put_b(1);
+  chunk(c, 0, true);
+  chunk(c + 1, 1, false);
+#endif
+}
+
+// LDS of a workgroup's four waves for tile_products.
+template <class T, int N>
+struct ProductStage {
+  int none;
+};
+template <>
+struct ProductStage<double, 1> {
+  BStage w[4];
+};
+template <int N>
+struct ProductStage<float, N> {
+  BStage32<N> w[4];
+};
+
 // q += sum_{u < ns} A_u B_u over 64-wide tiles: A_u = A + u sa, B_u = B + u sb
 // (FP64: consecutive in k, so that ns tiles are one product).
 template <class T, int N>
 __device__ __forceinline__ void tile_products(const GCx<T> *A, long sa, const GCx<T> *B, long sb,
-                                              long ld, int ns, Acc3<T, N> &q, BStage *st) {
-  if constexpr (sizeof(T) == 8 && N == 1) {
-    if (ns > 0) wave_gemm3m_staged(A, B, ld, 16 * ns, q, st[threadIdx.x >> 6]);
-  } else if constexpr (sizeof(T) == 8) {
-    if (ns > 0) wave_gemm3m_k(A, B, ld, 16 * ns, q);
-  } else {
-    for (int u = 0; u < ns; u++, A += sa, B += sb)
-      wave_gemm3m<T, N, N == 2 ? 3 : 7>([&](int i, int k) { return ldg<T>(A + (i + ld * k)); },
-                                        [&](int k, int j) { return ldg<T>(B + (k + ld * j)); },
-                                        kTile / 4, q);
-  }
+                                              long ld, int ns, Acc3<T, N> &q,
+                                              ProductStage<T, N> &st) {
+  if (ns <= 0) return;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if constexpr (sizeof(T) == 4) tile_products_f32<N>(A, sa, B, sb, ld, ns, q, st.w[w]);
+  else if constexpr (N == 1) wave_gemm3m_staged(A, B, ld, 16 * ns, q, st.w[w]);
+  else wave_gemm3m_k(A, B, ld, 16 * ns, q);
 }
 
 template <class T, int N>
@@ -403,7 +498,7 @@ template <class T, int N>
 struct PanelLds {
   union {
     __align__(16) CxT<T> c[kTile * ((N == 2 ? kTile : 16) + 1)];
-    BStage st[sizeof(T) == 8 && N == 1 ? 4 : 1];  // before that: B of the earlier steps
+    ProductStage<T, N> st;  // before that: B of the earlier steps
   };
   int rowpos[kTile];
   __device__ PanelLds() {}
@@ -455,7 +550,7 @@ __device__ __forceinline__ void panel_op(GCx<T> *__restrict__ C, bool load_c, bo
       }
   tile_products<T, N>(A + (r0 + wr), sa, B + ld * (c0 + wc), sb, ld, ns, q, lds.st);
   // rowpos is there, the staged operands are read
-  if (OP == kLeftL || (sizeof(T) == 8 && N == 1)) __syncthreads();
+  if (OP == kLeftL || sizeof(T) == 4 || N == 1) __syncthreads();
 #pragma unroll
   for (int bj = 0; bj < N; bj++)
 #pragma unroll

@@ -592,7 +592,7 @@ __device__ __forceinline__ void update_tile(const SolveDesc &d, int ti, int tj, 
       }
   const GCx<T> *A = tile_ptr<T>(d, ti, s0), *B = tile_ptr<T>(d, s0, tj);
   const long sa = tile_ptr<T>(d, ti, s0 + 1) - A, sb = tile_ptr<T>(d, s0 + 1, tj) - B;
-  __shared__ BStage st[sizeof(T) == 8 && N == 1 ? 4 : 1];
+  __shared__ ProductStage<T, N> st;
   tile_products<T, N>(A + wr, sa, B + ld * wc, sb, ld, ns, q, st);
 #pragma unroll
   for (int bj = 0; bj < N; bj++)
