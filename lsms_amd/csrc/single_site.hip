@@ -74,7 +74,7 @@ __device__ inline zd zexp_i(zd z) {  // e^{i z}
 }
 
 // Bulirsch-Stoer step-count sequence n_j = 2 n_{j-2} (bulirschStoerIntegrator.cpp:66-67)
-__device__ constexpr int kSeq[12] = {2, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
+__device__ constexpr int kSeq[13] = {2, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192};
 constexpr int kBsSteps = 11;
 constexpr int kBsTarget = 7;
 constexpr double kBsEps = 1.0e-12;
@@ -185,7 +185,9 @@ __device__ inline double quad_value(double v) {
 // extrapolate with all rows; the row that ends the step is the first that
 // passes the test, as when they are formed one by one.  A step that ends at
 // row 4 (94% of them on the radial meshes of the single-site problem) is a
-// chain of 9 derivatives, not of 24.
+// chain of 9 derivatives, not of 24.  Nearly all the others end at row 5, and a
+// wave waits for the slowest of its 16 tasks: row 5 is a block of its own (12
+// substeps, where rows 5 to 8 together are 32; 512 solves 1.22 -> 1.15 ms).
 template <int NQ>
 __device__ int bs_interval(double x0, double x1, double *y, double *dy, double rn,
                            const double *pc, const RhsPar &p, int q) {
@@ -200,13 +202,15 @@ __device__ int bs_interval(double x0, double x1, double *y, double *dy, double r
     bool more = true, ok = false;
     int step = 0;
 #pragma unroll
-    for (int ib = 0; ib < kBsSteps; ib += 4) {
+    for (int blk = 0; blk < 4; blk++) {
+      constexpr int kStart[5] = {0, 4, 5, 9, kBsSteps};
+      const int ib = kStart[blk], ie = kStart[blk + 1];
       if (more) {
-        double yb[4][4];  // the midpoint values of rows ib .. ib+3
+        double yb[4][4];  // the midpoint values of rows ib .. ie-1
         if (NQ == 4) {
           double y1[4];
           const int n = q == 0 ? kSeq[ib] : q == 1 ? kSeq[ib + 1] : q == 2 ? kSeq[ib + 2] : kSeq[ib + 3];
-          midpoint4(x, x + h, y, y1, ib + q < kBsSteps ? n : kSeq[ib], rn, pc, p);
+          midpoint4(x, x + h, y, y1, ib + q < ie ? n : kSeq[ib], rn, pc, p);
 #pragma unroll
           for (int d = 0; d < 4; d++) {
             yb[0][d] = quad_value<0>(y1[d]);
@@ -218,7 +222,7 @@ __device__ int bs_interval(double x0, double x1, double *y, double *dy, double r
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           const int i = ib + u;
-          if (i < kBsSteps && (NQ == 4 || more)) {
+          if (i < ie && (NQ == 4 || more)) {
             if (NQ == 1) midpoint4(x, x + h, y, yb[u], kSeq[i], rn, pc, p);
             double e = 0.0, mag = 0.0;
 #pragma unroll
@@ -515,7 +519,7 @@ __global__ void k_fitpot(const double *__restrict__ rmesh, const double *__restr
 // p, l): rwave.f with the outputs of semrel_c.f (solver 2).  The time is one
 // thread's chain of dependent FP64 operations over the mesh as long as the
 // threads do not fill the chip: 16 potentials x 32 energies x 4 l are 64 waves
-// at one thread each, 2.41 ms, and 256 at four, 1.27.  matom[(e*npot + p)*(lmax+1) + l];
+// at one thread each, 2.41 ms, and 256 at four, 1.15.  matom[(e*npot + p)*(lmax+1) + l];
 // zlr/jlr (may be null) columns of iprpts at ((e*npot + p)*(lmax+1) + l)*iprpts.
 template <int NQ>
 __global__ void __launch_bounds__(64) k_single_site(
