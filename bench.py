@@ -398,10 +398,10 @@ def main():
     # (kernel, elimination steps per trailing update)
     kernel, peak, flop_mult, cb, pb, dtype, prec, group = {
         # 3M: 3 real products (6 flops) per complex multiply-add (8 flops)
-        "fp64": ("k_lu_trail<double>", FP64_PEAK_TFLOPS, 0.75, 16, 16, "f64", "FP64", 2),
+        "fp64": ("k_lu_trail<double>", FP64_PEAK_TFLOPS, 0.75, 16, 16, "f64", "FP64", 4),
         "fp32_update": ("k_lu_trail<float>", FP32_PEAK_TFLOPS, 0.75, 8, 8,
                         "c32-factor+f64-refine",
-                        "mixed: complex FP32 LU on MFMA + FP64 iterative refinement", 2),
+                        "mixed: complex FP32 LU on MFMA + FP64 iterative refinement", 4),
         # 4M x 3 split products: 12 real products (24 flops) per complex multiply-add
         "split_f16_update": ("k_lu_trail_h", FP16_PEAK_TFLOPS, 3.0, 8, 8,
                              "f16x2-split-update+f32-factor+f64-refine",

@@ -61,7 +61,7 @@ struct SolveDesc {
   int pad;                // identity rows/cols at the front
   int nt;                 // Ns / kTile (solver layout)
   int step0;              // global step at which this solve's elimination starts
-  int group;              // elimination steps per trailing update (2, or 4 with split planes)
+  int group;              // elimination steps per trailing update (4; 4, 8 or 16 with split planes)
   // factorization state
   void *inv;              // per diagonal tile: L^-1 (strict lower) and U^-1 (upper), kTile^2
   long inv_stride;        // elements between the tiles of consecutive steps (0: one reused tile)
