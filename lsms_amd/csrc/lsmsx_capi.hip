@@ -41,8 +41,8 @@ template <class T>
 __global__ void k_lu_diag(const SolveDesc *, int);
 template <class T, int N>
 __global__ void k_lu_panel(const SolveDesc *, int, int, int);
-template <class T>
-__global__ void k_lu_cross_diag(const SolveDesc *, int, int);
+template <class T, int U>
+__global__ void k_lu_cross_diag(const SolveDesc *, int);
 template <class T, int N>
 __global__ void k_lu_trail(const SolveDesc *, int, int);
 template <class T>
@@ -510,7 +510,10 @@ int launch_lu_steps(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool 
       const int u = t - s, np = 2 * (nt_max - 1 - t);
       if (u > 0 && !split_f16) {
         ProfScope p(c, 9);
-        hipLaunchKernelGGL(k_lu_cross_diag<T>, dim3(4, nb), dim3(256), 0, st, dd, s, u);
+        const auto cross = u == 1   ? k_lu_cross_diag<T, 1>
+                           : u == 2 ? k_lu_cross_diag<T, 2>
+                                    : k_lu_cross_diag<T, 3>;  // u < lu_group() = 4
+        hipLaunchKernelGGL(cross, dim3(16, nb), dim3(256), 0, st, dd, s);
       }
       if (int r = check_launch("k_lu_cross_diag")) return r;
       {

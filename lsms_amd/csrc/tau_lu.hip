@@ -615,17 +615,64 @@ __device__ __forceinline__ int group_steps(const SolveDesc &d, int g) {
   return min(d.group, d.nt - 1 - g);
 }
 
-// Cross update of the diagonal tile of step t = g + u of the group starting at
-// global step s with the steps g .. t-1, a quarter of the tile per workgroup
-// (the panel tiles take theirs in k_lu_panel).
-template <class T>
+// Cross update of the diagonal tile of step t = g + U of the group starting at
+// global step s with the steps g .. t-1 (the panel tiles take theirs in
+// k_lu_panel): a 16x16 block per workgroup, a quarter of each step's k per
+// wave, summed through LDS.  It lies between two diagonal tiles, and its
+// latency counts: all operands are loaded at once, and the product's chain is
+// 12 U FP64 MFMAs (with a quarter tile per workgroup and a 16x16 block per wave
+// 48 U; one solve N = 2160: 7.0 -> 4.6 us a launch, of which most is the launch).  B goes through LDS as in
+// wave_gemm3m_staged.
+template <class T, int U>
 __global__ __launch_bounds__(256) void k_lu_cross_diag(const SolveDesc *__restrict__ descs,
-                                                       int step, int u) {
+                                                       int step) {
+  typedef CxT<T> V;
   const SolveDesc &d = descs[blockIdx.y];
-  const int g = step - d.step0, t = g + u;
-  if (g < 0 || u >= group_steps(d, g)) return;
+  const int g = step - d.step0, t = g + U;
+  if (g < 0 || U >= group_steps(d, g)) return;
   if (d.conv && *d.conv) return;
-  update_tile<T, 1>(d, t, t, g, u, blockIdx.x);
+  __shared__ __align__(16) V st[4][U][16][17];  // [wave][step][column][k], then [column][row]
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = 16 * (blockIdx.x & 3), c0 = 16 * (blockIdx.x >> 2);
+  const long ld = tile_ld(d);
+  GCx<T> *C = tile_ptr<T>(d, t, t) + (r0 + (tid & 15)) + ld * (c0 + (tid >> 4));
+  V a[U][4], b[U][4];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const GCx<T> *A = tile_ptr<T>(d, t, g + u) + (r0 + li) + ld * (16 * w + kq);
+    const GCx<T> *B = tile_ptr<T>(d, g + u, t) + (16 * w + li) + ld * (c0 + kq);
+#pragma unroll
+    for (int m = 0; m < 4; m++) b[u][m] = ldg<T>(B + 4 * m * ld);
+#pragma unroll
+    for (int m = 0; m < 4; m++) a[u][m] = ldg<T>(A + 4 * m * ld);
+  }
+  V c = ldg<T>(C);
+#pragma unroll
+  for (int u = 0; u < U; u++)
+#pragma unroll
+    for (int m = 0; m < 4; m++) st[w][u][kq + 4 * m][li] = b[u][m];
+  wave_lds_fence();
+  Acc3<T, 1> q;
+  zero_acc(q);
+#pragma unroll
+  for (int u = 0; u < U; u++)
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      V av[1] = {a[u][m]}, bv[1] = {st[w][u][li][4 * m + kq]};
+      gemm3m_step<T, 1>(av, bv, q);
+    }
+  wave_lds_fence();
+#pragma unroll
+  for (int r = 0; r < 4; r++) st[w][0][acc_row<T>(kq, r)][li] = minus_value<T, 1>(q, 0, 0, r);
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    const V p = st[v][0][tid >> 4][tid & 15];
+    c.x += p.x;
+    c.y += p.y;
+  }
+  *C = c;
 }
 
 // Trailing update of the group starting at global step s: A_ij -= sum over
@@ -727,8 +774,12 @@ template __global__ void k_lu_panel<double, 2>(const SolveDesc *, int, int, int)
 template __global__ void k_lu_panel<double, 1>(const SolveDesc *, int, int, int);
 template __global__ void k_lu_panel<float, 2>(const SolveDesc *, int, int, int);
 template __global__ void k_lu_panel<float, 1>(const SolveDesc *, int, int, int);
-template __global__ void k_lu_cross_diag<double>(const SolveDesc *, int, int);
-template __global__ void k_lu_cross_diag<float>(const SolveDesc *, int, int);
+template __global__ void k_lu_cross_diag<double, 1>(const SolveDesc *, int);
+template __global__ void k_lu_cross_diag<double, 2>(const SolveDesc *, int);
+template __global__ void k_lu_cross_diag<double, 3>(const SolveDesc *, int);
+template __global__ void k_lu_cross_diag<float, 1>(const SolveDesc *, int);
+template __global__ void k_lu_cross_diag<float, 2>(const SolveDesc *, int);
+template __global__ void k_lu_cross_diag<float, 3>(const SolveDesc *, int);
 template __global__ void k_lu_trail<double, 2>(const SolveDesc *, int, int);
 template __global__ void k_lu_trail<double, 1>(const SolveDesc *, int, int);
 template __global__ void k_lu_trail<float, 2>(const SolveDesc *, int, int);

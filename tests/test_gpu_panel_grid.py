@@ -46,3 +46,22 @@ def test_group_remainders(n):
     tau, info = capi.Context(0).solve_tau00_matrix(m, t0)
     assert info == 0
     assert np.linalg.norm(tau - ref[:16]) <= 8 * n * EPS * np.linalg.cond(m) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("precision", [capi.PREC_FP64, capi.PREC_MIXED_FP32])
+@pytest.mark.parametrize("right_align", [0, 1])
+def test_cross_updates_of_uneven_batch(precision, right_align):
+    """Solves of different tile counts in one launch sequence: a solve whose group
+    ends early leaves the later cross updates out.  A wrong FP32 update shows as a
+    refinement that does not converge and falls back to FP64 (iters = -1)."""
+    s = CF.config_c4()
+    ctx = capi.Context(0)
+    ctx.load_system(s)
+    ctx.set_schedule(right_align)
+    atoms, ie = pick(s, 6), 9
+    tau, info = ctx.tau00_batched(atoms, [ie] * 6, [s.prel(ie)] * 6, 16, precision=precision)
+    assert np.all(info == 0)
+    iters, _ = ctx.last_stats(6)
+    assert np.all(iters == 0 if precision == capi.PREC_FP64 else iters > 0)
+    for a, t in zip(atoms, tau):
+        assert rel(t, lapack_tau00(s, a, ie)) < 1e-10
