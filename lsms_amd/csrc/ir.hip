@@ -154,6 +154,57 @@ __global__ __launch_bounds__(256) void k_ir_residual(const SolveDesc *__restrict
 // (-1)^l of the lm index a = l(l+1) + m, a < 16.
 __device__ __forceinline__ double lsign(int a) { return (a == 0 || (a >= 4 && a < 9)) ? 1.0 : -1.0; }
 
+// Padding rows of the residual, R = -X (identity block, B = 0), by a workgroup
+// of 512 threads.
+__device__ __forceinline__ void residual_g_pad(const SolveDesc &d) {
+  const int tid = threadIdx.x, Ns = d.Ns, pad = d.pad, kc = d.kc;
+  const gd2 *__restrict__ X = (const gd2 *)d.X;
+  GCx<float> *__restrict__ R = (GCx<float> *)d.R;
+  for (int e = tid; e < pad * kc; e += 512) {
+    const int row = e % pad, col = e / pad;
+    const double2 x = ldg<double>(X + row + (long)Ns * col);
+    float2 o;
+    o.x = (float)-x.x;
+    o.y = (float)-x.y;
+    R[row + (long)Ns * col] = o;
+  }
+}
+
+// R_q = B_q - X_q + t_q Y_q (M = 1 - t G) of site q by a wave, Y_q in the MFMA
+// accumulator layout; R stored in FP32.
+__device__ __forceinline__ void residual_g_site(const SolveDesc &d, int q, const double2 (&yv)[4]) {
+  const int n = d.numLIZ, lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
+  const int Ns = d.Ns, pad = d.pad, kc = d.kc;
+  const gd2 *__restrict__ X = (const gd2 *)d.X;
+  GCx<float> *__restrict__ R = (GCx<float> *)d.R;
+  // t_q Y_q: a-operand t(li, 4u + kq), b-operand Y(4u + kq, li) = yv[u]
+  const int site = site_at_pos(q, n);
+  const gd2 *__restrict__ T = (const gd2 *)(d.tmat + d.ldT * d.store[site] + d.t_off);
+  d4 q1 = {0.0, 0.0, 0.0, 0.0}, q2 = q1, q3 = q1;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const double2 tv = ldg<double>(T + li + (long)d.ldt * (4 * u + kq));
+    q1 = mfma4(tv.x, yv[u].x, q1);
+    q2 = mfma4(tv.y, yv[u].y, q2);
+    q3 = mfma4(tv.x + tv.y, yv[u].x + yv[u].y, q3);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int row = pad + 16 * q + kq + 4 * r;
+    const double2 x = ldg<double>(X + row + (long)Ns * li);
+    double br = 0.0, bi = 0.0;
+    if (row >= Ns - kc) {
+      const double2 t = d.t0[(row - (Ns - kc)) + (long)d.ldt * li];
+      br = t.x;
+      bi = t.y;
+    }
+    float2 o;
+    o.x = (float)(br - x.x + (q1[r] - q2[r]));
+    o.y = (float)(bi - x.y + (q3[r] - q1[r] - q2[r]));
+    R[row + (long)Ns * li] = o;
+  }
+}
+
 // Residual of the mixed path without an FP64 M, first half: Y = G X from the
 // structure constants stored once per site pair (d.gh, G_pq for solver
 // positions p < q; G_qp = D G_pq D, D = diag (-1)^l), each block read once
@@ -173,7 +224,7 @@ __global__ __launch_bounds__(512) void k_ir_residual_g(const SolveDesc *__restri
   if (*d.conv) return;
   const int n = d.numLIZ, nbands = (n + kGBand - 1) / kGBand;
   const int wg = blockIdx.x;
-  if (wg >= (nbands + 1) / 2) return;
+  if (wg >= (nbands + 1) / 2 || nbands <= kGDirectBands) return;
   __shared__ double2 zs[kGWaves][kGSites][256];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, li = lane & 15, kq = lane >> 4;
   const int Ns = d.Ns, pad = d.pad;
@@ -300,22 +351,11 @@ __global__ __launch_bounds__(512) void k_ir_residual_g_finish(const SolveDesc *_
   const SolveDesc &d = descs[blockIdx.y];
   if (*d.conv) return;
   const int n = d.numLIZ, nbands = (n + kGBand - 1) / kGBand, c = blockIdx.x;
-  if (c >= nbands) return;
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, li = lane & 15, kq = lane >> 4;
-  const int Ns = d.Ns, pad = d.pad, kc = d.kc;
-  const gd2 *__restrict__ X = (const gd2 *)d.X;
+  if (c >= nbands || nbands <= kGDirectBands) return;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, kq = lane >> 4;
   const gd2 *__restrict__ YB = (const gd2 *)d.ybuf;
   const gd2 *__restrict__ GP = (const gd2 *)d.gpart;
-  GCx<float> *__restrict__ R = (GCx<float> *)d.R;
-  if (c == 0)
-    for (int e = tid; e < pad * kc; e += 512) {
-      const int row = e % pad, col = e / pad;
-      const double2 x = ldg<double>(X + row + (long)Ns * col);
-      float2 o;
-      o.x = (float)-x.x;
-      o.y = (float)-x.y;
-      R[row + (long)Ns * col] = o;
-    }
+  if (c == 0) residual_g_pad(d);
 #pragma unroll
   for (int sq = 0; sq < kGSites; sq++) {
     const int q = kGBand * c + kGSites * w + sq;
@@ -341,33 +381,95 @@ __global__ __launch_bounds__(512) void k_ir_residual_g_finish(const SolveDesc *_
       yv[r].x += sgn * zv[r].x;
       yv[r].y += sgn * zv[r].y;
     }
-    // t_q Y_q: a-operand t(li, 4u + kq), b-operand Y(4u + kq, li) = yv[u]
-    const int site = site_at_pos(q, n);
-    const gd2 *__restrict__ T = (const gd2 *)(d.tmat + d.ldT * d.store[site] + d.t_off);
-    d4 q1 = {0.0, 0.0, 0.0, 0.0}, q2 = q1, q3 = q1;
+    residual_g_site(d, q, yv);
+  }
+}
+
+// The residual of a solve of up to kGDirectBands bands, whole: workgroup p takes
+// site p, wave w the blocks of the sites q = w, w + 8, ..., Y_p summed over the
+// waves in order.  Every block is read twice, but a solve's products go to as
+// many compute units as it has sites, where in bands they are one's to four's,
+// in a chain of its stages (16 solves of 15 sites: 57 + 5 -> 26 us, a batch 729
+// -> 659 us; 96 of 56 to 128 sites: a batch 18.0 -> 16.8 ms with the line at four
+// bands, 16.3 at eight).  In large batches both run at the rate of HBM and the
+// caches (2048 of those: 348 ms either way) until the second read shows: 992
+// solves of 135 sites, 175 ms in bands, 178 so, and 248 of them 48.1 and 47.2.
+// The line is by size alone, so that a solve's result does not depend on its
+// batch.
+__global__ __launch_bounds__(512) void k_ir_residual_g_site(const SolveDesc *__restrict__ descs) {
+  const SolveDesc &d = descs[blockIdx.y];
+  if (*d.conv) return;
+  const int n = d.numLIZ, p = blockIdx.x;
+  if (p >= n || n > kGBand * kGDirectBands) return;
+  __shared__ double2 part[kGWaves][256];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
+  const int Ns = d.Ns, pad = d.pad;
+  const gd2 *__restrict__ X = (const gd2 *)d.X;
+  const gd2 *__restrict__ GH = (const gd2 *)d.gh;
+  if (p == 0) residual_g_pad(d);
+  // y over q > p, and z over q < p, where G_pq = D G_qp D is stored as G_qp
+  d4 y[3], z[3];
+#pragma unroll
+  for (int m = 0; m < 3; m++) y[m] = z[m] = d4{0.0, 0.0, 0.0, 0.0};
+  auto load_q = [&](int q, double2 (&g)[4], double2 (&x)[4]) __attribute__((always_inline)) {
+    const int q1 = min(q, n - 1);
+    // q == p has no block: any other one is read and not used
+    const int lo = q1 == p ? 0 : min(p, q1), hi = q1 == p ? n - 1 : max(p, q1);
+    const gd2 *G = GH + (lo < hi ? gh_index(lo, hi, n) * 256 : 0);
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      const double2 tv = ldg<double>(T + li + (long)d.ldt * (4 * u + kq));
-      q1 = mfma4(tv.x, yv[u].x, q1);
-      q2 = mfma4(tv.y, yv[u].y, q2);
-      q3 = mfma4(tv.x + tv.y, yv[u].x + yv[u].y, q3);
+      g[u] = ldg<double>(G + li + 16 * (4 * u + kq));
+      x[u] = ldg<double>(X + (pad + 16 * q1 + 4 * u + kq) + (long)Ns * li);
     }
+  };
+  auto add = [&](d4 (&a)[3], double2 g, double2 x) __attribute__((always_inline)) {
+    a[0] = mfma4(g.x, x.x, a[0]);
+    a[1] = mfma4(g.y, x.y, a[1]);
+    a[2] = mfma4(g.x + g.y, x.x + x.y, a[2]);
+  };
+  double2 g[4], x[4], gn[4], xn[4];
+  if (n > 1) {
+    load_q(w, g, x);
+    for (int q = w; q < n; q += kGWaves) {
+      load_q(q + kGWaves, gn, xn);
+      if (q > p) {
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int row = pad + 16 * q + kq + 4 * r;
-      const double2 x = ldg<double>(X + row + (long)Ns * li);
-      double br = 0.0, bi = 0.0;
-      if (row >= Ns - kc) {
-        const double2 t = d.t0[(row - (Ns - kc)) + (long)d.ldt * li];
-        br = t.x;
-        bi = t.y;
+        for (int u = 0; u < 4; u++) add(y, g[u], x[u]);
+      } else if (q < p) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const double s = lsign(4 * u + kq);
+          add(z, g[u], make_double2(s * x[u].x, s * x[u].y));
+        }
       }
-      float2 o;
-      o.x = (float)(br - x.x + (q1[r] - q2[r]));
-      o.y = (float)(bi - x.y + (q3[r] - q1[r] - q2[r]));
-      R[row + (long)Ns * li] = o;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        g[u] = gn[u];
+        x[u] = xn[u];
+      }
     }
   }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const double s = lsign(kq + 4 * r);
+    part[w][r * 64 + lane] = make_double2(y[0][r] - y[1][r] + s * (z[0][r] - z[1][r]),
+                                          y[2][r] - y[0][r] - y[1][r] +
+                                              s * (z[2][r] - z[0][r] - z[1][r]));
+  }
+  __syncthreads();
+  if (w > 0) return;
+  double2 yv[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    yv[r] = part[0][r * 64 + lane];
+#pragma unroll
+    for (int v = 1; v < kGWaves; v++) {
+      yv[r].x += part[v][r * 64 + lane].x;
+      yv[r].y += part[v][r * 64 + lane].y;
+    }
+  }
+  residual_g_site(d, p, yv);
 }
 
 // 3M sums of a wave's 16 x 16nb block in the refinement sweeps: transposed

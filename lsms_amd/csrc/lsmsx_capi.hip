@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <complex>
 #include <chrono>
 #include <cmath>
@@ -60,6 +61,7 @@ template <bool FIRST, int RB, SweepPart PART>
 __global__ void k_ir_sweep(const SolveDesc *, double);
 __global__ void k_ir_residual_g(const SolveDesc *);
 __global__ void k_ir_residual_g_finish(const SolveDesc *);
+__global__ void k_ir_residual_g_site(const SolveDesc *);
 __global__ void k_copy_m(const SolveDesc *);
 __global__ void k_fitpot(const double *, const double *, const int *, int, int, double *);
 template <int NQ>
@@ -655,14 +657,20 @@ int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int ma
 // return at once (16 solves of four tiles, eight sweeps left out: 792 -> 762 us
 // a batch).
 int refine_async(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int max_sweeps,
-                 double tol, hipStream_t st, int nbands_max, bool look) {
+                 double tol, hipStream_t st, int nbands_min, int nbands_max, bool look) {
   hipLaunchKernelGGL(k_ir_init<float>, dim3(nt_max, nb), dim3(256), 0, st, dd);
   for (int it = 0; it < max_sweeps; it++) {
     if (it > 0) {
       ProfScope p(c, 5);
       if (nbands_max > 0) {  // structure constants once per site pair
-        hipLaunchKernelGGL(k_ir_residual_g, dim3((nbands_max + 1) / 2, nb), dim3(512), 0, st, dd);
-        hipLaunchKernelGGL(k_ir_residual_g_finish, dim3(nbands_max, nb), dim3(512), 0, st, dd);
+        if (nbands_max > kGDirectBands) {
+          hipLaunchKernelGGL(k_ir_residual_g, dim3((nbands_max + 1) / 2, nb), dim3(512), 0, st, dd);
+          hipLaunchKernelGGL(k_ir_residual_g_finish, dim3(nbands_max, nb), dim3(512), 0, st, dd);
+        }
+        if (nbands_min <= kGDirectBands)
+          hipLaunchKernelGGL(k_ir_residual_g_site,
+                             dim3(kGBand * std::min(nbands_max, kGDirectBands), nb), dim3(512), 0,
+                             st, dd);
       } else {
         hipLaunchKernelGGL((k_ir_residual<float, 1>), dim3(nt_max, nb), dim3(256), 0, st, dd);
       }
@@ -826,7 +834,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
     while (end < nsolve && (end == done || acc + bytes[end] <= cap)) acc += bytes[end++];
     int nb = end - done;
     long mtot = 0, xtot = 0, ivtot = 0, htot = 0, ghtot = 0, ybtot = 0, gptot = 0;
-    int maxliz = 1, nt_max = 1, nbands_max = 0;
+    int maxliz = 1, nt_max = 1, nbands_min = INT_MAX, nbands_max = 0;
     for (int b = 0; b < nb; b++) {
       const AtomDev &a = c->atoms[atom_ids[done + b]];
       long Ns = roundup(nsc * a.nrmat, kTile);
@@ -841,6 +849,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
         ybtot += (long)a.numLIZ * 256;
         gptot += g_slots(a.numLIZ) * 256;
         nbands_max = std::max(nbands_max, (a.numLIZ + kGBand - 1) / kGBand);
+        nbands_min = std::min(nbands_min, (a.numLIZ + kGBand - 1) / kGBand);
       }
     }
     if (gmode) {
@@ -1066,7 +1075,8 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
       if (!mixed) return launch_lu<double>(c, dd, n, ntm, false, st, uniform);
       if (int r = launch_lu<float>(c, dd, n, ntm, split, st, uniform)) return r;
       if (ir_inline)
-        return refine_async(c, dd, n, ntm, c->ir_max_sweeps, c->ir_tol, st, gmode ? nbands_max : 0,
+        return refine_async(c, dd, n, ntm, c->ir_max_sweeps, c->ir_tol, st,
+                            gmode ? nbands_min : 0, gmode ? nbands_max : 0,
                             !two && !c->use_graph);
       return 0;
     };
@@ -1095,6 +1105,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
       std::vector<long> key = {nb, nt_max, maxliz, precision, c->sched, (long)c->desc.p,
                                (long)c->tmat.p, c->ldT, (long)c->cgnt.p, (long)c->illp.p,
                                c->lmax_tab, c->ir_max_sweeps, tol_bits, gmode ? nbands_max : -1,
+                               (long)(gmode && nbands_min <= kGDirectBands),
                                lu_group(c, split), share ? (long)own.size() : -1,
                                (long)c->desc_own.p, (long)uniform};
       auto it = c->graphs.find(key);

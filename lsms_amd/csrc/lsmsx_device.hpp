@@ -118,6 +118,7 @@ constexpr int kAsmG = 3;
 constexpr int kGBand = 16;
 constexpr int kGWaves = 8;
 constexpr int kGSites = kGBand / kGWaves;
+constexpr int kGDirectBands = 8;  // up to here a workgroup per site (k_ir_residual_g_site)
 
 // Block of the solver-position pair p < q among n sites (row-major upper triangle).
 __host__ __device__ inline long gh_index(int p, int q, int n) {
