@@ -622,8 +622,8 @@ __device__ __forceinline__ int group_steps(const SolveDesc &d, int g) {
 // latency counts: all operands are loaded at once, and the product's chain is
 // 12 U FP64 MFMAs (with a quarter tile per workgroup and a 16x16 block per wave
 // 48 U; one solve N = 2160: 7.0 -> 4.6 us a launch, of which most is the
-// launch; 992 at once, at the rate of HBM: 105 -> 125 us, 0.1% of their step).  B goes through LDS as in
-// wave_gemm3m_staged.
+// launch; 992 at once, at the rate of HBM: 105 -> 125 us, 0.1% of their step).
+// B goes through LDS as in wave_gemm3m_staged.
 template <class T, int U>
 __global__ __launch_bounds__(256) void k_lu_cross_diag(const SolveDesc *__restrict__ descs,
                                                        int step) {
