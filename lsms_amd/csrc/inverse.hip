@@ -41,10 +41,10 @@ __global__ __launch_bounds__(256) void k_inv_fwd(const SolveDesc *__restrict__ d
   __shared__ PanelLds<double, N> lds;
   const long ld = d.ld;
   GZ *M = (GZ *)d.M, *Y = (GZ *)d.Minv;
-  panel_op<double, N, kLeftL>(Y + kTile * (step + ld * c), false, c == step,
-                              M + kTile * (step + ld * c), 0, Y + kTile * (c + ld * c), 0, ld,
-                              step - c, (const GZ *)d.inv + step * d.inv_stride,
-                              (const LSMSX_GLOBAL int *)d.perm + step * kTile, piece, lds);
+  panel_op<double, N, kLeftL, true>(Y + kTile * (step + ld * c), false, c == step,
+                                    M + kTile * (step + ld * c), 0, Y + kTile * (c + ld * c), 0, ld,
+                                    step - c, (const GZ *)d.inv + step * d.inv_stride,
+                                    (const LSMSX_GLOBAL int *)d.perm + step * kTile, piece, lds);
 }
 
 // Backward step s: Y_sc for every column tile c; the forward half left rows
@@ -59,10 +59,10 @@ __global__ __launch_bounds__(256) void k_inv_bwd(const SolveDesc *__restrict__ d
   const long ld = d.ld;
   const int s1 = min(step + 1, d.nt - 1);
   GZ *M = (GZ *)d.M, *Y = (GZ *)d.Minv;
-  panel_op<double, N, kLeftU>(Y + kTile * (step + ld * c), step >= c, false,
-                              M + kTile * (step + ld * s1), 0, Y + kTile * (s1 + ld * c), 0, ld,
-                              d.nt - 1 - step, (const GZ *)d.inv + step * d.inv_stride, nullptr,
-                              piece, lds);
+  panel_op<double, N, kLeftU, true>(Y + kTile * (step + ld * c), step >= c, false,
+                                    M + kTile * (step + ld * s1), 0, Y + kTile * (s1 + ld * c), 0,
+                                    ld, d.nt - 1 - step, (const GZ *)d.inv + step * d.inv_stride,
+                                    nullptr, piece, lds);
 }
 template __global__ void k_inv_fwd<1>(const SolveDesc *, int);
 template __global__ void k_inv_fwd<2>(const SolveDesc *, int);

@@ -198,15 +198,22 @@ __device__ __forceinline__ void wave_gemm3m(FA fa, FB fb, int nk, Acc3<T, N> &q)
 // operands come by buffer loads whose k offset is scalar, and the only VALU
 // work left of a step are the sums of the 3M form (through pointers, with A
 // negated, it was 17 instructions; 64 solves of N = 2160: trailing updates
-// 23.8 -> 22.4 ms at K = 128).
+// 23.8 -> 22.4 ms at K = 128).  The offsets have 32 bits.  A's k runs over a
+// group's four tiles in the LU, 4096 ld bytes, but over whole tile rows in the
+// explicit inverse, 16 ld^2: LONG moves A's 64-bit base with k there, and an
+// offset spans 32 columns at most.
+template <bool LONG>
 __device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<double> *B, long ld,
                                               int nk, Acc3<double, 2> &q) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef unsigned b128 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
   constexpr int kRange = 0x7fffffff, kFlags = 0x00027000;  // raw buffer, byte offsets
-  const auto ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, kRange, kFlags);
-  const auto rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, kRange, kFlags);
+  auto resource = [](const GCx<double> *p) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, kRange, kFlags);
+  };
+  auto ra = resource(A);
+  const auto rb = resource(B);
   const int ld16 = (int)ld * 16;
   constexpr int N = 2, PF = 3;
   const int va = 16 * li + ld16 * kq;  // A(li, kq)
@@ -217,8 +224,9 @@ __device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<do
   auto get = [](b128 x) __attribute__((always_inline)) {
     return double2{__hiloint2double(x[1], x[0]), __hiloint2double(x[3], x[2])};
   };
-  auto load = [&](int slot, int ks) __attribute__((always_inline)) {
-    const int sa = 4 * ks * ld16, sb = 64 * ks;
+  // k-step ks0 + u; LONG: ra at ks0
+  auto load = [&](int slot, int ks0, int u) __attribute__((always_inline)) {
+    const int sa = 4 * (LONG ? u : ks0 + u) * ld16, sb = 64 * (ks0 + u);
 #pragma unroll
     for (int t = 0; t < N; t++)
       a[slot][t] = get(__builtin_amdgcn_raw_buffer_load_b128(ra, va + 256 * t, sa, 0));
@@ -236,17 +244,21 @@ __device__ __forceinline__ void wave_gemm3m_k(const GCx<double> *A, const GCx<do
     gemm3m_step<double, N>(av, bv, q);
   };
 #pragma unroll
-  for (int i = 0; i < PF; i++) load(i, i);
+  for (int i = 0; i < PF; i++) load(i, 0, i);
   int ks = 0;
 #pragma unroll 1
   for (; ks < nk - PF - 1; ks += PF + 1) {
 #pragma unroll
     for (int i = 0; i <= PF; i++) {
-      load((i + PF) & PF, ks + i + PF);
+      load((i + PF) & PF, ks, i + PF);
       step(i);
     }
+    if (LONG) {
+      A += 4 * (PF + 1) * ld;
+      ra = resource(A);
+    }
   }
-  load(PF, ks + PF);
+  load(PF, ks, PF);
 #pragma unroll
   for (int i = 0; i <= PF; i++) step(i);
 #endif
@@ -276,7 +288,8 @@ struct BStage {
 // load, 16 accesses, and turned in LDS: 1.06 -> 0.87 ms there.  A 32 x 32
 // block, with half the loads to an MFMA, gains nothing (64 solves of N = 2160:
 // trailing updates 18.4 ms either way, six of N = 4384 16.2 and 16.5), and
-// neither do loads further ahead.
+// neither do loads further ahead.  A's base always moves, an offset spans 48
+// columns at most (eight adjoint solves of N = 944 2.33 ms either way).
 __device__ __forceinline__ void wave_gemm3m_staged(const GCx<double> *A, const GCx<double> *B,
                                                    long ld, int nk, Acc3<double, 1> &q,
                                                    BStage &st) {
@@ -284,8 +297,11 @@ __device__ __forceinline__ void wave_gemm3m_staged(const GCx<double> *A, const G
   typedef unsigned b128 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
   constexpr int kRange = 0x7fffffff, kFlags = 0x00027000;  // raw buffer, byte offsets
-  const auto ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, kRange, kFlags);
-  const auto rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, kRange, kFlags);
+  auto resource = [](const GCx<double> *p) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, kRange, kFlags);
+  };
+  auto ra = resource(A);
+  const auto rb = resource(B);
   const int ld16 = (int)ld * 16;
   const int v0 = 16 * li + ld16 * kq;  // A(li, kq); B(li, kq): 16 k, columns kq + 4 m
   double2 a[8], b[4];
@@ -306,12 +322,13 @@ __device__ __forceinline__ void wave_gemm3m_staged(const GCx<double> *A, const G
     for (int m = 0; m < 4; m++) st.b[buf][kq + 4 * m][li] = b[m];
     wave_lds_fence();
   };
-  // chunk c from LDS buffer `buf` (c mod 2); the A k-steps 4c+4 .. 4c+7 are
-  // loaded on the way when `next`
-  auto chunk = [&](int c, int buf, bool next) __attribute__((always_inline)) {
+  // the chunk in LDS buffer `buf` (its number mod 2), ra at the k-step 0 of a
+  // chunk in buffer 0; the A k-steps of the chunk after it are loaded on the way
+  // when `next`
+  auto chunk = [&](int buf, bool next) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      if (next) load_a((4 * buf + u + 4) & 7, 4 * c + u + 4);
+      if (next) load_a((4 * buf + u + 4) & 7, 4 * buf + u + 4);
       double2 av[1] = {a[4 * buf + u]}, bv[1] = {st.b[buf][li][4 * u + kq]};
       gemm3m_step<double, 1>(av, bv, q);
     }
@@ -327,14 +344,16 @@ __device__ __forceinline__ void wave_gemm3m_staged(const GCx<double> *A, const G
   for (; c < nc - 2; c += 2) {
     put_b(1);
     load_b(c + 2);
-    chunk(c, 0, true);
+    chunk(0, true);
     put_b(0);
     load_b(c + 3);
-    chunk(c + 1, 1, true);
+    chunk(1, true);
+    A += 32 * ld;
+    ra = resource(A);
   }
   put_b(1);
-  chunk(c, 0, true);
-  chunk(c + 1, 1, false);
+  chunk(0, true);
+  chunk(1, false);
 #endif
 }
 
@@ -438,8 +457,9 @@ struct ProductStage<float, N> {
 };
 
 // q += sum_{u < ns} A_u B_u over 64-wide tiles: A_u = A + u sa, B_u = B + u sb
-// (FP64: consecutive in k, so that ns tiles are one product).
-template <class T, int N>
+// (FP64: consecutive in k, so that ns tiles are one product).  LONG: ns is not
+// bounded by a group's four steps (FP64 alone).
+template <class T, int N, bool LONG = false>
 __device__ __forceinline__ void tile_products(const GCx<T> *A, long sa, const GCx<T> *B, long sb,
                                               long ld, int ns, Acc3<T, N> &q,
                                               ProductStage<T, N> &st) {
@@ -447,7 +467,7 @@ __device__ __forceinline__ void tile_products(const GCx<T> *A, long sa, const GC
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if constexpr (sizeof(T) == 4) tile_products_f32<N>(A, sa, B, sb, ld, ns, q, st.w[w]);
   else if constexpr (N == 1) wave_gemm3m_staged(A, B, ld, 16 * ns, q, st.w[w]);
-  else wave_gemm3m_k(A, B, ld, 16 * ns, q);
+  else wave_gemm3m_k<LONG>(A, B, ld, 16 * ns, q);
 }
 
 template <class T, int N>
@@ -514,7 +534,7 @@ struct PanelLds {
 // 16x16 block per wave: a quarter of the time per tile on four times the
 // workgroups, at twice the operand loads per MFMA.  `piece` = 0..3 then.
 // perm: the pivots of kLeftL; identity: C' = the identity tile (nothing else).
-template <class T, int N, PanelOp OP>
+template <class T, int N, PanelOp OP, bool LONG = false>
 __device__ __forceinline__ void panel_op(GCx<T> *__restrict__ C, bool load_c, bool identity,
                                          const GCx<T> *A, long sa, const GCx<T> *B, long sb,
                                          long ld, int ns, const GCx<T> *__restrict__ inv,
@@ -548,7 +568,7 @@ __device__ __forceinline__ void panel_op(GCx<T> *__restrict__ C, bool load_c, bo
         else if (identity) c.x = r0 + wr + i == c0 + wc + j ? T(1) : T(0);
         set_minus<T, N>(q, bj, bi, r, c.x, c.y);
       }
-  tile_products<T, N>(A + (r0 + wr), sa, B + ld * (c0 + wc), sb, ld, ns, q, lds.st);
+  tile_products<T, N, LONG>(A + (r0 + wr), sa, B + ld * (c0 + wc), sb, ld, ns, q, lds.st);
   // rowpos is there, the staged operands are read
   if (OP == kLeftL || sizeof(T) == 4 || N == 1) __syncthreads();
 #pragma unroll
