@@ -528,7 +528,7 @@ template <class T, bool FWD>
 __global__ __launch_bounds__(256) void k_ir_step(const SolveDesc *__restrict__ descs, int step) {
   typedef CxT<T> V;
   const SolveDesc &d = descs[blockIdx.y];
-  if (*d.conv) return;
+  if (*d.conv || half_sweeps<T>(d.kc, d.nt)) return;
   const int nt = d.nt;
   const bool first = FWD && step == kIrFirstSweep;
   const int s = FWD ? (first ? nt - 2 : step) : nt - 1 - step;
@@ -662,7 +662,7 @@ template <class T>
 __global__ __launch_bounds__(256) void k_ir_accum(const SolveDesc *__restrict__ descs, int central) {
   typedef CxT<T> V;
   const SolveDesc &d = descs[blockIdx.y];
-  if (*d.conv) return;
+  if (*d.conv || half_sweeps<T>(d.kc, d.nt)) return;
   const int t = central ? d.nt - 1 : (int)blockIdx.x;
   if (!central && t >= d.nt - 1) return;
   __shared__ double red[2][256];
@@ -739,7 +739,8 @@ __global__ void k_ir_decide(const SolveDesc *__restrict__ descs, int n, double t
 // central rows between the forward and the backward halves, and X += dX.  It
 // does the work of k_ir_step, k_ir_accum and k_ir_decide for one sweep.
 // With kc = 32 a workgroup takes 16 of the columns, and the halves are
-// launches of their own (kSweepFwd, kSweepBwd) with k_ir_decide between them.
+// launches of their own (kSweepFwd, kSweepBwd) with k_ir_decide between them,
+// for the solves of a chunk that half_sweeps names.
 //
 // Left-looking by tile row, with the tile rows dealt round-robin to teams of
 // NW = 4/RB waves (one wave, or a pair): team p of n takes t = p, p+n, ...
@@ -776,6 +777,7 @@ __global__ __launch_bounds__(kSweepWaves * 64) void k_ir_sweep(const SolveDesc *
   constexpr int kSweepD = 16 / RB;
   const SolveDesc &d = descs[blockIdx.x];
   if (*d.conv) return;
+  if (PART != kSweepAll && !half_sweeps<float>(d.kc, d.nt)) return;
   const int nt = d.nt, Ns = d.Ns;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kq = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), team = w / NW, half = w % NW;

@@ -582,14 +582,16 @@ inline bool sweep_pairs(int nt_max) { return nt_max <= kSweepPairTiles; }
 
 // Refinement sweeps on a chunk whose factors (T = float: mixed path with 32
 // right-hand sides; T = double: FP64-refined path) are in place: one launch
-// per tile column (k_ir_step), or, for FP32 factors as far as a pair of waves
-// takes them (sweep_pairs), one per half sweep: a k_ir_step launch is 10 to 14
-// us long whatever its size, and the sweeps of 32 solves of 14 tiles took 1.19
-// ms, so 0.79.  Returns the number of
-// unconverged solves left in *left.
+// per tile column (k_ir_step), or, for solves with half sweeps (half_sweeps),
+// one per half: a k_ir_step launch is 10 to 14 us long whatever its size, and
+// the sweeps of 32 solves of 14 tiles took 1.19 ms, so 0.79.  The two round
+// differently, so a solve's form goes by its own size, and a chunk with both
+// kinds has the launches of both (nt_min, nt_max: its smallest and largest
+// solve).  Returns the number of unconverged solves left in *left.
 template <class T>
-int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int max_sweeps,
-           double tol, int *left) {
+int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_min, int nt_max, int kc,
+           int max_sweeps, double tol, int *left) {
+  const bool halves = half_sweeps<T>(kc, nt_min), steps = !half_sweeps<T>(kc, nt_max);
   hipLaunchKernelGGL(k_ir_init<T>, dim3(nt_max, nb), dim3(256), 0, c->stream, dd);
   if (int r = check_launch("k_ir_init")) return r;
   int done = 0;
@@ -602,32 +604,36 @@ int refine(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, int kc, int ma
         hipLaunchKernelGGL((k_ir_residual<T, 1>), dim3(nt_max, nb), dim3(256), 0, c->stream, dd);
     }
     if (int r = check_launch("k_ir_residual")) return r;
-    if (sizeof(T) == 4 && kc == 32 && sweep_pairs(nt_max)) {
+    {
       ProfScope p(c, 6);
       const dim3 grid(nb, 2), block(kSweepWaves * 64);
-      const auto fwd = it == 0 ? k_ir_sweep<true, 2, kSweepFwd> : k_ir_sweep<false, 2, kSweepFwd>;
-      hipLaunchKernelGGL(fwd, grid, block, 0, c->stream, dd, tol);
-      hipLaunchKernelGGL(k_ir_decide, dim3((nb + 255) / 256), dim3(256), 0, c->stream, dd, nb, tol);
-      hipLaunchKernelGGL((k_ir_sweep<false, 2, kSweepBwd>), grid, block, 0, c->stream, dd, tol);
-    } else {
-      ProfScope p(c, 6);
-      if (it == 0) {  // R = B: only the last tile of each solve (kIrFirstSweep)
-        hipLaunchKernelGGL((k_ir_step<T, true>), dim3(1, nb), dim3(256), 0, c->stream, dd,
-                           kIrFirstSweep);
-      } else {
-        for (int s = -1; s <= nt_max - 2; s++)
-          hipLaunchKernelGGL((k_ir_step<T, true>), dim3(s < 0 ? 1 : nt_max - 1 - s, nb), dim3(256),
-                             0, c->stream, dd, s);
+      if (halves) {
+        const auto fwd = it == 0 ? k_ir_sweep<true, 2, kSweepFwd> : k_ir_sweep<false, 2, kSweepFwd>;
+        hipLaunchKernelGGL(fwd, grid, block, 0, c->stream, dd, tol);
+      }
+      if (steps) {
+        if (it == 0) {  // R = B: only the last tile of each solve (kIrFirstSweep)
+          hipLaunchKernelGGL((k_ir_step<T, true>), dim3(1, nb), dim3(256), 0, c->stream, dd,
+                             kIrFirstSweep);
+        } else {
+          for (int s = -1; s <= nt_max - 2; s++)
+            hipLaunchKernelGGL((k_ir_step<T, true>), dim3(s < 0 ? 1 : nt_max - 1 - s, nb),
+                               dim3(256), 0, c->stream, dd, s);
+        }
+        hipLaunchKernelGGL(k_ir_accum<T>, dim3(1, nb), dim3(256), 0, c->stream, dd, 1);
       }
       // the central rows are final after the forward steps: test convergence
       // before the backward steps, which converged solves then skip
-      hipLaunchKernelGGL(k_ir_accum<T>, dim3(1, nb), dim3(256), 0, c->stream, dd, 1);
       hipLaunchKernelGGL(k_ir_decide, dim3((nb + 255) / 256), dim3(256), 0, c->stream, dd, nb, tol);
-      for (int j = 0; j <= nt_max - 2; j++)
-        hipLaunchKernelGGL((k_ir_step<T, false>), dim3(nt_max - 1 - j, nb), dim3(256), 0, c->stream,
-                           dd, j);
-      if (nt_max > 1)
-        hipLaunchKernelGGL(k_ir_accum<T>, dim3(nt_max - 1, nb), dim3(256), 0, c->stream, dd, 0);
+      if (halves)
+        hipLaunchKernelGGL((k_ir_sweep<false, 2, kSweepBwd>), grid, block, 0, c->stream, dd, tol);
+      if (steps) {
+        for (int j = 0; j <= nt_max - 2; j++)
+          hipLaunchKernelGGL((k_ir_step<T, false>), dim3(nt_max - 1 - j, nb), dim3(256), 0,
+                             c->stream, dd, j);
+        if (nt_max > 1)
+          hipLaunchKernelGGL(k_ir_accum<T>, dim3(nt_max - 1, nb), dim3(256), 0, c->stream, dd, 0);
+      }
     }
     if (int r = check_launch("k_ir_step")) return r;
     if (it >= 1) {  // the first correction never meets the tolerance
@@ -834,7 +840,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
     while (end < nsolve && (end == done || acc + bytes[end] <= cap)) acc += bytes[end++];
     int nb = end - done;
     long mtot = 0, xtot = 0, ivtot = 0, htot = 0, ghtot = 0, ybtot = 0, gptot = 0;
-    int maxliz = 1, nt_max = 1, nbands_min = INT_MAX, nbands_max = 0;
+    int maxliz = 1, nt_min = INT_MAX, nt_max = 1, nbands_min = INT_MAX, nbands_max = 0;
     for (int b = 0; b < nb; b++) {
       const AtomDev &a = c->atoms[atom_ids[done + b]];
       long Ns = roundup(nsc * a.nrmat, kTile);
@@ -843,6 +849,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
       ivtot += refining ? (Ns / kTile) * kTile * kTile : kTile * kTile;
       htot += 2 * lu_group(c, split) * (Ns / kTile + 1);
       maxliz = std::max(maxliz, a.numLIZ);
+      nt_min = std::min(nt_min, (int)(Ns / kTile));
       nt_max = std::max(nt_max, (int)(Ns / kTile));
       if (gmode) {
         ghtot += g_blocks(a.numLIZ) * 256;
@@ -1137,9 +1144,9 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
     if (refining) {
       int left = 0;
       int r = ir_inline ? 0
-              : mixed   ? refine<float>(c, c->desc.p, nb, nt_max, kc, c->ir_max_sweeps, c->ir_tol,
-                                        &left)
-                        : refine<double>(c, c->desc.p, nb, nt_max, kc, c->ir_max_sweeps,
+              : mixed   ? refine<float>(c, c->desc.p, nb, nt_min, nt_max, kc, c->ir_max_sweeps,
+                                        c->ir_tol, &left)
+                        : refine<double>(c, c->desc.p, nb, nt_min, nt_max, kc, c->ir_max_sweeps,
                                          c->ir_tol, &left);
       if (r) return r;
       std::vector<int> hconv(nb);

@@ -23,6 +23,14 @@ constexpr int kSweepWaves = 8;
 constexpr int kSweepMaxTiles = 128;
 constexpr int kSweepPairTiles = 15;  // tiles a sweep by pairs of waves takes (its y are in LDS)
 enum SweepPart { kSweepAll, kSweepFwd, kSweepBwd };
+// Whether the sweeps of a solve of nt tiles with factors of type T and kc
+// right-hand sides go by halves (k_ir_sweep, a launch each) rather than by tile
+// columns (k_ir_step): FP32 factors and 32 right-hand sides, as far as pairs of
+// waves take them.
+template <class T>
+__host__ __device__ constexpr bool half_sweeps(int kc, int nt) {
+  return sizeof(T) == 4 && kc == 32 && nt <= kSweepPairTiles;
+}
 constexpr unsigned kSweepSpinLimit = 1u << 24;  // bound of one k_ir_sweep flag wait
 constexpr int kInfoSweepStall = -2;             // per-solve info when that bound is hit
 // per-solve info of a solve whose FP64 refinement did not converge: its
