@@ -1059,19 +1059,19 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
     const bool uniform = std::all_of(hd.begin(), hd.end(), [&](const SolveDesc &d) { return d.nt == nt_max; });
     auto enqueue_part = [&](hipStream_t st, int b0, int n, hipEvent_t after_asm) -> int {
       const SolveDesc *dd = c->desc.p + b0;
-      // the step range is the chunk's: right-aligned starts are relative to it
+      // the step range is the chunk's: right-aligned starts are relative to it.
+      // Every size of a launch is the chunk's or in the graph key: a captured
+      // sequence is replayed with other solves in either half
       const int ntm = nt_max;
-      int mliz = 1;
-      for (int b = b0; b < b0 + n; b++) mliz = std::max(mliz, hd[b].numLIZ);
       hipLaunchKernelGGL(k_init_status, dim3((n + 255) / 256), dim3(256), 0, st, dd, n);
       if (int r = check_launch("k_init_status")) return r;
       {
         ProfScope p(c, 0);
         hipLaunchKernelGGL(k_pad_identity, dim3(ntm, n), dim3(256), 0, st, dd);
         if (share)
-          launch_assemble_from_g(c, dim3(mliz, n), st, dd, asm_mode);
+          launch_assemble_from_g(c, dim3(maxliz, n), st, dd, asm_mode);
         else
-          launch_assemble(c, nsc, dim3(mliz, n), st, dd, asm_mode);
+          launch_assemble(c, nsc, dim3(maxliz, n), st, dd, asm_mode);
       }
       if (int r = check_launch("k_assemble")) return r;
       if (after_asm) HIPCHK(hipEventRecord(after_asm, st));
@@ -1109,7 +1109,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
     if (c->use_graph) {
       long tol_bits = 0;
       std::memcpy(&tol_bits, &c->ir_tol, sizeof(tol_bits));
-      std::vector<long> key = {nb, nt_max, maxliz, precision, c->sched, (long)c->desc.p,
+      std::vector<long> key = {nb, nt_max, maxliz, nsc, precision, c->sched, (long)c->desc.p,
                                (long)c->tmat.p, c->ldT, (long)c->cgnt.p, (long)c->illp.p,
                                c->lmax_tab, c->ir_max_sweeps, tol_bits, gmode ? nbands_max : -1,
                                (long)(gmode && nbands_min <= kGDirectBands),
