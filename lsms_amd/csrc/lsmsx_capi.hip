@@ -106,7 +106,7 @@ __global__ void k_rel_tau(double2 *, int, const double *, const double2 *);
 __global__ void k_rel_blocks(double2 *, long, int, const double *);
 __global__ void k_lu_diag_h(const SolveDesc *, int, int);
 __global__ void k_lu_panel_h(const SolveDesc *, int, int, int, int);
-__global__ void k_lu_strip_h(const SolveDesc *, int);
+__global__ void k_lu_strip_h(const SolveDesc *, int, int);
 
 // Copy a caller matrix (central block first, n x n) into the solver layout;
 // rowperm (or null) reorders the n - k non-central rows: solver row xr takes
@@ -502,12 +502,15 @@ int launch_lu_steps(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool 
   for (int s = 0; s < nt_max - 1; s += G) {
     const int b = std::min(s + G - 1, nt_max - 2);  // the group's last step, largest solve
     const int nrest = nt_max - 1 - b;
-    // strips (k_lu_strip_h) where there are many to a compute unit: a strip is
-    // as long as its group's steps together, and so is the launch's end (248
-    // solves of N = 2160, 12896 to 4960 strips a group: 52.6 -> 51.5 ms; 96
-    // uneven ones of an alloy, up to 4224: 19.2 -> 19.4; 32 of N = 864, 384:
-    // 3.45 -> 3.5)
-    const bool strips = split_f16 && 2L * nrest * nb >= 4864;
+    // strips (k_lu_strip_h) for solves of one size, where there are many to a
+    // compute unit: a strip is as long as its group's steps together, and so is
+    // the launch's end.  N = 2160, panels against strips: 96 solves (4992 strips
+    // in the first group) 26.6 and 26.25 ms, 128 31.9 and 31.4, 192 44.0 and
+    // 43.5, 248 52.9 and 52.0; with all of 248's groups as strips (the last has
+    // 992) 52.3.  Uneven batches lose in either order: 2048 solves of an alloy
+    // (14 to 32 tiles) 200 ms by panels, 207 by strips in plain order and 211 by
+    // XCD; 512 56.4, 57.8 and 56.2; 192 25.6, 25.9 and 25.3
+    const bool strips = split_f16 && uniform && 2L * nrest * nb >= 4864;
     for (int t = s; t <= b; t++) {
       const int u = t - s, np = 2 * (nt_max - 1 - t);
       if (u > 0 && !split_f16) {
@@ -540,7 +543,7 @@ int launch_lu_steps(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool 
     }
     if (strips) {
       ProfScope p(c, 2);
-      hipLaunchKernelGGL(k_lu_strip_h, dim3(2 * nrest, nb), dim3(256), 0, st, dd, s);
+      hipLaunchKernelGGL(k_lu_strip_h, dim3(2 * nrest, nb), dim3(256), 0, st, dd, s, swz);
     }
     {
       ProfScope p(c, 3);

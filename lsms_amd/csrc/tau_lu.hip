@@ -517,7 +517,8 @@ __global__ __launch_bounds__(256) void k_lu_panel(const SolveDesc *__restrict__ 
 }
 
 // Panels of a group on the split-FP16 path.  k_lu_panel_h takes the tiles of
-// one step: all of its column and row, or in large launches (launch_lu_steps)
+// one step: all of its column and row, or in large launches of solves of one
+// size (launch_lu_steps)
 // those inside the group's diagonal block alone (rows and columns up to its
 // last step), which the next diagonal tiles wait for; then each tile row below
 // the block, and each tile column right of it, runs through all the group's
@@ -525,8 +526,8 @@ __global__ __launch_bounds__(256) void k_lu_panel(const SolveDesc *__restrict__ 
 // earlier step of the group again, from HBM mostly; a strip shares the block's
 // planes with the others at the same step through L2, and saves the launches'
 // ends (248 solves N = 2160: 14.7 -> 13.4 ms a pass for the panels).
-// The workgroups of one solve run on one XCD (xcd_remap; for k_lu_panel_h with
-// xcd_swizzle), so that the planes they share are fetched into one L2.
+// With xcd_swizzle the workgroups of one solve run on one XCD, so that the planes
+// they share are fetched into one L2.
 
 // the last step of the group starting at solve step g
 __device__ __forceinline__ int group_last(const SolveDesc &d, int g) {
@@ -546,9 +547,10 @@ __global__ __launch_bounds__(256) void k_lu_panel_h(const SolveDesc *__restrict_
   panel_tile_h(d, s, ncross, bx < n, s + 1 + (bx < n ? bx : bx - n));
 }
 
-__global__ __launch_bounds__(256, 3) void k_lu_strip_h(const SolveDesc *__restrict__ descs, int step) {
+__global__ __launch_bounds__(256, 3) void k_lu_strip_h(const SolveDesc *__restrict__ descs, int step,
+                                                       int xcd_swizzle) {
   int bx = blockIdx.x, by = blockIdx.y;
-  xcd_remap(bx, by);
+  if (xcd_swizzle) xcd_remap(bx, by);
   const SolveDesc &d = descs[by];
   const int g = step - d.step0;
   if (g < 0) return;
