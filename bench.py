@@ -275,7 +275,8 @@ def main():
         prec = {"fp64": capi.PREC_FP64, "fp32": capi.PREC_MIXED_FP32,
                 "f16": capi.PREC_MIXED_F16}[args.profile_step]
         ctx.set_graph(False)
-        ctx.set_schedule(max(args.schedule, 0) & ~capi.SCHED_TWO_STREAMS)
+        if args.schedule >= 0:
+            ctx.set_schedule(args.schedule & ~capi.SCHED_TWO_STREAMS)
         ctx.set_split_group(args.split_group)
         ctx.tau00_batched(atoms, iies, prels, k, precision=prec)
         t0 = time.perf_counter()

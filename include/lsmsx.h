@@ -263,11 +263,13 @@ int lsmsx_tau00_adjoint(lsmsx_ctx *ctx, int nsolve, const int *atom_ids,
  *                            updates, the panels with their fused cross
  *                            updates) are remapped so that each of the 8 XCDs
  *                            works on whole solves and reads their panels
- *                            into its own L2 (split-FP16 batches of one size
- *                            always are);
+ *                            into its own L2;
  *   LSMSX_SCHED_TWO_STREAMS  the two halves of a chunk run on two streams (of
  *                            default priority), so one half's diagonal-tile
  *                            and panel steps overlap the other's updates.
+ * Until one is set, here or by lsmsx_autotune, the schedule is 0 (which
+ * lsmsx_get_schedule returns), except that split-FP16 batches of one size take
+ * the XCD order.
  * No reference counterpart (the reference solves one matrix per OpenMP
  * thread, calculateTauMatrix.cpp:891-900). */
 #define LSMSX_SCHED_RIGHT_ALIGN 1

@@ -326,8 +326,10 @@ struct lsmsx_ctx {
   DevBuf<int> it_i;       // cell_of, ncrit
   double ir_tol = 1e-12;
   double pivot_guard = 1e-2;  // plain FP64 solves with a smaller tile pivot are refined
-  // schedule (LSMSX_SCHED_* flags) and hipGraph replay of the batched path
+  // schedule (LSMSX_SCHED_* flags; sched_set: by the caller or the autotuner) and
+  // hipGraph replay of the batched path
   int sched = 0;
+  bool sched_set = false;
   int split_group = 8;                     // steps per trailing update, split-FP16 path
   double group_ms[3] = {-1.0, -1.0, -1.0};  // last autotune: split groups 4, 8, 16
   bool use_graph = false;
@@ -491,13 +493,13 @@ inline bool lu_small_grid(long tiles) { return tiles <= 256; }
 template <class T>
 int launch_lu_steps(lsmsx_ctx *c, const SolveDesc *dd, int nb, int nt_max, bool split_f16,
                     hipStream_t st, bool uniform) {
-  // XCD order where the caller asked for it, and on the split-FP16 path where
-  // all solves have the same size (`uniform`): each XCD then has the same work,
-  // and a solve's planes are in its own L2 (248 solves N = 2160: 48.3 -> 47.5
-  // ms, 32 of N = 864: 2.63 -> 2.53; 96 of an alloy, from 14 to 32 tiles, would
-  // take 15.9 -> 16.9, and FP64 solves, bound by the MFMAs, gain nothing: six of
-  // N = 4384 21.6 -> 21.9)
-  const int swz = (uniform && split_f16) || (c->sched & LSMSX_SCHED_XCD_SWIZZLE) ? 1 : 0;
+  // XCD order where the schedule has it; without a schedule set, on the split-FP16
+  // path where all solves have the same size (`uniform`): each XCD then has the
+  // same work, and a solve's planes are in its own L2 (248 solves N = 2160: 48.3
+  // -> 47.5 ms, 32 of N = 864: 2.63 -> 2.53; 96 of an alloy, from 14 to 32 tiles,
+  // would take 15.9 -> 16.9, and FP64 solves, bound by the MFMAs, gain nothing:
+  // six of N = 4384 21.6 -> 21.9)
+  const int swz = c->sched_set ? (c->sched & LSMSX_SCHED_XCD_SWIZZLE) != 0 : uniform && split_f16;
   const int G = lu_group(c, split_f16);
   for (int s = 0; s < nt_max - 1; s += G) {
     const int b = std::min(s + G - 1, nt_max - 2);  // the group's last step, largest solve
@@ -1117,7 +1119,7 @@ int run_batched(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *ispins
                                c->lmax_tab, c->ir_max_sweeps, tol_bits, gmode ? nbands_max : -1,
                                (long)(gmode && nbands_min <= kGDirectBands),
                                lu_group(c, split), share ? (long)own.size() : -1,
-                               (long)c->desc_own.p, (long)uniform};
+                               (long)c->desc_own.p, (long)uniform, (long)c->sched_set};
       auto it = c->graphs.find(key);
       if (it == c->graphs.end()) {
         const bool prof = c->profiling;
@@ -2276,6 +2278,7 @@ int lsmsx_set_schedule(lsmsx_ctx *c, int flags) {
   if (flags & ~(LSMSX_SCHED_RIGHT_ALIGN | LSMSX_SCHED_XCD_SWIZZLE | LSMSX_SCHED_TWO_STREAMS))
     return fail(-2, "unknown schedule flags");
   c->sched = flags;
+  c->sched_set = true;
   return 0;
 }
 
@@ -2325,8 +2328,10 @@ int lsmsx_autotune(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *isp
                        tau.data(), info.data());  // warm-up: allocations, graphs of sched 0
   double tbest = 1e300;
   int sbest = c->sched;
+  const bool was_set = c->sched_set;
   for (int sch = 0; sch < 8 && rc == 0; sch++) {
     c->sched = sch;
+    c->sched_set = true;
     if (c->use_graph) {  // capture outside the timed run
       rc = run_batched(c, nsolve, atom_ids, ispins, iies, prel, nsc, nspola, precision,
                        tau.data(), info.data());
@@ -2343,6 +2348,7 @@ int lsmsx_autotune(lsmsx_ctx *c, int nsolve, const int *atom_ids, const int *isp
     }
   }
   c->sched = sbest;
+  c->sched_set = was_set || tbest < 1e300;
   // split-FP16 path: the steps per trailing update under the chosen schedule
   if (precision == LSMSX_PREC_MIXED_F16 && rc == 0) {
     // a single timed run per size: another size replaces the default 8 only
