@@ -332,6 +332,14 @@ __device__ void bessel_jh(zd x, zd *bj, zd *hm, zd &eiz) {
   for (int l = 2; l <= LB; l++) hm[l] = (double)(2 * l - 1) * hm[l - 1] * x1 - hm[l - 2];
 }
 
+// (no recursion, whose arrays would have no second element)
+template <>
+__device__ inline void bessel_jh<0>(zd x, zd *bj, zd *hm, zd &eiz) {
+  bj[0] = zsin(x) / x;
+  hm[0] = mk(0.0, -1.0);
+  eiz = zexp_i(x);
+}
+
 // j_l, j_{l-1} (or j_1 at l = 0) and the same of hm, at argument x
 struct BesselPick {
   zd bj_l, bj_o, hm_l, hm_o, hm_0, bj_0, eiz;
