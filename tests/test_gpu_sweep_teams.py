@@ -32,3 +32,35 @@ def test_alone_and_beside_a_large_solve(precision, nsites):
     assert s.nrmat_ns(big) > 12 * 64
     assert np.array_equal(one[0], two[0])
     assert rel(one[0], lapack_tau00(s, small, ie)) < 1e-10
+
+
+@pytest.mark.parametrize("precision", [capi.PREC_MIXED_FP32, capi.PREC_MIXED_F16])
+def test_both_sides_of_the_line(precision):
+    """14 to 16 tiles (the line is at 15, where the pairs' y just fit LDS): each
+    size alone, beside others on the pairs' side and beside the largest zone."""
+    s = CF.config_c4()
+    sizes = [56, 57, 60, 61, 64]
+    big = pick(s, 2)[1]
+    small = [a for a in range(len(s.atoms)) if s.atoms[a].numLIZ >= 64 and a != big][:len(sizes)]
+    for i, n in zip(small, sizes):
+        a = s.atoms[i]
+        a.LIZPos = np.asfortranarray(a.LIZPos[:, :n])
+        a.LIZlmax, a.LIZStoreIdx = a.LIZlmax[:n].copy(), a.LIZStoreIdx[:n].copy()
+        a.numLIZ, a.nrmat = n, int(np.sum((a.LIZlmax + 1) ** 2))
+    assert [-(-s.nrmat_ns(i) // 64) for i in small] == [14, 15, 15, 16, 16]
+    assert s.nrmat_ns(big) > 16 * 64
+    ctx = capi.Context(0)
+    ctx.load_system(s)
+    ie = 11
+
+    def solve(atoms):
+        tau, info = ctx.tau00_batched(atoms, [ie] * len(atoms), [s.prel(ie)] * len(atoms), 16,
+                                      precision=precision)
+        assert np.all(info == 0) and np.all(ctx.last_stats(len(atoms))[0] > 0)
+        return tau
+
+    for i, beside in zip(small, solve(small + [big])):
+        alone = solve([i])[0]
+        assert np.array_equal(alone, beside), s.atoms[i].numLIZ
+        assert np.array_equal(alone, solve([small[0], i])[1])
+        assert rel(alone, lapack_tau00(s, i, ie)) < 1e-10

@@ -1,9 +1,9 @@
-"""The 64 x 64 tile factorization on the GPU (register LU with pivoting inside
-the tile, its triangular inverses, the last tile's solve), through
-solve_tau00_matrix, against LAPACK.
+"""The 64 x 64 tile factorization on the GPU (LU in LDS with pivoting inside the
+tile, by panels of four columns, its triangular inverses, the last tile's solve),
+through solve_tau00_matrix, against LAPACK.
 
-Sizes at the edges of the tile and of its 8-column panels, every kind of
-right-hand-side count.  Tolerance: the backward error of LU with partial
+Sizes at the edges of the tile and of its panels, every kind of right-hand-side
+count.  Tolerance: the backward error of LU with partial
 pivoting is a small multiple of n eps here (no growth: random matrices and
 matrices near 1), so the forward error is held to 8 n eps cond(M)."""
 import numpy as np
@@ -66,3 +66,10 @@ def test_zero_pivot_position(ctx, col):
     m[:, k + col] = 0.0
     _, info = ctx.solve_tau00_matrix(m, np.eye(k, dtype=complex))
     assert info == col + 1
+
+
+@pytest.mark.parametrize("n,k", [(3, 2), (4, 4), (5, 1), (61, 3), (67, 4), (68, 5), (69, 8)])
+def test_panel_edges(ctx, n, k):
+    """Sizes on both sides of a panel of four columns."""
+    test_tile_solve(ctx, "near1", n, k)
+    test_tile_solve(ctx, "ties", n, k)
