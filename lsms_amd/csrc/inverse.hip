@@ -20,9 +20,9 @@
 // one workgroup (or four): every tile of Y is written once in each half, and
 // its sum and the product with the diagonal inverse are one pass (panel_op).
 // With a panel and an update launch per step, which read and wrote the tiles
-// of Y once for every u, eight solves of N = 944 took 1.33 ms, so 1.07 (MFMAs
-// busy 40%: the quarter tiles of such a small batch keep the L1 caches busy
-// with operands).
+// of Y once for every u, eight solves of N = 944 took 1.33 ms, so 0.89: forward
+// 0.39 with the MFMAs busy 21%, backward 0.50 and 47% (a launch is as long as
+// its longest tile).
 // Work: Ns^3/6 (forward) + Ns^3/2 (backward) complex MACs on FP64 MFMA, 3M form.
 #include "lu_common.hpp"
 

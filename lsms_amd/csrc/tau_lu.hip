@@ -680,7 +680,7 @@ __global__ __launch_bounds__(256) void k_lu_cross_diag(const SolveDesc *__restri
 
 // Trailing update of the group starting at global step s: A_ij -= sum over
 // the group's steps k of L_ik U_kj for all i, j beyond the group, one pass
-// over C with K = 64 ns.  64 solves N = 2160 in FP64: 19.2 ms with the MFMAs
+// over C with K = 64 ns.  64 solves N = 2160 in FP64: 18.2 ms with the MFMAs
 // busy 85% (22.4 ms and 75% with groups of two steps).
 template <class T, int N>
 __global__ __launch_bounds__(256) void k_lu_trail(const SolveDesc *__restrict__ descs, int step,
